@@ -103,7 +103,7 @@ __global__ __launch_bounds__(64) void cr_asm_kernel(
                 ok[r] = in[r] && wb[r] > 0.0 && cr_row_ok(f[r], yv[r]);
                 seed[r] = ok[r] ? sqrt(wb[r]) : 0.0;
             }
-            const V fin = vm_reverse<V, dv16, dv16, dv8>((const uint2 *)(code + d.rev_off), d.nrev,
+            const V fin = vm_reverse<V, VM_TAPE_U, dv16, dv16, dv8>((const uint2 *)(code + d.rev_off), d.nrev,
                                                          seed, cst, U0, U1, B0, B1, A0, A1,
                                                          (char *)(X + lane));
 #pragma unroll

@@ -1446,33 +1446,53 @@ std::vector<FtRows> rc_fit_rows(RcCtx *c)
 struct FtVmCode {
     int vorc = -1, vmrc = -1;
     bool vm4 = false;
+    int tape = 0;   /* 4-row streams: 1 VMC_TAPE_B, 2 VMC_TAPE_L */
+    int lslots = 0; /* LDS tape slots (VMC_TAPE_L) */
     std::vector<uint32_t> vf, vr, vt;
 };
 
 /* Compile a candidate for the fit VM: the value-pass stream (value-only
-   form, inputs in U, 8-slot file) and the forward/reverse pair, at 4 rows
-   per lane when the program fits that block's files (an 8-slot B file, one
-   saved adjoint, and a value-pass stream for the f64 polish), else at 2 rows
-   per lane, whose block has the 2-row column stride.  A stream that does not
-   compile leaves its code nonzero: the candidate then runs on the general
-   interpreter. */
+   form, inputs in U, 8-slot file) and the forward/reverse pair.  The pair is
+   for 4 rows per lane when the program fits that block's files (an 8-slot B
+   file, one saved adjoint, and a value-pass stream for the f64 polish): first
+   with the tape in U alone, then with what U cannot hold in B, then in LDS.
+   U has 15 slots less the inputs, which a sum of a dozen terms fills; an LDS
+   slot costs 1 KB of each wave's block, so B comes first.  Else it is for 2
+   rows per lane, whose block has 16 B slots, 8 saved adjoints and its own
+   column stride.  A stream that does not compile leaves its code nonzero: the
+   candidate then runs on the general interpreter, at some ten times the time
+   per row. */
 static void vm_compile(FtVmCode &o, const uint32_t *rec, int words, int p, int nv, int tune_rows,
                        bool all64)
 {
     uint32_t vf[2 * 4 * FT_MAX_NODES], vr[2 * 8 * FT_MAX_NODES], vt[2 * 4 * FT_MAX_NODES];
     int info[6] = {0, 0, 0, 0, 0, 0}, tinfo[6] = {0, 0, 0, 0, 0, 0};
     const int nf = (int)(sizeof(vf) / 4), nr = (int)(sizeof(vr) / 4), ntv = (int)(sizeof(vt) / 4);
+    auto pair = [&](int col_bytes, unsigned flags) {
+        o.vmrc = rch_fitvm_compile(rec, words, p, nv, col_bytes, VMC_INPUTS_IN_U | flags, vf, nf,
+                                   vr, nr, info);
+        return o.vmrc == 0;
+    };
     o.vorc = rch_fitvm_compile(rec, words, p, nv, VM_XS(4) * 4,
                                VMC_INPUTS_IN_U | VMC_VALUE_ONLY | VMC_SMALL_U, vt, ntv, nullptr, 0,
                                tinfo);
-    o.vmrc = rch_fitvm_compile(rec, words, p, nv, VM_XS(4) * 4, VMC_INPUTS_IN_U, vf, nf, vr, nr,
-                               info);
-    o.vm4 = o.vmrc == 0 && info[3] <= 8 && info[4] <= 1 && o.vorc == 0 && tune_rows != 2 && !all64;
-    /* The 2-row block: f32 columns, or the plain FP64 arm's f64 columns
-       (same register files, wider column stride). */
-    if (o.vmrc == 0 && !o.vm4)
-        o.vmrc = rch_fitvm_compile(rec, words, p, nv, all64 ? VM64_XS(2) * 8 : VM_XS(2) * 4,
-                                   VMC_INPUTS_IN_U, vf, nf, vr, nr, info);
+    if (all64) {
+        /* The plain FP64 arm: 2 f64 rows, the tape in U alone. */
+        pair(VM64_XS(2) * 8, 0);
+    } else {
+        if (o.vorc == 0 && tune_rows != 2) {
+            o.vm4 = pair(VM_XS(4) * 4, 0) && info[3] <= 8 && info[4] <= 1;
+            for (int t = 1; t <= 2 && !o.vm4; ++t) {
+                o.vm4 = pair(VM_XS(4) * 4, VMC_SMALL_B | (t == 1 ? VMC_TAPE_B : VMC_TAPE_L)) &&
+                        info[4] <= 1;
+                if (o.vm4) {
+                    o.tape = t;
+                    o.lslots = info[5];
+                }
+            }
+        }
+        if (!o.vm4) pair(VM_XS(2) * 4, 0);
+    }
     if (o.vorc == 0) o.vt.assign(vt, vt + 2 * tinfo[0]);
     if (o.vmrc == 0) {
         o.vf.assign(vf, vf + 2 * info[0]);
@@ -1540,14 +1560,17 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
     /* Assembly classes: fit VM with 4 rows per lane (KC16, KC32), fit VM
        with 2 rows per lane (KC16, KC32), general interpreter with the
        register stores (KC16, KC32) and with the oversized stores (KC16,
-       KC32).  Value-pass classes: fit VM, general small, general big. */
-    enum { NA = 8, NT = 3 };
+       KC32), fit VM with 4 rows per lane and tape values in B (KC16, KC32),
+       the same with tape values in LDS (KC16, KC32).
+       Value-pass classes: fit VM, general small, general big. */
+    enum { NA = 12, NT = 3 };
     std::vector<int> list[NA];
     std::vector<int> tlist[NT];
     /* The trial lists split per candidate into the first (nitems + 1) / 2
        items and the rest, for the LM trial passes' early rejection. */
     std::vector<int> tlist_a[NT], tlist_b[NT];
     int maxK = 2;
+    int lslots[2] = {0, 0}; /* LDS tape slots of classes 10 and 11 */
     const int tile_rows = c->tune_fit_tile > 0 ? c->tune_fit_tile : TILE_ROWS;
     size_t p64_blocks = 0; /* f64 prediction buffer, in 64-row blocks */
     for (int i = 0; i < nprog; ++i) {
@@ -1595,8 +1618,9 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
         d.item0 = (int)items.size();
         const bool big = prog_is_big(progs[i]);
         const int kc = d.k + 2 <= 16 ? 0 : 1;
-        const int cls = d.vm ? (vm4 ? 0 : 2) + kc : (big ? 6 : 4) + kc;
+        const int cls = d.vm ? (!vm4 ? 2 : vc.tape ? 6 + 2 * vc.tape : 0) + kc : (big ? 6 : 4) + kc;
         maxK = std::max(maxK, d.k + 2);
+        if (vm4 && vc.tape == 2) lslots[kc] = std::max(lslots[kc], vc.lslots);
         const int ntiles = (n + tile_rows - 1) / tile_rows;
         for (int r0 = 0, tix = 0; r0 < n; r0 += tile_rows, ++tix) {
             FtItem it;
@@ -1765,7 +1789,7 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
                                 d_cp32, d_cp64, d_pgram, tri_stride, d_ploss, d_pbad, d_pskip);
     };
     auto vm_asm = [&](int kc, int r, bool polish, int q, hipStream_t st) {
-        vm_launch_asm(kc, r, polish, lofs[q + 1] - lofs[q], st, d_items, d_lists + lofs[q], d_cand,
+        vm_launch_asm(kc, r, q >= 8 ? q / 2 - 3 : 0, lslots[q & 1], polish, lofs[q + 1] - lofs[q], st, d_items, d_lists + lofs[q], d_cand,
                       d_rows, d_code, d_run_a, d_cp32, d_cp64, d_pgram, tri_stride, d_ploss,
                       d_pbad, d_pskip, d_p64);
     };
@@ -1783,7 +1807,7 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
     auto asm_pass0 = [&](int polish) {
         fork();
         if (all64) {
-            /* Classes 0 and 1 (4 f32 rows per lane) are empty here. */
+            /* The classes of 4 f32 rows per lane (0, 1, 8..11) are empty here. */
             vm_asm64(16, polish != 0, 2, s);
             vm_asm64(32, polish != 0, 3, s);
             if (polish) {
@@ -1800,6 +1824,10 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
         } else if (polish) {
             vm_asm(16, 4, true, 0, s);
             vm_asm(32, 4, true, 1, s);
+            vm_asm(16, 4, true, 8, s);
+            vm_asm(32, 4, true, 9, s);
+            vm_asm(16, 4, true, 10, s);
+            vm_asm(32, 4, true, 11, s);
             vm_asm(16, 2, true, 2, sd);
             vm_asm(32, 2, true, 3, sd);
             asm_launch(ft_asm_kernel<16, false, true>, 4, sd);
@@ -1809,6 +1837,10 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
         } else {
             vm_asm(16, 4, false, 0, s);
             vm_asm(32, 4, false, 1, s);
+            vm_asm(16, 4, false, 8, s);
+            vm_asm(32, 4, false, 9, s);
+            vm_asm(16, 4, false, 10, s);
+            vm_asm(32, 4, false, 11, s);
             vm_asm(16, 2, false, 2, sd);
             vm_asm(32, 2, false, 3, sd);
             asm_launch(ft_asm_kernel<16, false, false>, 4, sd);
@@ -1865,6 +1897,8 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
     /* The launch sequence: recorded as a hipGraph per batch shape. */
     std::vector<uint64_t> key = ft_graph_key(nprog, nitems, iters, any_irls, kmax, tri_stride, D,
                                              rg, lofs, NA + 1, tofs, NT + 1, f->mode);
+    key.push_back((uint64_t)lslots[0]);
+    key.push_back((uint64_t)lslots[1]);
     for (int q = 0; q <= NT; ++q) {
         key.push_back((uint64_t)tofs_a[q]);
         key.push_back((uint64_t)tofs_b[q]);

@@ -72,6 +72,7 @@ struct Unit {
     int gl, gr;           /* gradient columns (constant slots) or -1 */
     int nodes_next;       /* children that continue the sweep: 0, 1 or 2 */
     bool ffused;          /* its forward word was folded into the previous one */
+    bool tb;              /* ut is a B or LDS slot (VMC_TAPE_B / _L) */
 };
 
 struct Compiler {
@@ -79,6 +80,10 @@ struct Compiler {
     int nvars = 0;
     bool vo = false;       /* value only: no tape */
     int usink = VM_U_SINK; /* the U sink slot */
+    bool tape_b = false, tape_l = false; /* tape values may take B / LDS slots */
+    int lnext = 0;
+    int bslots = VM_B_SINK; /* usable B slots */
+    int reserve = 0;       /* U slots then kept for spilled operands */
     int depth = 0;
     std::vector<int> spill;
     bool ufree[VM_U_SLOTS];
@@ -97,12 +102,29 @@ struct Compiler {
         overflow = true;
         return usink;
     }
-    /* A tape slot: none in value-only code. */
-    int talloc() { return vo ? usink : ualloc(); }
+    /* A tape slot (none in value-only code): a U slot, or a B or LDS slot (tb)
+       once U holds no more than the spilled operands may still need. */
+    int talloc(bool &tb)
+    {
+        tb = false;
+        if (vo) return usink;
+        if (tape_b || tape_l) {
+            int left = 0;
+            for (int s = 0; s < usink; ++s) left += ufree[s] ? 1 : 0;
+            if (left + (int)spill.size() <= reserve) {
+                tb = true;
+                if (tape_b) return balloc();
+                if (lnext < VM_L_SLOTS) return lnext++;
+                overflow = true;
+                return VM_U_SINK;
+            }
+        }
+        return ualloc();
+    }
     int balloc()
     {
         if (vo) return VM_B_SINK;
-        if (bnext >= VM_B_SINK) {
+        if (bnext >= bslots) {
             overflow = true;
             return VM_B_SINK;
         }
@@ -167,9 +189,11 @@ struct Compiler {
             const int ch = N.l;
             emit(ch);
             const bool need = nd[ch].on && !vo;
-            const int us = need ? talloc() : usink;
+            bool tb = false;
+            const int us = need ? talloc(tb) : usink;
             Unit u = blank();
-            u.fx = VMF_UN | (need ? VMF_NEED : 0u) | un_bits(N.op);
+            u.tb = tb;
+            u.fx = VMF_UN | (need ? VMF_NEED : 0u) | (tb ? VMF_TB : 0u) | un_bits(N.op);
             u.fy = yf(-1, us, 0, VM_B_SINK, -1, N.op);
             if (N.on) {
                 if (kind(ch) == K_CONST) {
@@ -212,10 +236,12 @@ struct Compiler {
             const int g = NL.l;
             emit(g);
             const bool need = nd[g].on && !vo;
-            const int us = talloc();
+            bool tb = false;
+            const int us = talloc(tb);
             const int bs = need ? balloc() : VM_B_SINK;
             Unit u = blank();
-            u.fx = VMF_UNMC | (need ? VMF_NEED : 0u) | un_bits(NL.op);
+            u.tb = tb;
+            u.fx = VMF_UNMC | (need ? VMF_NEED : 0u) | (tb ? VMF_TB : 0u) | un_bits(NL.op);
             u.fy = yf((int)NR.slot, us, 0, bs, -1, NL.op);
             u.rkind = need ? VMR_UNMC_N : VMR_UNMC_P;
             u.ut = us;
@@ -229,9 +255,11 @@ struct Compiler {
         /* (.) * c */
         if (N.op == O_MUL && NR.op == O_CONST && !leaf(L)) {
             emit(L);
-            const int us = talloc();
+            bool tb = false;
+            const int us = talloc(tb);
             Unit u = blank();
-            u.fx = VMF_MULC;
+            u.tb = tb;
+            u.fx = VMF_MULC | (tb ? VMF_TB : 0u);
             u.fy = yf((int)NR.slot, us, 0, VM_B_SINK, -1, 0);
             u.rkind = NL.on ? VMR_MULC_N : VMR_MULC_P;
             u.ut = us;
@@ -289,7 +317,8 @@ struct Compiler {
             spill.pop_back();
             --depth;
         }
-        const int us = dl ? ualloc() : usink;
+        const int us = dl ? talloc(u.tb) : usink;
+        if (u.tb) fx |= VMF_TB;
         const int bs = dr ? balloc() : VM_B_SINK;
         if (!(fx & (VMF_RC | VMF_RV))) ufree[ur] = true;
         if (dl) fx |= VMF_D0;
@@ -341,7 +370,7 @@ extern "C" {
    p constants; nvars inputs; col_bytes: LDS bytes between gradient columns;
    flags: VMC_* options.
    fwd / rev receive word pairs (2 words each).  info[0..5] = forward pairs,
-   reverse pairs, U slots, B slots, saved-adjoint slots, peak value depth.
+   reverse pairs, U slots, B slots, saved-adjoint slots, LDS slots.
    Returns 0, or -1 malformed records, -2 unsupported operator, -3 the
    program does not fit the VM, -4 an output buffer is too small. */
 int rch_fitvm_compile(const unsigned int *rec, int words, int p, int nvars, int col_bytes,
@@ -411,6 +440,18 @@ int rch_fitvm_compile(const unsigned int *rec, int words, int p, int nvars, int 
         for (int s = 0; s < nvars; ++s) C.ufree[s] = false;
         C.umax = nvars;
     }
+    if ((flags & (VMC_TAPE_B | VMC_TAPE_L)) && !C.vo) {
+        /* The spilled operands' peak: a value-only run keeps nothing else in
+           U (its own overflow is this program's too). */
+        Compiler V = C;
+        V.vo = true;
+        V.emit(m - 1);
+        if (V.overflow) return -3;
+        C.tape_b = (flags & VMC_TAPE_B) != 0;
+        C.tape_l = !C.tape_b;
+        C.reserve = V.umax - C.umax;
+    }
+    if (flags & VMC_SMALL_B) C.bslots = 8;
     C.emit(m - 1);
     if (C.overflow) return -3;
     /* A lone constant: its gradient is the seed. */
@@ -458,6 +499,7 @@ int rch_fitvm_compile(const unsigned int *rec, int words, int p, int nvars, int 
         y |= ((uint32_t)ar & 0x7u) << 19;
         y |= ((uint32_t)(u.xv < 0 ? 0 : u.xv) & 0x7u) << 22;
         y |= (u.rop & 0x1fu) << 25;
+        if (u.tb) y |= VMR_Y_TB;
         rv.push_back(x);
         rv.push_back(y);
         if (u.rkind == VMR_GEN) {
@@ -483,7 +525,7 @@ int rch_fitvm_compile(const unsigned int *rec, int words, int p, int nvars, int 
         info[2] = C.umax;
         info[3] = C.bnext;
         info[4] = apeak;
-        info[5] = 0;
+        info[5] = C.lnext;
     }
     return 0;
 }

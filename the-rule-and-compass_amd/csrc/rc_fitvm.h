@@ -32,6 +32,7 @@
 #define VM_U_SLOTS 16
 #define VM_B_SLOTS 16
 #define VM_A_SLOTS 8
+#define VM_L_SLOTS 16
 #define VM_U_SINK 15
 #define VM_B_SINK 15
 #define VM_A_SINK 7
@@ -41,6 +42,9 @@
 #define VMC_INPUTS_IN_U 1u /* inputs live in U slots 0..nvars-1 (no X file)  */
 #define VMC_VALUE_ONLY 2u  /* forward only: no tape, no reverse stream       */
 #define VMC_SMALL_U 4u     /* an 8-slot U file: slot 7 is the sink           */
+#define VMC_TAPE_B 8u      /* a tape value that finds no U slot takes a B slot */
+#define VMC_SMALL_B 16u    /* an 8-slot B file                               */
+#define VMC_TAPE_L 32u     /* ... takes an LDS slot                          */
 #define VM_U_SINK_SMALL 7
 
 /* ---- forward handlers (x bits 0..9) ------------------------------------ */
@@ -80,6 +84,9 @@
    whose handler does not read ur itself; when the word spills the left
    operand itself, us == ur). */
 #define VMF_ACC (1u << 20)
+/* The tape value this word keeps goes to B[us] (VMC_TAPE_B) or to LDS slot us
+   (VMC_TAPE_L) instead of U[us]. */
+#define VMF_TB (1u << 21)
 
 /* ---- reverse handlers (x bits 0..10) ----------------------------------- */
 /* R_UNMC_N  g = A*U[ut]; A = (A*c)*B[bt]                                    */
@@ -123,7 +130,8 @@
 /* forward:  bits 0..7 c byte offset (slot * 4) | 8..11 us | 12..15 ur |
              16..19 bs | 20..22 xv | 23..27 operator code                  */
 /* reverse:  bits 0..7 c byte offset | 8..11 ut | 12..15 bt | 16..18 as |
-             19..21 ar | 22..24 xv | 25..29 operator code (R_GEN)          */
+             19..21 ar | 22..24 xv | 25..29 operator code (R_GEN) |
+             30 the tape value is in B[ut] or LDS slot ut, not U[ut]        */
 #define VM_Y_COFS(y) ((y) & 0xffu)
 #define VMF_Y_US(y) (((y) >> 8) & 0xfu)
 #define VMF_Y_UR(y) (((y) >> 12) & 0xfu)
@@ -136,6 +144,7 @@
 #define VMR_Y_AR(y) (((y) >> 19) & 0x7u)
 #define VMR_Y_XV(y) (((y) >> 22) & 0x7u)
 #define VMR_Y_OP(y) (((y) >> 25) & 0x1fu)
+#define VMR_Y_TB (1u << 30)
 
 /* R_GEN occupies two word pairs: the first carries the left (or only)
    child's gradient column in x, the second carries the right child's column

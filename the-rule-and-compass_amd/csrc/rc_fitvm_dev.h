@@ -338,15 +338,21 @@ __device__ __forceinline__ uint2 vm_word(const uint2 *__restrict__ s, uint32_t o
 /* Runs the forward stream on one pack of rows.  With TAPE the partials the
    reverse stream reads are left in U and B.  Every step writes U once (the
    sink slot when it has nothing to keep), so no branch join merges two
-   versions of the file. */
-template <typename V, bool TAPE, typename FX, typename FU, typename FB>
+   versions of the file.  TM says where a VMF_TB word's tape value goes
+   instead: nowhere (the stream has none), to B (VMC_TAPE_B) or to the LDS
+   slots at tl, this lane's address of slot 0 (VMC_TAPE_L). */
+enum { VM_TAPE_U = 0, VM_TAPE_B = 1, VM_TAPE_L = 2 };
+/* Bytes of an LDS tape slot: one 16-byte pack for each lane. */
+#define VM_LSLOT 1024u
+template <typename V, bool TAPE, int TM = VM_TAPE_U, typename FX, typename FU, typename FB>
 __device__ __forceinline__ V vm_forward(const uint2 *__restrict__ fc, int nf,
                                         const typename VmScalar<V>::T *__restrict__ cst,
                                         const FX &X0, const FX &X1, const FX &X2, const FX &X3,
                                         FU &U0, FU &U1, FU &U2, FU &U3, FB &B0, FB &B1, FB &B2,
-                                        FB &B3)
+                                        FB &B3, char *tl = nullptr)
 {
     typedef VmPack<V> P;
+    static_assert(TM != VM_TAPE_L || sizeof(V) == 16, "an LDS tape slot holds 16 bytes a lane");
     V tos = vm_bcast<V>(0);
     const uint32_t end = 8u * (uint32_t)nf;
     for (uint32_t o = 0; o < end; o += 8u) {
@@ -409,6 +415,14 @@ __device__ __forceinline__ V vm_forward(const uint2 *__restrict__ fc, int nf,
                 uv = d0;
                 if (x & VMF_D1) P::set(B0, B1, B2, B3, VMF_Y_BS(y), d1);
             }
+        }
+        if (TM != VM_TAPE_U && (x & VMF_TB)) {
+            /* U is written all the same, its sink: two stores of which a
+               branch takes one are merged into one through a selected
+               address, and the files would leave the registers. */
+            if (TM == VM_TAPE_B) P::set(B0, B1, B2, B3, us, uv);
+            else *(V *)(tl + VM_LSLOT * us) = uv;
+            us = VM_U_SINK;
         }
         P::set(U0, U1, U2, U3, us, uv);
         /* After the U write: a word that spills the left operand itself
@@ -481,15 +495,25 @@ template <typename V> __device__ __forceinline__ void vm_gwrite(char *xl, uint32
    (this lane's byte address of row 0, column 0; the stream's column offsets
    were compiled for that block's stride and element size).  Returns the
    finiteness accumulator. */
-template <typename V, typename FU, typename FB, typename FA>
+template <typename V, int TM, typename FU, typename FB, typename FA>
 __device__ __forceinline__ V vm_reverse(const uint2 *__restrict__ rc, int nr, V seed,
                                         const typename VmScalar<V>::T *__restrict__ cst,
                                         const FU &U0, const FU &U1, const FB &B0, const FB &B1,
-                                        FA &A0, FA &A1, char *xl)
+                                        FA &A0, FA &A1, char *xl, const char *tl = nullptr)
 {
     typedef VmPack<V> P;
     typedef typename VmScalar<V>::T T;
     V a = seed, fin = vm_bcast<V>((T)0);
+    /* A word's tape value: U[ut], or where the forward sweep's VMF_TB word put
+       it (TM). */
+    auto tape = [&](uint32_t y) {
+        V t = P::get(U0, U1, U1, U1, VMR_Y_UT(y));
+        if (TM != VM_TAPE_U && (y & VMR_Y_TB)) {
+            if (TM == VM_TAPE_B) t = P::get(B0, B1, B1, B1, VMR_Y_UT(y));
+            else t = *(const V *)(tl + VM_LSLOT * VMR_Y_UT(y));
+        }
+        return t;
+    };
     const uint32_t end = 8u * (uint32_t)nr;
     for (uint32_t o = 0; o < end; o += 8u) {
         const uint2 w = vm_word(rc, o);
@@ -501,23 +525,23 @@ __device__ __forceinline__ V vm_reverse(const uint2 *__restrict__ rc, int nr, V 
             vm_gwrite<V>(xl, x, vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_XV(y)), fin), fin);
             a = P::get(A0, A1, A1, A1, VMR_Y_AR(y));
         } else if (x & VMR_UNMC_N) {
-            vm_gwrite<V>(xl, x, vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_UT(y)), fin), fin);
+            vm_gwrite<V>(xl, x, vm_zmul<V>(a, tape(y), fin), fin);
             a = vm_zmul<V>(vm_zmul<V>(a, vm_const(cst, y), fin), P::get(B0, B1, B1, B1, VMR_Y_BT(y)), fin);
         } else if (x & VMR_MULV) {
             a = vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_XV(y)), fin);
         } else if (x & VMR_ADDC_N) {
             vm_gwrite<V>(xl, x, a, fin);
         } else if (x & VMR_MULC_N) {
-            vm_gwrite<V>(xl, x, vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_UT(y)), fin), fin);
+            vm_gwrite<V>(xl, x, vm_zmul<V>(a, tape(y), fin), fin);
             a = vm_zmul<V>(a, vm_const(cst, y), fin);
         } else if (x & VMR_MULC_P) {
-            vm_gwrite<V>(xl, x, vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_UT(y)), fin), fin);
+            vm_gwrite<V>(xl, x, vm_zmul<V>(a, tape(y), fin), fin);
             a = P::get(A0, A1, A1, A1, VMR_Y_AR(y));
         } else if (x & VMR_UNMC_P) {
-            vm_gwrite<V>(xl, x, vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_UT(y)), fin), fin);
+            vm_gwrite<V>(xl, x, vm_zmul<V>(a, tape(y), fin), fin);
             a = P::get(A0, A1, A1, A1, VMR_Y_AR(y));
         } else if (x & VMR_UN) {
-            a = vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_UT(y)), fin);
+            a = vm_zmul<V>(a, tape(y), fin);
         } else if (x & VMR_ADDC_P) {
             vm_gwrite<V>(xl, x, a, fin);
             a = P::get(A0, A1, A1, A1, VMR_Y_AR(y));
@@ -528,7 +552,7 @@ __device__ __forceinline__ V vm_reverse(const uint2 *__restrict__ rc, int nr, V 
             const unsigned op = VMR_Y_OP(y);
             V gl, gr;
             if (x & VMR_UNARY) {
-                gl = vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_UT(y)), fin);
+                gl = vm_zmul<V>(a, tape(y), fin);
                 gr = gl;
             } else if (op == OP_ADD) {
                 gl = a;
@@ -537,7 +561,7 @@ __device__ __forceinline__ V vm_reverse(const uint2 *__restrict__ rc, int nr, V 
                 gl = a;
                 gr = -a;
             } else {
-                gl = vm_zmul<V>(a, P::get(U0, U1, U1, U1, VMR_Y_UT(y)), fin);
+                gl = vm_zmul<V>(a, tape(y), fin);
                 gr = vm_zmul<V>(a, P::get(B0, B1, B1, B1, VMR_Y_BT(y)), fin);
             }
             if (x & VMR_LCONST) vm_gwrite<V>(xl, x, gl, fin);

@@ -25,8 +25,10 @@
    polish reads each row's f64 prediction from p64 when it is non-null (the
    exact pass at the same constants wrote it there) and otherwise computes it
    on the candidate's value-pass stream; with r = 2 it computes it on the
-   tape stream. */
-void vm_launch_asm(int kc, int r, bool polish, int nl, hipStream_t s, const FtItem *items,
+   tape stream.  tape says how the list's 4-row streams were compiled: 0 the
+   tape in U, 1 with VMC_TAPE_B, 2 with VMC_TAPE_L and at most lslots LDS
+   slots. */
+void vm_launch_asm(int kc, int r, int tape, int lslots, bool polish, int nl, hipStream_t s, const FtItem *items,
                    const int *list, const FtCand *cands, const FtRows *rows, const uint32_t *code,
                    const int *run, const float *cp32, const double *cp64, double *pgram,
                    int tri_stride, double *ploss, int *pbad, int *pskip, const double *p64);

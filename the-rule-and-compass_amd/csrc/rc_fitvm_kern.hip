@@ -79,7 +79,7 @@ template <> struct VmAsmShape<4> {
    lane, and measured 1.9 ms faster per C3 fit than at one wave, with the
    same bits); 2 (R = 4) the f64 prediction read from p64in, where the exact
    pass at the same constants stored what PM = 1 computes. */
-template <int KC, int PM, int R>
+template <int KC, int PM, int R, int TM>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PM != 0 ? 2 : 1))) void vm_asm_kernel(
     const FtItem *__restrict__ items, const int *__restrict__ list, int nlist,
     const FtCand *__restrict__ cands, const FtRows *__restrict__ rowsd,
@@ -120,6 +120,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PM != 0 ? 2 
     const uint2 *fc = (const uint2 *)(code + d.fwd_off);
     const uint2 *rc = (const uint2 *)(code + d.rev_off);
     char *xl = (char *)(X + lane);
+    /* The LDS tape slots (TM == VM_TAPE_L) follow the launch's request. */
+    extern __shared__ __align__(16) char ltape[];
+    char *tl = TM == VM_TAPE_L ? ltape + 16 * lane : nullptr;
     /* KC = 16: acc00 is the Gram block.  KC = 32: acc00 and acc10 are the
        products P and Q of ft_pair_store<6>. */
     floatx4 acc00 = {0, 0, 0, 0}, acc10 = {0, 0, 0, 0};
@@ -155,8 +158,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PM != 0 ? 2 
                 for (int r = 0; r < R; ++r) xv[r] = col[q[r]];
                 P::set(U0, U1, U1, U1, v, xv);
             }
-        const V pred = vm_forward<V, true>(fc, d.m, cst, U0, U1, U1, U1, U0, U1, U1, U1, B0, B1, B1,
-                                           B1);
+        const V pred = vm_forward<V, true, TM>(fc, d.m, cst, U0, U1, U1, U1, U0, U1, U1, U1, B0, B1,
+                                               B1, B1, tl);
         double p64[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) p64[r] = (double)pred[r];
@@ -208,7 +211,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PM != 0 ? 2 
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) seed[r] = a[r].ok ? (float)a[r].s64 : 0.0f;
-        const V fin = vm_reverse<V, FU, FB, FA>(rc, d.nrev, seed, cst, U0, U1, B0, B1, A0, A1, xl);
+        const V fin = vm_reverse<V, TM, FU, FB, FA>(rc, d.nrev, seed, cst, U0, U1, B0, B1, A0, A1,
+                                                    xl, tl);
         bool fix = false;
         bool use[R];
 #pragma unroll
@@ -409,7 +413,7 @@ __global__ __launch_bounds__(64) void vm_asm64_kernel(
             rs[r] = f.s * f.r;
             rho[r] = f.rho;
         }
-        const V fin = vm_reverse<V, FU, FB, FA>(rc, d.nrev, seed, cst, U0, U1, B0, B1, A0, A1, xl);
+        const V fin = vm_reverse<V, VM_TAPE_U, FU, FB, FA>(rc, d.nrev, seed, cst, U0, U1, B0, B1, A0, A1, xl);
         bool fix = false;
         bool use[R];
 #pragma unroll
@@ -574,31 +578,39 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void vm
 
 } /* namespace */
 
-void vm_launch_asm(int kc, int r, bool polish, int nl, hipStream_t s, const FtItem *items,
+void vm_launch_asm(int kc, int r, int tape, int lslots, bool polish, int nl, hipStream_t s, const FtItem *items,
                    const int *list, const FtCand *cands, const FtRows *rows, const uint32_t *code,
                    const int *run, const float *cp32, const double *cp64, double *pgram,
                    int tri_stride, double *ploss, int *pbad, int *pskip, const double *p64)
 {
     if (nl <= 0) return;
-#define VM_ASM(KC, PM, R)                                                                       \
-    vm_asm_kernel<KC, PM, R><<<nl, 64, 0, s>>>(items, list, nl, cands, rows, code, run, cp32, cp64, \
-                                              pgram, tri_stride, ploss, pbad, pskip, p64)
-    if (polish && r == 4 && p64) {
-        if (kc == 16) VM_ASM(16, 2, 4);
-        else VM_ASM(32, 2, 4);
-    } else if (polish && r == 4) {
-        if (kc == 16) VM_ASM(16, 1, 4);
-        else VM_ASM(32, 1, 4);
-    } else if (polish) {
-        if (kc == 16) VM_ASM(16, 1, 2);
-        else VM_ASM(32, 1, 2);
-    } else if (r == 4) {
-        if (kc == 16) VM_ASM(16, 0, 4);
-        else VM_ASM(32, 0, 4);
+#define VM_ASM(KC, PM, R, TM)                                                                  \
+    vm_asm_kernel<KC, PM, R, TM><<<nl, 64, TM == VM_TAPE_L ? VM_LSLOT * lslots : 0, s>>>(       \
+        items, list, nl, cands, rows, code, run, cp32, cp64, pgram, tri_stride, ploss, pbad,    \
+        pskip, p64)
+#define VM_ASM_KC(PM, R, TM)                                                                   \
+    do {                                                                                       \
+        if (kc == 16) VM_ASM(16, PM, R, TM);                                                   \
+        else VM_ASM(32, PM, R, TM);                                                            \
+    } while (0)
+#define VM_ASM_PM(TM)                                                                          \
+    do {                                                                                       \
+        if (polish && p64) VM_ASM_KC(2, 4, TM);                                                \
+        else if (polish) VM_ASM_KC(1, 4, TM);                                                  \
+        else VM_ASM_KC(0, 4, TM);                                                              \
+    } while (0)
+    if (r == 2) {
+        if (polish) VM_ASM_KC(1, 2, VM_TAPE_U);
+        else VM_ASM_KC(0, 2, VM_TAPE_U);
+    } else if (tape == VM_TAPE_B) {
+        VM_ASM_PM(VM_TAPE_B);
+    } else if (tape == VM_TAPE_L) {
+        VM_ASM_PM(VM_TAPE_L);
     } else {
-        if (kc == 16) VM_ASM(16, 0, 2);
-        else VM_ASM(32, 0, 2);
+        VM_ASM_PM(VM_TAPE_U);
     }
+#undef VM_ASM_PM
+#undef VM_ASM_KC
 #undef VM_ASM
 }
 
