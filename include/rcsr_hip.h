@@ -238,7 +238,9 @@ int rc_set_fit_mode(void *ctx, int mode);
    the built-in choice.  A candidate's results depend on its own program and
    rows and on these shapes, never on the rest of its batch.
      RC_TUNE_FIT_TILE_ROWS      rows per fit work item: a multiple of 256 in
-                                [256, 4194304] (built-in 8192)
+                                [256, 4194304] (built-in: 8192 where the
+                                batch makes enough of those, else 512 to 2048
+                                by the row count, with the same sums)
      RC_TUNE_FIT_ROWS_PER_LANE  rows per lane of the fit VM assembly: 4 where
                                 the program fits the 4-row files (built-in) or 2
      RC_TUNE_EVAL_TILE_ROWS     rows per evaluation tile: a multiple of 256 in

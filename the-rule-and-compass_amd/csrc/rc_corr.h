@@ -28,6 +28,7 @@ struct CrCand {
     int k;            /* constants */
     int vm;           /* 1: the fit VM streams, 0: the records */
     int item0, nitems;
+    int sub, group;   /* rows of a sub-tile, items of a group (RcSplit) */
     int pre;          /* >= 0: a status decided on the host */
     int gs, go;       /* gauge slots (scale, offset), -1 for none */
 };

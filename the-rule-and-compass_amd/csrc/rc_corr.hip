@@ -31,7 +31,6 @@
 
 namespace {
 
-constexpr int CR_TILE = 8192;
 constexpr int CR_POLISH = 4;
 
 /* Candidate stages. */
@@ -190,7 +189,7 @@ __global__ __launch_bounds__(64) void cr_ctrl_kernel(
     if (asm_step) {
         const int q = p + 3;
         for (int t = lane; t < q * (q + 1) / 2; t += 64)
-            G[t] = rc_ordered_sum(pgram + (size_t)d.item0 * CR_TRI + t, CR_TRI, d.nitems);
+            G[t] = rc_grouped_sum(pgram + (size_t)d.item0 * CR_TRI + t, CR_TRI, d.nitems, d.group);
     }
     if (lane == 0) {
         int b = 0;
@@ -198,7 +197,8 @@ __global__ __launch_bounds__(64) void cr_ctrl_kernel(
         if (score_step) {
             b |= rc_batched_or(pbad_s + d.item0, d.nitems);
             for (int qd = 0; qd < CR_NMOM; ++qd)
-                sh_mom[qd] = rc_ordered_sum(pmom + (size_t)d.item0 * CR_NMOM + qd, CR_NMOM, d.nitems);
+                sh_mom[qd] = rc_grouped_sum(pmom + (size_t)d.item0 * CR_NMOM + qd, CR_NMOM,
+                                            d.nitems, d.group);
         }
         sh_bad = b;
     }
@@ -462,7 +462,9 @@ int rc_corr_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const int *
     std::vector<FtItem> items;
     enum { NA = 4, NS = 2 };
     std::vector<int> alist[NA], slist[NS];
-    const int tile = c->tune_fit_tile > 0 ? c->tune_fit_tile : CR_TILE;
+    const RcSplit sp =
+        rc_split(r->n, nprog * rc_groups_of(r->n) >= RC_ITEMS_WANTED, c->tune_fit_tile);
+    const int tile = sp.rows;
     for (int i = 0; i < nprog; ++i) {
         CrCand &d = cands[i];
         if (d.pre >= 0) continue;
@@ -485,6 +487,8 @@ int rc_corr_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const int *
         const int kc = d.k + 3 <= 16 ? 0 : 1;
         const int acls = (d.vm ? 0 : 2) + kc;
         d.item0 = (int)items.size();
+        d.sub = sp.sub;
+        d.group = sp.group;
         for (int r0 = 0; r0 < r->n; r0 += tile) {
             FtItem it;
             it.cand = i;

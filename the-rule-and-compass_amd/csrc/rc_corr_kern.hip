@@ -75,6 +75,8 @@ __global__ __launch_bounds__(64) void cr_asm_kernel(
     dv16 U0 = (dv16)(0.0), U1 = U0, B0 = U0, B1 = U0;
     dv8 A0 = (dv8)(0.0), A1 = A0;
     const int row_end = it.row0 + it.rows;
+    double *pg = pgram + (size_t)item * CR_TRI;
+    int sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += BLOCK) {
         int rq[R];
         bool in[R];
@@ -162,16 +164,22 @@ __global__ __launch_bounds__(64) void cr_asm_kernel(
             }
         }
         __syncthreads();
-    }
-    /* FP64 MFMA output: lane l, register r holds D[l/16 + 4 r][l % 16] of
-       each 16x16 block. */
-    double *pg = pgram + (size_t)item * CR_TRI;
-    const int j = lane & 15;
+        /* The end of a sub-tile: its sums go onto the item's.  FP64 MFMA
+           output: lane l, register r holds D[l/16 + 4 r][l % 16] of each
+           16x16 block. */
+        if (base + BLOCK >= sub_end || base + BLOCK >= row_end) {
+            const bool add = sub_end != it.row0 + d.sub;
+            const int j = lane & 15;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = (lane >> 4) + 4 * r;
-        if (KC == 16 && i >= j && i < q) pg[i * (i + 1) / 2 + j] = acc00[r];
-        if (KC == 32) ft_pair_store<PS>(pg, i, j, q, acc00[r], acc10[r]);
+            for (int r = 0; r < 4; ++r) {
+                const int i = (lane >> 4) + 4 * r;
+                if (KC == 16 && i >= j && i < q) rc_put(pg + i * (i + 1) / 2 + j, acc00[r], add);
+                if (KC == 32) ft_pair_store<PS>(pg, i, j, q, acc00[r], acc10[r], add);
+                acc00[r] = 0.0;
+                if (KC == 32) acc10[r] = 0.0;
+            }
+            sub_end += d.sub;
+        }
     }
     const int anybad = __any(bad) ? 1 : 0;
     if (lane == 0) pbad[item] = anybad;
@@ -200,6 +208,15 @@ __global__ __launch_bounds__(64) void cr_score_kernel(
     int bad = 0;
     dv8 U0 = (dv8)(0.0), U1 = U0, U2 = U0, U3 = U0, Bd = U0;
     const int row_end = it.row0 + it.rows;
+    double out[CR_NMOM] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int sub_end = it.row0 + d.sub;
+    auto take = [&]() {
+#pragma unroll
+        for (int qd = 0; qd < CR_NMOM; ++qd) {
+            out[qd] += rc_wave_sum_f64(mo[qd]);
+            mo[qd] = 0.0;
+        }
+    };
     for (int base = it.row0; base < row_end; base += 64 * R) {
         int rq[R];
         bool in[R];
@@ -244,10 +261,12 @@ __global__ __launch_bounds__(64) void cr_score_kernel(
             mo[4] += wb * y;
             mo[5] += wb * y * y;
         }
+        if (base + 64 * R >= sub_end) {
+            take();
+            sub_end += d.sub;
+        }
     }
-    double out[CR_NMOM];
-#pragma unroll
-    for (int qd = 0; qd < CR_NMOM; ++qd) out[qd] = rc_wave_sum_f64(mo[qd]);
+    if (sub_end - d.sub < row_end) take();
     const int anybad = __any(bad) ? 1 : 0;
     if (lane == 0) {
 #pragma unroll

@@ -312,6 +312,34 @@ __device__ __forceinline__ double rc_ordered_sum(const double *__restrict__ p, s
     return acc;
 }
 
+/* The same with every `group` items summed by themselves first (RcSplit). */
+__device__ __forceinline__ double rc_grouped_sum(const double *__restrict__ p, size_t stride, int n,
+                                                 int group)
+{
+    if (group == 1) return rc_ordered_sum(p, stride, n);
+    double acc = 0.0, part = 0.0;
+    int left = group;
+    for (int t0 = 0; t0 < n; t0 += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[(size_t)min(t0 + u, n - 1) * stride];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (t0 + u < n) {
+                part += v[u];
+                if (--left == 0) {
+                    acc += part;
+                    part = 0.0;
+                    left = group;
+                }
+            }
+    }
+    return left < group ? acc + part : acc;
+}
+
+/* A sub-tile's sum into an item's partial: the first stores, the others add. */
+__device__ __forceinline__ void rc_put(double *p, double v, bool add) { *p = add ? *p + v : v; }
+
 /* p[0] | p[1] | ... | p[n - 1], n >= 0, loads issued eight at a time. */
 __device__ __forceinline__ int rc_batched_or(const int *__restrict__ p, int n)
 {

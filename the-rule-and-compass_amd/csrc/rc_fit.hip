@@ -9,9 +9,9 @@
  * MI355X design.  The reference runs one thread block per candidate for the
  * whole fit, so a candidate's rows are limited to one SM and uneven candidates
  * leave SMs idle.  Here every LM iteration is a short sequence of batch-wide
- * launches over work items (candidate, 8192-row tile), so all 256 CUs share
- * every pass whatever the mix of program lengths, constant counts and row
- * counts:
+ * launches over work items (candidate, row tile of up to 8192; RcSplit), so
+ * all 256 CUs share every pass whatever the mix of program lengths, constant
+ * counts and row counts:
  *   ft_asm_kernel    f32 forward + adjoint per row (one wave per item), the
  *                    augmented row [s*J | s*r_hi | s*r_lo] written to LDS and
  *                    reduced on FP32 MFMA (v_mfma_f32_16x16x4f32): J^T J,
@@ -44,7 +44,6 @@
 namespace {
 
 constexpr int XS = 66;          /* LDS column stride of the augmented rows */
-constexpr int TILE_ROWS = 8192; /* built-in rows per work item (a multiple of 256) */
 /* Largest f64 prediction buffer of a fit (bytes): 8 bytes per row of every
    candidate; 1024 candidates over 262 144 rows take 2 GiB. */
 constexpr size_t FT_P64_CAP = (size_t)32 << 30;
@@ -390,7 +389,10 @@ __global__ __launch_bounds__(64) void ft_asm_kernel(
     double lsum = 0.0;
     int bad = 0, skip = 0;
     const int row_end = it.row0 + it.rows;
-    int step = 0;
+    const int K = k + 2;
+    double *pg = pgram + (size_t)item * (size_t)tri_stride;
+    double ltot = 0.0;
+    int step = 0, sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += 64, ++step) {
         const int row = base + lane;
         bool live = row < row_end;
@@ -461,35 +463,40 @@ __global__ __launch_bounds__(64) void ft_asm_kernel(
                 }
             }
         }
-    }
+        /* The end of a sub-tile: its sums go onto the item's.  Lane l,
+           register r holds D[4*(l/16) + r][l % 16] of each 16x16 block. */
+        if (base + 64 >= sub_end || base + 64 >= row_end) {
+            const bool add = sub_end != it.row0 + d.sub;
+            const int j = lane & 15;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        g00[r] += (double)acc00[r];
-        if (KC == 32) {
-            g10[r] += (double)acc10[r];
-            g11[r] += (double)acc11[r];
+            for (int r = 0; r < 4; ++r) {
+                const int i = 4 * (lane >> 4) + r;
+                g00[r] += (double)acc00[r];
+                acc00[r] = 0.0f;
+                if (i >= j && i < K) rc_put(pg + i * (i + 1) / 2 + j, g00[r], add);
+                g00[r] = 0.0;
+                if (KC == 32) {
+                    const int i1 = 16 + i;
+                    g10[r] += (double)acc10[r];
+                    g11[r] += (double)acc11[r];
+                    acc10[r] = 0.0f;
+                    acc11[r] = 0.0f;
+                    if (i1 < K) rc_put(pg + i1 * (i1 + 1) / 2 + j, g10[r], add);
+                    if (i >= j && i1 < K) rc_put(pg + i1 * (i1 + 1) / 2 + 16 + j, g11[r], add);
+                    g10[r] = 0.0;
+                    g11[r] = 0.0;
+                }
+            }
+            ltot += rc_wave_sum_f64(lsum);
+            lsum = 0.0;
+            sub_end += d.sub;
         }
     }
-    /* Lane l, register r holds D[4*(l/16) + r][l % 16] of each 16x16 block. */
-    const int K = k + 2;
-    double *pg = pgram + (size_t)item * (size_t)tri_stride;
-    const int j = lane & 15;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = 4 * (lane >> 4) + r;
-        if (i >= j && i < K) pg[i * (i + 1) / 2 + j] = g00[r];
-        if (KC == 32) {
-            const int i1 = 16 + i;
-            if (i1 < K) pg[i1 * (i1 + 1) / 2 + j] = g10[r];
-            if (i >= j && i1 < K) pg[i1 * (i1 + 1) / 2 + 16 + j] = g11[r];
-        }
-    }
-    const double ls = rc_wave_sum_f64(lsum);
     int sk = skip;
     for (int off = 32; off > 0; off >>= 1) sk += __shfl_xor(sk, off, 64);
     const int anybad = __any(bad) ? 1 : 0;
     if (lane == 0) {
-        ploss[item] = ls;
+        ploss[item] = ltot;
         pbad[item] = anybad;
         pskip[item] = sk;
     }
@@ -532,6 +539,10 @@ __global__ __launch_bounds__(64) void ft_asm64_kernel(
     double lsum = 0.0;
     int bad = 0, skip = 0;
     const int row_end = it.row0 + it.rows;
+    const int K = k + 2;
+    double *pg = pgram + (size_t)item * (size_t)tri_stride;
+    double ltot = 0.0;
+    int sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += 64) {
         const int row = base + lane;
         bool live = row < row_end;
@@ -577,27 +588,34 @@ __global__ __launch_bounds__(64) void ft_asm64_kernel(
             }
         }
         __syncthreads();
-    }
-    /* FP64 MFMA output: lane l, register r holds D[l/16 + 4 r][l % 16]. */
-    const int K = k + 2;
-    double *pg = pgram + (size_t)item * (size_t)tri_stride;
-    const int j = lane & 15;
+        /* The end of a sub-tile: its sums go onto the item's.  FP64 MFMA
+           output: lane l, register r holds D[l/16 + 4 r][l % 16]. */
+        if (base + 64 >= sub_end || base + 64 >= row_end) {
+            const bool add = sub_end != it.row0 + d.sub;
+            const int j = lane & 15;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = (lane >> 4) + 4 * r;
-        if (i >= j && i < K) pg[i * (i + 1) / 2 + j] = acc00[r];
-        if (KC == 32) {
-            const int i1 = 16 + i;
-            if (i1 < K) pg[i1 * (i1 + 1) / 2 + j] = acc10[r];
-            if (i >= j && i1 < K) pg[i1 * (i1 + 1) / 2 + 16 + j] = acc11[r];
+            for (int r = 0; r < 4; ++r) {
+                const int i = (lane >> 4) + 4 * r;
+                if (i >= j && i < K) rc_put(pg + i * (i + 1) / 2 + j, acc00[r], add);
+                acc00[r] = 0.0;
+                if (KC == 32) {
+                    const int i1 = 16 + i;
+                    if (i1 < K) rc_put(pg + i1 * (i1 + 1) / 2 + j, acc10[r], add);
+                    if (i >= j && i1 < K) rc_put(pg + i1 * (i1 + 1) / 2 + 16 + j, acc11[r], add);
+                    acc10[r] = 0.0;
+                    acc11[r] = 0.0;
+                }
+            }
+            ltot += rc_wave_sum_f64(lsum);
+            lsum = 0.0;
+            sub_end += d.sub;
         }
     }
-    const double ls = rc_wave_sum_f64(lsum);
     int sk = skip;
     for (int off = 32; off > 0; off >>= 1) sk += __shfl_xor(sk, off, 64);
     const int anybad = __any(bad) ? 1 : 0;
     if (lane == 0) {
-        ploss[item] = ls;
+        ploss[item] = ltot;
         pbad[item] = anybad;
         pskip[item] = sk;
     }
@@ -632,6 +650,8 @@ __global__ __launch_bounds__(64) void ft_trial_kernel(
     else cols = (const T *)(const void *)R_.cols64;
     double lsum = 0.0;
     const int row_end = it.row0 + it.rows;
+    double ltot = 0.0;
+    int sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += 64 * R) {
         int xrow[R];
         bool live[R];
@@ -653,9 +673,14 @@ __global__ __launch_bounds__(64) void ft_trial_kernel(
             if (sizeof(T) == 4) hard = hard || fabs((double)pred[r]) > 1e30;
             lsum += hard ? 1e30 : wb * rc_row_stat((double)pred[r], yr, d.metric);
         }
+        if (base + 64 * R >= sub_end) {
+            ltot += rc_wave_sum_f64(lsum);
+            lsum = 0.0;
+            sub_end += d.sub;
+        }
     }
-    const double ls = rc_wave_sum_f64(lsum);
-    if (lane == 0) ploss[item] = ls;
+    if (sub_end - d.sub < row_end) ltot += rc_wave_sum_f64(lsum);
+    if (lane == 0) ploss[item] = ltot;
 }
 
 /* ---- per-row probe (test hook): pred, constant and input gradients -------- */
@@ -761,8 +786,8 @@ __global__ __launch_bounds__(64) void ft_ctrl_kernel(
                             ran_trial) || want_gram;
     if (want_gram) {
         for (int q = lane; q < tri; q += 64)
-            G[q] = rc_ordered_sum(pgram + (size_t)d.item0 * (size_t)tri_stride + q,
-                                  (size_t)tri_stride, d.nitems);
+            G[q] = rc_grouped_sum(pgram + (size_t)d.item0 * (size_t)tri_stride + q,
+                                  (size_t)tri_stride, d.nitems, d.group);
     }
     if (lane == 0 && want_gram) s->n_asm += 1;
     if (lane == 0 && want_loss && !want_gram) {
@@ -788,7 +813,7 @@ __global__ __launch_bounds__(64) void ft_ctrl_kernel(
                     }
             }
         }
-        sh_loss = rc_ordered_sum(ploss + d.item0, 1, d.nitems);
+        sh_loss = rc_grouped_sum(ploss + d.item0, 1, d.nitems, d.group);
         sh_bad = b;
         sh_skip = sk;
     }
@@ -1131,7 +1156,7 @@ __global__ void ft_trial_prune(int nprog, FtState *__restrict__ S, const FtCand 
     if (run_t[c] && st->stage == ST_NEED_TRIAL && isfinite(st->best)) {
         const FtCand d = cands[c];
         const int h = (d.nitems + 1) / 2;
-        pr = rc_ordered_sum(ploss + d.item0, 1, h) >= st->best ? 1 : 0;
+        pr = rc_grouped_sum(ploss + d.item0, 1, h, d.group) >= st->best ? 1 : 0;
     }
     st->pruned = pr;
     run_b[c] = (run_t[c] && !pr) ? 1 : 0;
@@ -1571,7 +1596,9 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
     std::vector<int> tlist_a[NT], tlist_b[NT];
     int maxK = 2;
     int lslots[2] = {0, 0}; /* LDS tape slots of classes 10 and 11 */
-    const int tile_rows = c->tune_fit_tile > 0 ? c->tune_fit_tile : TILE_ROWS;
+    long long groups = 0;
+    for (int i = 0; i < nprog; ++i)
+        if (progs[i].pre_status < 0) groups += rc_groups_of(c->sets[rowset[i]].n);
     size_t p64_blocks = 0; /* f64 prediction buffer, in 64-row blocks */
     for (int i = 0; i < nprog; ++i) {
         FtCand &d = cands[i];
@@ -1615,6 +1642,10 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
             tcls = progs[i].max_stack > SMALL_S ? 2 : 1;
         }
         const int n = c->sets[rowset[i]].n;
+        const RcSplit sp = rc_split(n, groups >= RC_ITEMS_WANTED, c->tune_fit_tile);
+        const int tile_rows = sp.rows;
+        d.sub = sp.sub;
+        d.group = sp.group;
         d.item0 = (int)items.size();
         const bool big = prog_is_big(progs[i]);
         const int kc = d.k + 2 <= 16 ? 0 : 1;

@@ -52,6 +52,8 @@ struct FtCand {
     int metric;
     int item0;   /* first work item */
     int nitems;
+    int sub;     /* rows of a sub-tile, items of a group (RcSplit) */
+    int group;
     int vm;      /* 1: fit VM code (word pairs, m / nrev count pairs) */
     uint32_t t_off; /* value-pass stream (trial and exact losses) */
     int t_m;        /* its instruction count */
@@ -65,15 +67,16 @@ struct FtCand {
    a >= 8 and b < 16, else from Q (both below 8 or both at least 16), so
    every entry is stored once and is the same dot product over the same rows
    as in the blockwise Gram.  (i, j) is the caller's position in both
-   products. */
+   products; add: onto what the entries hold. */
 template <int S>
-__device__ __forceinline__ void ft_pair_store(double *pg, int i, int j, int K, double p, double q)
+__device__ __forceinline__ void ft_pair_store(double *pg, int i, int j, int K, double p, double q,
+                                              bool add)
 {
     static_assert(S >= 0 && S <= 8, "Q covers the columns below 8 and from 16");
     const int a = S + j;
-    if (a >= 8 && i <= a && a < K) pg[a * (a + 1) / 2 + i] = p;
+    if (a >= 8 && i <= a && a < K) rc_put(pg + a * (a + 1) / 2 + i, p, add);
     const int ci = i < 8 ? i : 8 + i, cj = j < 8 ? j : 8 + j;
-    if (i >= j && ci < K && (ci < 8 || cj >= 16)) pg[ci * (ci + 1) / 2 + cj] = q;
+    if (i >= j && ci < K && (ci < 8 || cj >= 16)) rc_put(pg + ci * (ci + 1) / 2 + cj, q, add);
 }
 
 /* One resident row set as the kernels see it. */

@@ -134,7 +134,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PM != 0 ? 2 
     FA A0 = (FA)(0), A1 = A0;
     const int row_end = it.row0 + it.rows;
     const bool unit_w = Rw.w64 == nullptr && d.metric == RC_LOSS_SQUARED;
-    int step = 0;
+    const int K = k + 2;
+    double *pg = pgram + (size_t)item * (size_t)tri_stride;
+    double ltot = 0.0;
+    int step = 0, sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += BLOCK, ++step) {
         int q[R];
         bool in[R];
@@ -300,27 +303,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PM != 0 ? 2 
                 }
             }
         }
-    }
+        /* The end of a sub-tile: its sums go onto the item's. */
+        if (base + BLOCK >= sub_end || base + BLOCK >= row_end) {
+            const bool add = sub_end != it.row0 + d.sub;
+            const int j = lane & 15;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        g00[r] += (double)acc00[r];
-        if (KC == 32) g10[r] += (double)acc10[r];
+            for (int r = 0; r < 4; ++r) {
+                const int i = 4 * (lane >> 4) + r;
+                g00[r] += (double)acc00[r];
+                acc00[r] = 0.0f;
+                if (KC == 32) {
+                    g10[r] += (double)acc10[r];
+                    acc10[r] = 0.0f;
+                }
+                if (KC == 16 && i >= j && i < K) rc_put(pg + i * (i + 1) / 2 + j, g00[r], add);
+                if (KC == 32) ft_pair_store<6>(pg, i, j, K, g00[r], g10[r], add);
+                g00[r] = 0.0;
+                if (KC == 32) g10[r] = 0.0;
+            }
+            ltot += rc_wave_sum_f64(lsum);
+            lsum = 0.0;
+            sub_end += d.sub;
+        }
     }
-    const int K = k + 2;
-    double *pg = pgram + (size_t)item * (size_t)tri_stride;
-    const int j = lane & 15;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = 4 * (lane >> 4) + r;
-        if (KC == 16 && i >= j && i < K) pg[i * (i + 1) / 2 + j] = g00[r];
-        if (KC == 32) ft_pair_store<6>(pg, i, j, K, g00[r], g10[r]);
-    }
-    const double ls = rc_wave_sum_f64(lsum);
     int sk = skip;
     for (int off = 32; off > 0; off >>= 1) sk += __shfl_xor(sk, off, 64);
     const int anybad = __any(bad) ? 1 : 0;
     if (lane == 0) {
-        ploss[item] = ls;
+        ploss[item] = ltot;
         pbad[item] = anybad;
         pskip[item] = sk;
     }
@@ -381,6 +391,10 @@ __global__ __launch_bounds__(64) void vm_asm64_kernel(
     FB B0 = (FB)(0.0), B1 = B0;
     FA A0 = (FA)(0.0), A1 = A0;
     const int row_end = it.row0 + it.rows;
+    const int K = k + 2;
+    double *pg = pgram + (size_t)item * (size_t)tri_stride;
+    double ltot = 0.0;
+    int sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += BLOCK) {
         int q[R];
         bool in[R];
@@ -457,24 +471,30 @@ __global__ __launch_bounds__(64) void vm_asm64_kernel(
             }
         }
         __syncthreads();
-    }
-    /* FP64 MFMA output: lane l, register r holds D[l/16 + 4 r][l % 16] of
-       each 16x16 block (not the FP32 form's 4 (l/16) + r). */
-    const int K = k + 2;
-    double *pg = pgram + (size_t)item * (size_t)tri_stride;
-    const int j = lane & 15;
+        /* The end of a sub-tile: its sums go onto the item's.  FP64 MFMA
+           output: lane l, register r holds D[l/16 + 4 r][l % 16] of each
+           16x16 block (not the FP32 form's 4 (l/16) + r). */
+        if (base + BLOCK >= sub_end || base + BLOCK >= row_end) {
+            const bool add = sub_end != it.row0 + d.sub;
+            const int j = lane & 15;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = (lane >> 4) + 4 * r;
-        if (KC == 16 && i >= j && i < K) pg[i * (i + 1) / 2 + j] = acc00[r];
-        if (KC == 32) ft_pair_store<6>(pg, i, j, K, acc00[r], acc10[r]);
+            for (int r = 0; r < 4; ++r) {
+                const int i = (lane >> 4) + 4 * r;
+                if (KC == 16 && i >= j && i < K) rc_put(pg + i * (i + 1) / 2 + j, acc00[r], add);
+                if (KC == 32) ft_pair_store<6>(pg, i, j, K, acc00[r], acc10[r], add);
+                acc00[r] = 0.0;
+                if (KC == 32) acc10[r] = 0.0;
+            }
+            ltot += rc_wave_sum_f64(lsum);
+            lsum = 0.0;
+            sub_end += d.sub;
+        }
     }
-    const double ls = rc_wave_sum_f64(lsum);
     int sk = skip;
     for (int off = 32; off > 0; off >>= 1) sk += __shfl_xor(sk, off, 64);
     const int anybad = __any(bad) ? 1 : 0;
     if (lane == 0) {
-        ploss[item] = ls;
+        ploss[item] = ltot;
         pbad[item] = anybad;
         pskip[item] = sk;
     }
@@ -513,6 +533,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void vm
     double lsum = 0.0;
     const bool sq_unit = d.metric == RC_LOSS_SQUARED && R_.w64 == nullptr;
     const int row_end = it.row0 + it.rows;
+    double ltot = 0.0;
+    int sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += 64 * RR) {
         int xrow[RR];
         bool live[RR];
@@ -571,9 +593,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void vm
                 lsum += (live[r] && wb > 0.0) ? term : 0.0;
             }
         }
+        if (base + 64 * RR >= sub_end) {
+            ltot += rc_wave_sum_f64(lsum);
+            lsum = 0.0;
+            sub_end += d.sub;
+        }
     }
-    const double ls = rc_wave_sum_f64(lsum);
-    if (lane == 0) ploss[item] = ls;
+    if (sub_end - d.sub < row_end) ltot += rc_wave_sum_f64(lsum);
+    if (lane == 0) ploss[item] = ltot;
 }
 
 } /* namespace */

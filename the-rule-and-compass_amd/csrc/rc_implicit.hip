@@ -12,7 +12,7 @@
  *   d        undefined when f, a gradient component, the norm or d is not
  *            finite, or the norm is not positive (signed_distance 68-96).
  *
- * Layout.  Work items are (candidate, 8192-row tile) with one wave each; a
+ * Layout.  Work items are (candidate, row tile; RcSplit) with one wave each; a
  * lane walks its rows of the tile and evaluates the candidate's post-order
  * records (the rch_fit_plan form) with per-lane value and adjoint arrays.
  * Three kinds of pass:
@@ -40,7 +40,6 @@
 
 namespace {
 
-constexpr int IM_TILE = 8192;
 constexpr int IM_MAX_NODES = 96;
 constexpr int IM_KMAX = 20;
 constexpr int IM_STATS = (IM_KMAX + 1) * (IM_KMAX + 2) / 2; /* [J | r] lower triangle */
@@ -53,6 +52,8 @@ struct ImCand {
     int m;        /* nodes */
     int k;        /* constants */
     int fast;     /* 1: runs the register-stack sweep (im_fast_kernel) */
+    int sub;      /* rows of a sub-tile, items of a group (RcSplit) */
+    int group;
 };
 
 /* The register-stack sweep's limits: values below the top of the stack
@@ -275,6 +276,9 @@ __global__ __launch_bounds__(64) void im_pass_kernel(
     double s0 = 0.0, s1 = 0.0;
     int flag = 0;
     const int row_end = it.row0 + it.rows;
+    double *p = part + (size_t)it_i * (size_t)pstride;
+    double t0 = 0.0, t1 = 0.0;
+    int sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += 64) {
         const int row = base + lane;
         const bool live = row < row_end;
@@ -339,22 +343,28 @@ __global__ __launch_bounds__(64) void im_pass_kernel(
             }
             __syncthreads();
         }
+        /* The end of a sub-tile: its sums go onto the item's. */
+        if (base + 64 >= sub_end || base + 64 >= row_end) {
+            const bool add = sub_end != it.row0 + d.sub;
+            if (MODE == IM_JAC) {
+                for (int q = 0; q < 4; ++q) {
+                    const int s = lane + 64 * q;
+                    if (s < nstats) rc_put(p + s, acc[q], add);
+                    acc[q] = 0.0;
+                }
+            } else {
+                t0 += rc_wave_sum_f64(s0);
+                t1 += rc_wave_sum_f64(s1);
+                s0 = s1 = 0.0;
+            }
+            sub_end += d.sub;
+        }
     }
-    double *p = part + (size_t)it_i * (size_t)pstride;
     int f = flag;
     for (int off = 32; off > 0; off >>= 1) f |= __shfl_xor(f, off, 64);
-    if (MODE == IM_JAC) {
-        for (int q = 0; q < 4; ++q) {
-            const int s = lane + 64 * q;
-            if (s < nstats) p[s] = acc[q];
-        }
-    } else {
-        const double t0 = rc_wave_sum_f64(s0);
-        const double t1 = rc_wave_sum_f64(s1);
-        if (lane == 0) {
-            p[0] = t0;
-            p[1] = t1;
-        }
+    if (MODE != IM_JAC && lane == 0) {
+        p[0] = t0;
+        p[1] = t1;
     }
     if (lane == 0) bad[it_i] = f;
 }
@@ -565,7 +575,7 @@ __device__ __forceinline__ bool im_fast_distance(const uint32_t *__restrict__ r4
    fast (the general kernel skips them, this one skips the others); NV is
    the row set's input count. */
 template <int MODE, int NV>
-__global__ __launch_bounds__(64) void im_fast_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void im_fast_kernel(
     const ImItem *__restrict__ items, int nitems, const ImCand *__restrict__ cands,
     const uint32_t *__restrict__ rec, const double *__restrict__ cs, int kmax,
     const double *__restrict__ cols64, const double *__restrict__ w64, int n, int metric,
@@ -593,6 +603,9 @@ __global__ __launch_bounds__(64) void im_fast_kernel(
     double s0 = 0.0, s1 = 0.0;
     int flag = 0;
     const int row_end = it.row0 + it.rows;
+    double *p = part + (size_t)it_i * (size_t)pstride;
+    double t0 = 0.0, t1 = 0.0;
+    int sub_end = it.row0 + d.sub;
     for (int base = it.row0; base < row_end; base += 64) {
         const int row = base + lane;
         const bool live = row < row_end;
@@ -671,30 +684,34 @@ __global__ __launch_bounds__(64) void im_fast_kernel(
             }
             __syncthreads();
         }
+        /* The end of a sub-tile: its sums go onto the item's.  FP64 MFMA
+           output: lane l, register r holds D[l/16 + 4 r][l % 16] of each
+           16x16 block; p is the packed lower triangle a (a + 1) / 2 + b. */
+        if (base + 64 >= sub_end || base + 64 >= row_end) {
+            const bool add = sub_end != it.row0 + d.sub;
+            if (MODE == IM_JAC) {
+                const int jj = lane & 15;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int ii = (lane >> 4) + 4 * r, i1 = 16 + ii;
+                    if (ii >= jj && ii < K1) rc_put(p + ii * (ii + 1) / 2 + jj, acc00[r], add);
+                    if (i1 < K1) rc_put(p + i1 * (i1 + 1) / 2 + jj, acc10[r], add);
+                    if (ii >= jj && i1 < K1) rc_put(p + i1 * (i1 + 1) / 2 + 16 + jj, acc11[r], add);
+                    acc00[r] = acc10[r] = acc11[r] = 0.0;
+                }
+            } else {
+                t0 += rc_wave_sum_f64(s0);
+                t1 += rc_wave_sum_f64(s1);
+                s0 = s1 = 0.0;
+            }
+            sub_end += d.sub;
+        }
     }
-    double *p = part + (size_t)it_i * (size_t)pstride;
     int f = flag;
     for (int off = 32; off > 0; off >>= 1) f |= __shfl_xor(f, off, 64);
-    if (MODE == IM_JAC) {
-        /* FP64 MFMA output: lane l, register r holds D[l/16 + 4 r][l % 16]
-           of each 16x16 block; p is the packed lower triangle
-           a (a + 1) / 2 + b. */
-        const int jj = lane & 15;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int ii = (lane >> 4) + 4 * r;
-            if (ii >= jj && ii < K1) p[ii * (ii + 1) / 2 + jj] = acc00[r];
-            const int i1 = 16 + ii;
-            if (i1 < K1) p[i1 * (i1 + 1) / 2 + jj] = acc10[r];
-            if (ii >= jj && i1 < K1) p[i1 * (i1 + 1) / 2 + 16 + jj] = acc11[r];
-        }
-    } else {
-        const double t0 = rc_wave_sum_f64(s0);
-        const double t1 = rc_wave_sum_f64(s1);
-        if (lane == 0) {
-            p[0] = t0;
-            p[1] = t1;
-        }
+    if (MODE != IM_JAC && lane == 0) {
+        p[0] = t0;
+        p[1] = t1;
     }
     if (lane == 0) bad[it_i] = f;
 }
@@ -778,13 +795,14 @@ __global__ __launch_bounds__(64) void im_ctrl_kernel(
     if (op == IC_AFTER_JAC && !host_done && st.active && ran) {
         const int nst = (k + 1) * (k + 2) / 2;
         for (int t = lane; t < nst; t += 64)
-            G[t] = rc_ordered_sum(part + (size_t)i0 * IM_STATS + t, IM_STATS, ni);
+            G[t] = rc_grouped_sum(part + (size_t)i0 * IM_STATS + t, IM_STATS, ni,
+                                  cands[cand].group);
     }
     __syncthreads();
     if (lane == 0) {
         double *cc = cs + (size_t)cand * (size_t)kmax;
         auto flag_sum = [&](double &sum) {
-            sum = rc_ordered_sum(part + (size_t)i0 * IM_STATS, IM_STATS, ni);
+            sum = rc_grouped_sum(part + (size_t)i0 * IM_STATS, IM_STATS, ni, cands[cand].group);
             return rc_batched_or(bad + i0, ni);
         };
         int next_run = 0;
@@ -812,9 +830,7 @@ __global__ __launch_bounds__(64) void im_ctrl_kernel(
             case IC_AFTER_JAC: {
                 st.want = 0;
                 if (host_done || !st.active || !ran) break;
-                int f = 0;
-                for (int u = 0; u < ni; ++u) f |= bad[i0 + u];
-                if (f != 0) {
+                if (rc_batched_or(bad + i0, ni) != 0) {
                     st.active = 0;
                     break;
                 }
@@ -920,21 +936,21 @@ struct ImBatch {
     /* One pass over ni items of mode MODE on stream s: the register-stack
        kernel for the fast candidates, the node-array kernel for the rest. */
     template <int MODE>
-    void launch(hipStream_t s, int ni, int metric, const int *run)
+    void launch(hipStream_t s, int ni, int metric, const int *run, int stride)
     {
         if (ni <= 0) return;
         RcRows &R = c->sets[0];
         if (any_fast) {
             switch (R.v) {
-                case 1: im_fast_kernel<MODE, 1><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, IM_STATS, d_bad, run); break;
-                case 2: im_fast_kernel<MODE, 2><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, IM_STATS, d_bad, run); break;
-                case 3: im_fast_kernel<MODE, 3><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, IM_STATS, d_bad, run); break;
-                default: im_fast_kernel<MODE, 4><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, IM_STATS, d_bad, run); break;
+                case 1: im_fast_kernel<MODE, 1><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, stride, d_bad, run); break;
+                case 2: im_fast_kernel<MODE, 2><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, stride, d_bad, run); break;
+                case 3: im_fast_kernel<MODE, 3><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, stride, d_bad, run); break;
+                default: im_fast_kernel<MODE, 4><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, stride, d_bad, run); break;
             }
         }
         if (any_general)
             im_pass_kernel<MODE><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64,
-                                                   R.w64, R.n, R.v, metric, d_part, IM_STATS, d_bad,
+                                                   R.w64, R.n, R.v, metric, d_part, stride, d_bad,
                                                    run);
     }
 
@@ -957,7 +973,7 @@ struct ImBatch {
         nprog = np;
         kmax = km;
         RcRows &R = c->sets[0];
-        cands.assign((size_t)np, ImCand{0, 0, 0, 0});
+        cands.assign((size_t)np, ImCand{0, 0, 0, 0, 0, 0});
         pre.assign((size_t)np, -1);
         for (int i = 0; i < np; ++i) {
             const int words = (int)(off[i + 1] - off[i]);
@@ -1005,10 +1021,13 @@ struct ImBatch {
             rec.insert(rec.end(), w, w + words);
         }
         if (rec.empty()) rec.push_back(0);
+        const RcSplit sp = rc_split(R.n, np * rc_groups_of(R.n) >= RC_ITEMS_WANTED, 0);
         for (int i = 0; i < np; ++i) {
+            cands[i].sub = sp.sub;
+            cands[i].group = sp.group;
             if (pre[i] >= 0) continue;
-            for (int r0 = 0; r0 < R.n; r0 += IM_TILE)
-                h_items.push_back(ImItem{i, r0, std::min(IM_TILE, R.n - r0), 0});
+            for (int r0 = 0; r0 < R.n; r0 += sp.rows)
+                h_items.push_back(ImItem{i, r0, std::min(sp.rows, R.n - r0), 0});
         }
         const size_t ni = std::max<size_t>(1, h_items.size());
         if (hipMalloc((void **)&d_rec, rec.size() * 4) != hipSuccess ||
@@ -1026,55 +1045,46 @@ struct ImBatch {
             (!h_items.empty() && hipMemcpyAsync(d_items, h_items.data(), sizeof(ImItem) * h_items.size(),
                                                 hipMemcpyHostToDevice, s) != hipSuccess))
             return -1;
-        h_part.resize(ni * IM_STATS);
-        h_bad.resize(ni);
         return 0;
     }
 
-    /* Runs one pass over the items of the candidates with run[i] != 0 at
-       constants cs (np x kmax); fills per-candidate sums: out[i][0..] and the
-       OR of the item flags. */
-    int pass(int mode, int metric, const std::vector<double> &cs, const std::vector<char> &run,
-             std::vector<std::vector<double>> &sums, std::vector<int> &flags)
+    /* Scores every item's candidate at constants cs (np x kmax): per candidate
+       the two sums (2 i, 2 i + 1) and the OR of the item flags. */
+    int score(int metric, const double *cs, std::vector<double> &sums, std::vector<int> &flags)
     {
-        std::vector<ImItem> sel;
-        std::vector<int> from;
-        for (size_t q = 0; q < h_items.size(); ++q)
-            if (run[(size_t)h_items[q].cand]) {
-                sel.push_back(h_items[q]);
-                from.push_back((int)q);
-            }
-        sums.assign((size_t)nprog, std::vector<double>());
+        sums.assign(2 * (size_t)nprog, 0.0);
         flags.assign((size_t)nprog, 0);
-        if (sel.empty()) return 0;
+        const int ni = (int)h_items.size();
+        if (ni == 0) return 0;
         hipStream_t s = c->s_fit;
-        if (hipMemcpyAsync(d_items, sel.data(), sizeof(ImItem) * sel.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
-            hipMemcpyAsync(d_cs, cs.data(), sizeof(double) * cs.size(), hipMemcpyHostToDevice, s) != hipSuccess)
+        if (hipMemcpyAsync(d_cs, cs, sizeof(double) * (size_t)nprog * (size_t)kmax,
+                           hipMemcpyHostToDevice, s) != hipSuccess)
             return -1;
-        const int ni = (int)sel.size();
         (void)hipEventRecord(c->t0, s);
-        if (mode == IM_SCORE) launch<IM_SCORE>(s, ni, metric, nullptr);
-        else if (mode == IM_RSS) launch<IM_RSS>(s, ni, metric, nullptr);
-        else launch<IM_JAC>(s, ni, metric, nullptr);
+        launch<IM_SCORE>(s, ni, metric, nullptr, 2);
         (void)hipEventRecord(c->t1, s);
         if (hipGetLastError() != hipSuccess) return -1;
-        if (hipMemcpyAsync(h_part.data(), d_part, sizeof(double) * (size_t)ni * IM_STATS,
+        h_part.resize(2 * (size_t)ni);
+        h_bad.resize((size_t)ni);
+        if (hipMemcpyAsync(h_part.data(), d_part, sizeof(double) * h_part.size(),
                            hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipMemcpyAsync(h_bad.data(), d_bad, sizeof(int) * (size_t)ni, hipMemcpyDeviceToHost, s) != hipSuccess ||
             hipStreamSynchronize(s) != hipSuccess)
             return -1;
-        float e = 0.0f;
-        (void)hipEventElapsedTime(&e, c->t0, c->t1);
-        ms += e;
-        /* Items of one candidate are consecutive and in row order. */
-        for (int q = 0; q < ni; ++q) {
-            const int cand = sel[(size_t)q].cand;
-            const int K1 = cands[(size_t)cand].k + 1;
-            const int nst = (mode == IM_JAC) ? K1 * (K1 + 1) / 2 : 2;
-            std::vector<double> &t = sums[(size_t)cand];
-            if (t.empty()) t.assign((size_t)nst, 0.0);
-            for (int j = 0; j < nst; ++j) t[(size_t)j] += h_part[(size_t)q * IM_STATS + j];
-            flags[(size_t)cand] |= h_bad[(size_t)q];
+        (void)hipEventElapsedTime(&ms, c->t0, c->t1);
+        /* Items of one candidate are consecutive and in row order; a group's
+           items are summed by themselves first (RcSplit). */
+        for (int q = 0; q < ni;) {
+            const int cand = h_items[(size_t)q].cand;
+            double part[2] = {0.0, 0.0};
+            for (int u = 0; u < cands[(size_t)cand].group && q < ni &&
+                            h_items[(size_t)q].cand == cand; ++u, ++q) {
+                part[0] += h_part[2 * (size_t)q];
+                part[1] += h_part[2 * (size_t)q + 1];
+                flags[(size_t)cand] |= h_bad[(size_t)q];
+            }
+            sums[2 * (size_t)cand] += part[0];
+            sums[2 * (size_t)cand + 1] += part[1];
         }
         return 0;
     }
@@ -1099,20 +1109,17 @@ float rc_implicit_score_batch(void *ctx, const unsigned int *prog, const unsigne
     if (rc_rows_ensure_f64(cx, &cx->sets[0]) != 0) return -1.0f;
     ImBatch B;
     if (B.setup(cx, prog, off, pcount, nprog, kmax) != 0) return -1.0f;
-    std::vector<double> cs(c, c + (size_t)nprog * (size_t)kmax);
-    std::vector<char> run((size_t)nprog, 1);
-    for (int i = 0; i < nprog; ++i) run[i] = B.pre[i] < 0;
-    std::vector<std::vector<double>> sums;
+    std::vector<double> sums;
     std::vector<int> flags;
-    if (B.pass(IM_SCORE, metric, cs, run, sums, flags) != 0) return -1.0f;
+    if (B.score(metric, c, sums, flags) != 0) return -1.0f;
     for (int i = 0; i < nprog; ++i) {
         if (B.pre[i] >= 0) {
             out[i] = RC_F64_NAN;
             status[i] = 1;
             continue;
         }
-        const std::vector<double> &t = sums[(size_t)i];
-        const bool fin = !t.empty() && flags[i] == 0 && isfinite(t[1]) && t[1] > 0.0;
+        const double *t = &sums[2 * (size_t)i];
+        const bool fin = flags[i] == 0 && isfinite(t[1]) && t[1] > 0.0;
         out[i] = fin ? t[0] / t[1] : IM_INF;
         status[i] = fin ? 0 : 2;
     }
@@ -1177,8 +1184,8 @@ float rc_implicit_fit_batch(void *ctx, const unsigned int *prog, const unsigned 
                                             d_sse, d_st);
     };
     auto pass = [&](int mode) {
-        if (mode == IM_RSS) B.launch<IM_RSS>(s, ni, 0, d_run);
-        else B.launch<IM_JAC>(s, ni, 0, d_run);
+        if (mode == IM_RSS) B.launch<IM_RSS>(s, ni, 0, d_run, IM_STATS);
+        else B.launch<IM_JAC>(s, ni, 0, d_run, IM_STATS);
     };
     if (ok) {
         (void)hipEventRecord(cx->t0, s);

@@ -173,6 +173,44 @@ struct RcCtx {
 };
 
 /* Host helpers (rc_ctx.hip). */
+/* How a candidate's rows are split into work items, in the fit, correlation
+   and implicit arms.  Every sum over rows is a sum of groups of RC_GROUP_ROWS
+   rows, a group the sum of its sub-tiles, each added up in row order; an item
+   is a sub-tile or a whole group.  So the result depends on n (which sets the
+   sub-tile) and not on the item size, and that may follow the batch: groups
+   where they make RC_ITEMS_WANTED items (four for each of the 2048 one-wave
+   slots that two waves per SIMD are), for an item's fixed part (clearing its
+   block, its partial triangle, the control kernel's reading of that) is small
+   beside 8192 rows; sub-tiles where they would leave slots empty.  A small
+   table has small sub-tiles, or one island's 200 candidates of 1000 rows would
+   be 200 waves; 512 rows are one step of the f32 loss kernel.  Measured against
+   groups throughout: 64 absolute-error fits x 100 003 rows 37.1 -> 11.2 ms, 128
+   correlation fits x 50 021 rows 20.3 -> 11.4, 128 implicit fits x 65 537 rows
+   242 -> 97, 200 fits x 1000 rows 1.38 -> 1.21; 1024 fits x 262 144 rows, which
+   keep groups, 198 -> 197. */
+constexpr int RC_GROUP_ROWS = 8192;
+constexpr long long RC_ITEMS_WANTED = 8192;
+struct RcSplit {
+    int rows;  /* of an item */
+    int sub;   /* of a sub-tile */
+    int group; /* items of a group */
+};
+inline int rc_sub_rows(int n)
+{
+    return n <= 8192 ? 512 : n <= 32768 ? 1024 : 2048;
+}
+/* The split of n rows; groups: the batch has enough of them.  A caller's own
+   item size (tuned > 0, a multiple of 256) has sub-tiles where it is a
+   multiple of them, and is a part of a group where it divides one. */
+inline RcSplit rc_split(int n, bool groups, int tuned)
+{
+    const int sub = rc_sub_rows(n);
+    const int rows = tuned > 0 ? tuned : groups ? RC_GROUP_ROWS : sub;
+    return {rows, rows % sub == 0 ? sub : rows,
+            rows < RC_GROUP_ROWS && RC_GROUP_ROWS % rows == 0 ? RC_GROUP_ROWS / rows : 1};
+}
+inline long long rc_groups_of(int n) { return ((long long)n + RC_GROUP_ROWS - 1) / RC_GROUP_ROWS; }
+
 double rc_now_ms();
 int rc_dev_alloc(RcCtx *c, void **p, size_t bytes);
 void rc_dev_free(RcCtx *c, void *p);
