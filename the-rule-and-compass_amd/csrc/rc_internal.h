@@ -44,10 +44,7 @@ struct RcVaryState; /* rc_vary.hip */
 /* Buffers of the order / rank / maximum stages (rc_order.hip); device
    pointers grow with rc_grow, the host vectors stage asynchronous uploads. */
 struct RcOrderBufs {
-    uint32_t *prog = nullptr;   size_t prog_cap = 0;
-    uint32_t *off = nullptr;    size_t off_cap = 0;
-    int *pcount = nullptr;      size_t pcount_cap = 0;
-    double *c0 = nullptr;       size_t c0_cap = 0;
+    unsigned char *in = nullptr; size_t in_cap = 0;  /* a call's inputs */
     int *seg = nullptr;         size_t seg_cap = 0;
     unsigned long long *keys = nullptr;     size_t keys_cap = 0;
     unsigned long long *keys_out = nullptr; size_t keys_out_cap = 0;
@@ -55,7 +52,6 @@ struct RcOrderBufs {
     uint32_t *rows_out = nullptr; size_t rows_out_cap = 0;
     int *start_of = nullptr;    size_t start_cap = 0;
     void *temp = nullptr;       size_t temp_cap = 0;
-    int *status = nullptr;      size_t status_cap = 0;
     double *val = nullptr;      size_t val_cap = 0;
     unsigned long long *out = nullptr; size_t out_cap = 0;
     long long *B = nullptr;     size_t B_cap = 0;    /* target's doubled centred ranks */
@@ -64,11 +60,9 @@ struct RcOrderBufs {
     unsigned long long h_bb[2] = {0, 0};             /* Sigma B^2 (hi, lo) */
     int rank_ready = 0;
     RcMaxOut *mx = nullptr;     size_t mx_cap = 0;
-    int *coords = nullptr;      size_t coords_cap = 0;
-    double *levels = nullptr;   size_t levels_cap = 0;
+    void *part = nullptr;       size_t part_cap = 0; /* tiles of a maximum scan */
     std::vector<int> h_seg;
-    std::vector<int> h_coords;
-    std::vector<double> h_levels;
+    std::vector<unsigned char> h_in, h_out; /* a call's inputs and outputs */
 };
 
 struct RcCtx {

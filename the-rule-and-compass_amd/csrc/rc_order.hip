@@ -13,28 +13,40 @@
  * right over the sorted window, the CPU's order, so it agrees bit for bit.
  *
  * MI355X layout:
- *  - one thread per (segment, row) evaluates the records into a private value
- *    array and writes one 64-bit sort key (and the row, for ranks);
- *  - rocPRIM's segmented radix sort (through hipCUB) orders each segment;
- *  - order statistics read the sorted keys directly (one wave per segment);
+ *  - the row kernels of rc_order_kern.hip evaluate the records and write one
+ *    64-bit sort key (and the row, for ranks), or a tile's maximum; programs
+ *    that do not fit their registers run here, one thread per (segment, row)
+ *    with a private value array;
+ *  - the median is a selection: one workgroup per segment narrows the range of
+ *    keys that holds the middle ones by histograms of its leading bits;
+ *  - rocPRIM's segmented radix sort (through hipCUB) orders each segment for
+ *    the interquartile mean, summed by one wave per segment, and for ranks;
  *  - average ranks come from two scans per segment in one workgroup: a
  *    forward max-scan finds each position's tie-run start, a backward
  *    min-scan its run end, and A = start + end - n is the doubled centred
  *    rank; its products with the target's cached ranks accumulate in exact
  *    128-bit integers (two 64-bit halves), so the reduction order is free;
- *  - the maximum scan is one workgroup per segment reducing an integer key
- *    (|r| bit patterns order like the values), the lowest maximising row and
- *    the feasibility interval of a level along one constant.
+ *  - the maximum scan reduces an integer key (|r| bit patterns order like the
+ *    values), the lowest maximising row and the feasibility interval of a level
+ *    along one constant, over tiles and then over a segment's tiles.
  */
 #include "rc_fit_dev.h"
+#include "rc_fitvm.h"
 #include "rc_internal.h"
+#include "rc_order_kern.h"
 
 #include <hipcub/hipcub.hpp>
 
 #include <string.h>
 
+#include <math.h>
+
 #include <algorithm>
 #include <vector>
+
+extern "C" int rch_fitvm_compile(const unsigned int *rec, int words, int p, int nvars, int col_bytes,
+                                 unsigned int flags, unsigned int *fwd, int cap_f,
+                                 unsigned int *rev, int cap_r, int *info);
 
 namespace {
 
@@ -71,7 +83,7 @@ __device__ __forceinline__ double seg_predict(const uint32_t *__restrict__ prog,
     return v[m - 1];
 }
 
-/* Sort keys of every (segment, row): |pred - y| bit patterns (order
+/* Sort keys of every (listed segment, row): |pred - y| bit patterns (order
    statistics, eval.cu:4383-4419) or rank keys of pred with the row as the
    payload (ranks, eval.cu:2952-2982).  A non-finite value keys last and
    flags its segment (status 2). */
@@ -79,14 +91,16 @@ template <bool RANK>
 __global__ __launch_bounds__(256) void os_keys_kernel(
     const uint32_t *__restrict__ prog, const uint32_t *__restrict__ off,
     const double *__restrict__ c0, int kmax, const double *__restrict__ cols64,
-    const double *__restrict__ y64, int n, int nsegs, int ntrials,
+    const double *__restrict__ y64, int n, const int *__restrict__ segs, int nlist, int ntrials,
     unsigned long long *__restrict__ keys, uint32_t *__restrict__ rows, int *__restrict__ status)
 {
-    const long long total = (long long)n * (long long)nsegs;
+    const long long total = (long long)n * (long long)nlist;
     const long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        const int seg = (int)(i / n);
-        const int row = (int)(i - (long long)seg * n);
+    for (long long u = (long long)blockIdx.x * blockDim.x + threadIdx.x; u < total; u += stride) {
+        const int li = (int)(u / n);
+        const int row = (int)(u - (long long)li * n);
+        const int seg = segs[li];
+        const long long i = (long long)seg * n + row;
         double v[FT_MAX_NODES];
         const double pred = seg_predict(prog, off, c0, kmax, cols64, n, seg, ntrials, row, v);
         if (RANK) {
@@ -126,33 +140,200 @@ __global__ void rk_target_keys_kernel(const double *__restrict__ y64, int n,
     rows[i] = (uint32_t)i;
 }
 
-/* Median (what 0) or interquartile mean (what 1) of one sorted segment
-   (metrics.rs:1193-1223): one wave per segment; the window sum runs left to
-   right on one lane, the CPU's order. */
-__global__ __launch_bounds__(64) void os_pick_kernel(const unsigned long long *__restrict__ keys,
-                                                     int n, int nsegs, int what,
-                                                     double *__restrict__ out,
-                                                     const int *__restrict__ status)
+/* The median of one segment's unsorted keys (metrics.rs:1193-1208), by
+   selection.  The keys that can be the lower middle one lie in [base, base +
+   range]; a histogram of their leading 11 bits says in which bin, which is the
+   next range, until a bin has no more than SEL_CAP keys: those are gathered and
+   sorted in LDS.  The upper middle key is the next of them, or the least key
+   above the last range.  Two to three passes over the keys in all, each at the
+   rate one CU reads, where the full sort made eight and wrote as much: 256
+   segments of 262 144 keys take 0.30 ms, their sort 9.1. */
+constexpr int SEL_THREADS = 1024;
+constexpr int SEL_BINS = 2048;
+constexpr int SEL_CAP = 4096;
+__global__ __launch_bounds__(SEL_THREADS) void os_select_kernel(
+    const unsigned long long *__restrict__ keys, int n, int nsegs, double *__restrict__ out,
+    const int *__restrict__ status)
 {
+    __shared__ unsigned int hist[SEL_BINS];
+    __shared__ unsigned int wsum[SEL_THREADS / 64];
+    __shared__ unsigned long long buf[SEL_CAP];
+    __shared__ unsigned long long wa[SEL_THREADS / 64], wb[SEL_THREADS / 64];
+    __shared__ unsigned int sh_n;
+    __shared__ int sh_bin;
+    __shared__ unsigned int sh_before;
     const int seg = blockIdx.x;
-    if (seg >= nsegs || threadIdx.x != 0) return;
-    if (status[seg] != 0) {
-        out[seg] = __builtin_nan("");
+    if (seg >= nsegs) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (status[seg] != 0) { /* block-uniform */
+        if (tid == 0) out[seg] = __builtin_nan("");
         return;
     }
     const unsigned long long *k = keys + (size_t)seg * (size_t)n;
-    if (what == 0) {
-        out[seg] = (n & 1) ? os_value(k[n / 2]) : 0.5 * (os_value(k[n / 2 - 1]) + os_value(k[n / 2]));
+    /* Every key of the segment, four loads in flight a thread. */
+    auto each = [&](auto &&f) {
+        const unsigned int m = (unsigned int)n;
+        for (unsigned int i0 = tid; i0 < m; i0 += 4u * SEL_THREADS) {
+            unsigned long long v[4];
+#pragma unroll
+            for (unsigned int u = 0; u < 4u; ++u) v[u] = k[min(i0 + u * SEL_THREADS, m - 1u)];
+#pragma unroll
+            for (unsigned int u = 0; u < 4u; ++u)
+                if (i0 + u * SEL_THREADS < m) f(v[u]);
+        }
+    };
+    /* The block's least a and greatest b, in every thread. */
+    auto ends = [&](unsigned long long &a, unsigned long long &b) {
+        for (int o = 32; o > 0; o >>= 1) {
+            const unsigned long long x = __shfl_xor(a, o, 64), y = __shfl_xor(b, o, 64);
+            a = x < a ? x : a;
+            b = y > b ? y : b;
+        }
+        if (lane == 0) {
+            wa[wave] = a;
+            wb[wave] = b;
+        }
+        __syncthreads();
+        for (int w = 0; w < SEL_THREADS / 64; ++w) {
+            a = wa[w] < a ? wa[w] : a;
+            b = wb[w] > b ? wb[w] : b;
+        }
+        __syncthreads();
+    };
+    unsigned long long least = KEY_BAD, most = 0ull;
+    each([&](unsigned long long v) {
+        least = v < least ? v : least;
+        most = v > most ? v : most;
+    });
+    ends(least, most);
+    unsigned long long base = least, range = most - least;
+    unsigned int rank = (unsigned int)((n - 1) / 2), count = (unsigned int)n;
+    while (range != 0ull && count > SEL_CAP) {
+        const int bits = 64 - __clzll((long long)range);
+        const int shift = bits > 11 ? bits - 11 : 0;
+        for (int i = tid; i < SEL_BINS; i += SEL_THREADS) hist[i] = 0u;
+        __syncthreads();
+        each([&](unsigned long long v) {
+            const unsigned long long d = v - base; /* below base: wraps past range */
+            if (d <= range) atomicAdd(&hist[(unsigned int)(d >> shift)], 1u);
+        });
+        __syncthreads();
+        /* The bin that holds `rank`: a scan of two bins a thread. */
+        const unsigned int h0 = hist[2 * tid], h1 = hist[2 * tid + 1];
+        unsigned int run = h0 + h1;
+        for (int o = 1; o < 64; o <<= 1) {
+            const unsigned int x = __shfl_up(run, o, 64);
+            if (lane >= o) run += x;
+        }
+        if (lane == 63) wsum[wave] = run;
+        __syncthreads();
+        for (int w = 0; w < wave; ++w) run += wsum[w];
+        const unsigned int before = run - h0 - h1;
+        if (rank >= before && rank < before + h0) {
+            sh_bin = 2 * tid;
+            sh_before = before;
+        } else if (rank >= before + h0 && rank < run) {
+            sh_bin = 2 * tid + 1;
+            sh_before = before + h0;
+        }
+        __syncthreads();
+        const unsigned long long start = (unsigned long long)sh_bin << shift;
+        count = hist[sh_bin];
+        rank -= sh_before;
+        base += start;
+        const unsigned long long width = (1ull << shift) - 1ull, rest = range - start;
+        range = width < rest ? width : rest;
+        __syncthreads();
+    }
+    /* The keys of the last range into LDS (one value of them where it is a
+       single key), and the least key above it. */
+    if (tid == 0) sh_n = 0u;
+    __syncthreads();
+    unsigned long long above = KEY_BAD, unused = 0ull;
+    const unsigned long long last = base + range;
+    each([&](unsigned long long v) {
+        if (v > last) above = v < above ? v : above;
+        else if (range != 0ull && v >= base) buf[atomicAdd(&sh_n, 1u)] = v;
+    });
+    ends(above, unused);
+    unsigned long long low = base, high = base;
+    if (range != 0ull) {
+        const unsigned int m = sh_n; /* = count <= SEL_CAP */
+        unsigned int p2 = 2u;
+        while (p2 < m) p2 <<= 1;
+        for (unsigned int i = m + tid; i < p2; i += SEL_THREADS) buf[i] = KEY_BAD;
+        __syncthreads();
+        for (unsigned int size = 2u; size <= p2; size <<= 1)
+            for (unsigned int step = size >> 1; step > 0u; step >>= 1) {
+                for (unsigned int t = tid; t < p2 / 2u; t += SEL_THREADS) {
+                    const unsigned int i = 2u * t - (t & (step - 1u)), j = i + step;
+                    const bool up = (i & size) == 0u;
+                    const unsigned long long x = buf[i], y = buf[j];
+                    if ((x > y) == up) {
+                        buf[i] = y;
+                        buf[j] = x;
+                    }
+                }
+                __syncthreads();
+            }
+        low = buf[rank];
+        high = rank + 1u < m ? buf[rank + 1u] : above;
+    } else if (rank + 1u >= count) {
+        high = above;
+    }
+    if (tid == 0) out[seg] = (n & 1) ? os_value(low) : 0.5 * (os_value(low) + os_value(high));
+}
+
+/* The interquartile mean of one sorted segment (metrics.rs:1209-1223): one
+   wave per segment; the window is summed left to right, the CPU's order, from
+   blocks that the wave has staged in LDS while the previous one is summed (a
+   chain of dependent f64 adds; one lane that loaded each value itself waited
+   on memory for every one: 256 segments of 262 144 keys 8.5 ms, now 0.74). */
+constexpr int MEAN_BLOCK = 1024;
+__global__ __launch_bounds__(64) void os_mean_kernel(const unsigned long long *__restrict__ keys,
+                                                     int n, int nsegs, double *__restrict__ out,
+                                                     const int *__restrict__ status)
+{
+    __shared__ __align__(16) double stage[MEAN_BLOCK];
+    const int seg = blockIdx.x;
+    if (seg >= nsegs) return;
+    const int lane = threadIdx.x;
+    if (status[seg] != 0) { /* wave-uniform */
+        if (lane == 0) out[seg] = __builtin_nan("");
         return;
     }
+    const unsigned long long *k = keys + (size_t)seg * (size_t)n;
     int lo = 0, hi = n;
     if (n >= 4) {
         lo = n / 4;
         hi = max((3 * n) / 4, lo + 1);
     }
+    constexpr int PER = MEAN_BLOCK / 64;
+    unsigned long long v[PER];
+    auto load = [&](int at) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u) v[u] = k[min(at + 64 * u + lane, n - 1)];
+    };
     double s = 0.0;
-    for (int i = lo; i < hi; ++i) s += os_value(k[i]);
-    out[seg] = s / (double)(hi - lo);
+    load(lo);
+    for (int at = lo; at < hi; at += MEAN_BLOCK) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < PER; ++u) stage[64 * u + lane] = os_value(v[u]);
+        __syncthreads();
+        if (at + MEAN_BLOCK < hi) load(at + MEAN_BLOCK);
+        const int m = min(MEAN_BLOCK, hi - at);
+        int i = 0;
+        for (; i + 16 <= m; i += 16) {
+            double w[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) w[u] = stage[i + u];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) s += w[u];
+        }
+        for (; i < m; ++i) s += stage[i];
+    }
+    if (lane == 0) out[seg] = s / (double)(hi - lo);
 }
 
 /* ---- exact 128-bit accumulation ------------------------------------------- */
@@ -291,7 +472,9 @@ __global__ __launch_bounds__(RK_THREADS) void rk_runs_kernel(
 
 /* ---- the exact maximum-error scan ----------------------------------------- */
 
-/* One workgroup per segment (eval.cu:4505-4600): max |r| as an integer
+/* One workgroup per segment marked in redo, those that the row kernels do not
+   run and those in which they met a row that is not finite
+   (eval.cu:4505-4600): max |r| as an integer
    max of bit patterns with the lowest row on ties; with a constant `coord`
    and a finite level t >= 0, the intersection of the per-row intervals
    {delta : |r_i + b_i delta| <= t}, b_i = d pred_i / d c_coord from the f64
@@ -301,7 +484,7 @@ __global__ __launch_bounds__(MX_THREADS) void mx_scan_kernel(
     const int *__restrict__ pcount, const double *__restrict__ c0, int kmax,
     const int *__restrict__ coords, const double *__restrict__ levels,
     const double *__restrict__ cols64, const double *__restrict__ y64, int n, int nsegs,
-    int ntrials, RcMaxOut *__restrict__ out)
+    int ntrials, const int *__restrict__ redo, RcMaxOut *__restrict__ out)
 {
     __shared__ unsigned long long skey[MX_THREADS];
     __shared__ int srow[MX_THREADS];
@@ -309,7 +492,7 @@ __global__ __launch_bounds__(MX_THREADS) void mx_scan_kernel(
     __shared__ double shi[MX_THREADS];
     __shared__ int sbad[MX_THREADS];
     const int seg = blockIdx.x;
-    if (seg >= nsegs) return;
+    if (seg >= nsegs || !redo[seg]) return;
     const int tid = threadIdx.x;
     const int set = seg / ntrials;
     const uint32_t *nd = prog + off[set];
@@ -388,37 +571,168 @@ __global__ __launch_bounds__(MX_THREADS) void mx_scan_kernel(
     }
 }
 
-/* ---- host side ------------------------------------------------------------- */
-
-/* Device copies of a call's programs and constants. */
-struct StageInput {
-    uint32_t *prog = nullptr;
-    uint32_t *off = nullptr;
-    int *pcount = nullptr;
-    double *c0 = nullptr;
-};
-
-int upload(RcCtx *c, void **dst, size_t *cap, const void *src, size_t bytes)
+/* A listed segment's tiles in one: the greatest |r| with its lowest row, the
+   intersection of the intervals. */
+__global__ __launch_bounds__(64) void mx_finish_kernel(const int *__restrict__ segs, int nlist,
+                                                       const OrMax *__restrict__ part, int tiles,
+                                                       RcMaxOut *__restrict__ out)
 {
-    if (rc_grow(c, dst, cap, bytes > 0 ? bytes : 1, 1) != 0) return -1;
-    if (bytes && hipMemcpyAsync(*dst, src, bytes, hipMemcpyHostToDevice, c->s_fit) != hipSuccess)
-        return -1;
-    return 0;
+    const int li = blockIdx.x;
+    if (li >= nlist) return;
+    unsigned long long key = 0ull;
+    int row = 0x7fffffff, veto = 0;
+    double lo = -__builtin_inf(), hi = __builtin_inf();
+    for (int t = threadIdx.x; t < tiles; t += 64) {
+        const OrMax m = part[(size_t)li * (size_t)tiles + (size_t)t];
+        if (m.key > key || (m.key == key && m.row < row)) {
+            key = m.key;
+            row = m.row;
+        }
+        lo = fmax(lo, m.lo);
+        hi = fmin(hi, m.hi);
+        veto |= m.veto;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long k = __shfl_xor(key, o, 64);
+        const int r = __shfl_xor(row, o, 64);
+        if (k > key || (k == key && r < row)) {
+            key = k;
+            row = r;
+        }
+        lo = fmax(lo, __shfl_xor(lo, o, 64));
+        hi = fmin(hi, __shfl_xor(hi, o, 64));
+    }
+    if (__any(veto)) {
+        lo = __builtin_inf();
+        hi = -__builtin_inf();
+    }
+    if (threadIdx.x == 0) {
+        RcMaxOut o;
+        o.status = 0;
+        o.vmax = os_value(key);
+        o.row = row;
+        o.lo = lo;
+        o.hi = hi;
+        out[segs[li]] = o;
+    }
 }
 
+/* ---- host side ------------------------------------------------------------- */
+
+/* A call's inputs on the device, gathered in one host block and sent in one
+   copy: programs, constants, value streams, segment lists and what the kernels
+   find cleared. */
+struct StageInput {
+    std::vector<OrSet> sets;
+    std::vector<uint32_t> code;
+    std::vector<int> fast, general; /* segments by the route of their set */
+    uint32_t *prog = nullptr, *off = nullptr, *d_code = nullptr;
+    int *pcount = nullptr, *coords = nullptr, *lists = nullptr, *flags = nullptr;
+    double *c0 = nullptr, *levels = nullptr;
+    OrSet *d_sets = nullptr;
+};
+
+/* What the record sweep takes: a canonical post-order tree (each record's
+   children are the tops of the evaluation stack) no deeper than its stack. */
+bool stack_tree(const unsigned int *nd, int m)
+{
+    std::vector<uint32_t> st;
+    size_t depth = 0;
+    for (int i = 0; i < m; ++i) {
+        const uint32_t op = nd[4 * i], k0 = nd[4 * i + 1], k1 = nd[4 * i + 2];
+        if (op != OP_CONST && op != OP_VAR) {
+            const bool two = op == OP_ADD || op == OP_SUB || op == OP_MUL || op == OP_DIV || op == OP_POW;
+            if (two) {
+                if (st.size() < 2 || st.back() != k1) return false;
+                st.pop_back();
+            }
+            if (st.empty() || st.back() != k0) return false;
+            st.pop_back();
+        }
+        st.push_back((uint32_t)i);
+        depth = std::max(depth, st.size());
+    }
+    return st.size() == 1 && depth <= OR_SDEPTH + 1;
+}
+
+/* The sets' records and value streams (none where the program does not fit
+   the stream's files). */
+void stage_sets(const RcCtx *c, const unsigned int *prog, const unsigned int *off,
+                const int *pcount, int nsets, StageInput *in)
+{
+    uint32_t buf[OR_STREAM_WORDS];
+    in->sets.resize((size_t)nsets);
+    for (int s = 0; s < nsets; ++s) {
+        OrSet &d = in->sets[(size_t)s];
+        const int words = (int)(off[s + 1] - off[s]);
+        int info[6];
+        d.r_off = off[s];
+        d.m = words / 4;
+        d.t_off = (uint32_t)in->code.size();
+        d.t_m = 0;
+        if (c->sets[0].n <= OR_MAX_ROWS &&
+            rch_fitvm_compile(prog + off[s], words, pcount[s], c->sets[0].v, 8,
+                              VMC_INPUTS_IN_U | VMC_VALUE_ONLY | VMC_SMALL_U, buf,
+                              OR_STREAM_WORDS, nullptr, 0, info) == 0) {
+            d.t_m = info[0];
+            in->code.insert(in->code.end(), buf, buf + 2 * info[0]);
+        }
+    }
+}
+
+size_t stage_take(size_t &cur, size_t bytes)
+{
+    const size_t o = (cur + 255) & ~(size_t)255;
+    cur = o + bytes;
+    return o;
+}
+
+/* coords / levels: nsegs each, or null; flags: nsegs ints at the device. */
 int stage_inputs(RcCtx *c, const unsigned int *prog, const unsigned int *off, const int *pcount,
-                 int nsets, int nsegs, int kmax, const double *c0, StageInput *in)
+                 int nsets, int nsegs, int kmax, const double *c0, const int *coords,
+                 const double *levels, const std::vector<int> &flags, StageInput *in)
 {
     RcOrderBufs &b = c->order;
-    if (upload(c, (void **)&b.prog, &b.prog_cap, prog, sizeof(uint32_t) * (size_t)off[nsets]) != 0 ||
-        upload(c, (void **)&b.off, &b.off_cap, off, sizeof(uint32_t) * (size_t)(nsets + 1)) != 0 ||
-        upload(c, (void **)&b.pcount, &b.pcount_cap, pcount, sizeof(int) * (size_t)nsets) != 0 ||
-        upload(c, (void **)&b.c0, &b.c0_cap, c0, sizeof(double) * (size_t)nsegs * (size_t)kmax) != 0)
+    std::vector<int> lists(in->fast);
+    lists.insert(lists.end(), in->general.begin(), in->general.end());
+    const size_t ns = (size_t)nsegs;
+    size_t cur = 0;
+    const size_t o_prog = stage_take(cur, 4 * (size_t)off[nsets]);
+    const size_t o_off = stage_take(cur, 4 * ((size_t)nsets + 1));
+    const size_t o_pc = stage_take(cur, 4 * (size_t)nsets);
+    const size_t o_c0 = stage_take(cur, 8 * ns * (size_t)kmax);
+    const size_t o_code = stage_take(cur, 4 * in->code.size());
+    const size_t o_sets = stage_take(cur, sizeof(OrSet) * in->sets.size());
+    const size_t o_list = stage_take(cur, 4 * lists.size());
+    const size_t o_flag = stage_take(cur, 4 * flags.size());
+    const size_t o_co = stage_take(cur, coords ? 4 * ns : 0);
+    const size_t o_lv = stage_take(cur, levels ? 8 * ns : 0);
+    cur = stage_take(cur, 1);
+    std::vector<unsigned char> &h = b.h_in;
+    h.resize(cur);
+    memcpy(&h[o_prog], prog, 4 * (size_t)off[nsets]);
+    memcpy(&h[o_off], off, 4 * ((size_t)nsets + 1));
+    memcpy(&h[o_pc], pcount, 4 * (size_t)nsets);
+    memcpy(&h[o_c0], c0, 8 * ns * (size_t)kmax);
+    if (!in->code.empty()) memcpy(&h[o_code], in->code.data(), 4 * in->code.size());
+    memcpy(&h[o_sets], in->sets.data(), sizeof(OrSet) * in->sets.size());
+    memcpy(&h[o_list], lists.data(), 4 * lists.size());
+    memcpy(&h[o_flag], flags.data(), 4 * flags.size());
+    if (coords) memcpy(&h[o_co], coords, 4 * ns);
+    if (levels) memcpy(&h[o_lv], levels, 8 * ns);
+    if (rc_grow(c, (void **)&b.in, &b.in_cap, cur, 1) != 0 ||
+        hipMemcpyAsync(b.in, h.data(), cur, hipMemcpyHostToDevice, c->s_fit) != hipSuccess)
         return -1;
-    in->prog = b.prog;
-    in->off = b.off;
-    in->pcount = b.pcount;
-    in->c0 = b.c0;
+    in->prog = (uint32_t *)(b.in + o_prog);
+    in->off = (uint32_t *)(b.in + o_off);
+    in->pcount = (int *)(b.in + o_pc);
+    in->c0 = (double *)(b.in + o_c0);
+    in->d_code = (uint32_t *)(b.in + o_code);
+    in->d_sets = (OrSet *)(b.in + o_sets);
+    in->lists = (int *)(b.in + o_list);
+    in->flags = (int *)(b.in + o_flag);
+    in->coords = coords ? (int *)(b.in + o_co) : nullptr;
+    in->levels = levels ? (double *)(b.in + o_lv) : nullptr;
     return 0;
 }
 
@@ -430,15 +744,22 @@ int segment_offsets(RcCtx *c, int nsegs, int n)
     std::vector<int> &h = c->order.h_seg;
     h.resize((size_t)nsegs + 1);
     for (int s = 0; s <= nsegs; ++s) h[s] = s * n;
-    return upload(c, (void **)&c->order.seg, &c->order.seg_cap, h.data(), sizeof(int) * h.size());
+    RcOrderBufs &b = c->order;
+    if (rc_grow(c, (void **)&b.seg, &b.seg_cap, h.size(), sizeof(int)) != 0) return -1;
+    return hipMemcpyAsync(b.seg, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice,
+                          c->s_fit) == hipSuccess
+               ? 0
+               : -1;
 }
 
-/* Sort buffers for `total` keys (with row payloads when `pairs`). */
-int sort_buffers(RcCtx *c, long long total, bool pairs)
+/* Buffers for `total` keys: to be sorted, or not; with row payloads when
+   `pairs`. */
+int sort_buffers(RcCtx *c, long long total, bool sorted, bool pairs)
 {
     RcOrderBufs &b = c->order;
     const size_t t = (size_t)total;
-    if (rc_grow(c, (void **)&b.keys, &b.keys_cap, t, sizeof(unsigned long long)) != 0 ||
+    if (rc_grow(c, (void **)&b.keys, &b.keys_cap, t, sizeof(unsigned long long)) != 0) return -1;
+    if (sorted &&
         rc_grow(c, (void **)&b.keys_out, &b.keys_out_cap, t, sizeof(unsigned long long)) != 0)
         return -1;
     if (pairs &&
@@ -481,6 +802,29 @@ unsigned grid_for(long long total)
     return (unsigned)(blocks < 1 ? 1 : blocks);
 }
 
+/* The sort keys of every segment: value streams where the set has one, the
+   general kernel for the others. */
+int launch_keys(RcCtx *c, bool rank, const StageInput &in, int kmax, int ntrials, int *status)
+{
+    RcRows *r = &c->sets[0];
+    RcOrderBufs &b = c->order;
+    const int nf = (int)in.fast.size(), ng = (int)in.general.size();
+    or_launch_keys(rank, nf, c->s_fit, in.lists, in.d_sets, in.d_code, in.c0, kmax, ntrials,
+                   {r->cols64, r->y64, r->n, r->v}, b.keys, b.rows, status);
+    if (ng > 0) {
+        const unsigned grid = grid_for((long long)r->n * ng);
+        if (rank)
+            os_keys_kernel<true><<<grid, 256, 0, c->s_fit>>>(
+                in.prog, in.off, in.c0, kmax, r->cols64, r->y64, r->n, in.lists + nf, ng, ntrials,
+                b.keys, b.rows, status);
+        else
+            os_keys_kernel<false><<<grid, 256, 0, c->s_fit>>>(
+                in.prog, in.off, in.c0, kmax, r->cols64, r->y64, r->n, in.lists + nf, ng, ntrials,
+                b.keys, nullptr, status);
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 /* The target's doubled centred ranks B (cached until the f64 rows change)
    and Sigma B^2. */
 int rank_prepare(RcCtx *c)
@@ -490,7 +834,7 @@ int rank_prepare(RcCtx *c)
     RcRows *r = &c->sets[0];
     const int n = r->n;
     if (n <= 1 || rc_rows_ensure_f64(c, r) != 0) return -1;
-    if (sort_buffers(c, n, true) != 0 || segment_offsets(c, 1, n) != 0) return -1;
+    if (sort_buffers(c, n, true, true) != 0 || segment_offsets(c, 1, n) != 0) return -1;
     if (rc_grow(c, (void **)&b.B, &b.B_cap, (size_t)n, sizeof(long long)) != 0 ||
         rc_grow(c, (void **)&b.flag, &b.flag_cap, 1, sizeof(int)) != 0 ||
         rc_grow(c, (void **)&b.bb, &b.bb_cap, 2, sizeof(unsigned long long)) != 0)
@@ -561,9 +905,8 @@ int rc_order_invalidate(RcCtx *c)
 void rc_order_free(RcCtx *c)
 {
     RcOrderBufs &b = c->order;
-    void *ptrs[] = {b.prog, b.off, b.pcount, b.c0, b.seg, b.keys, b.keys_out, b.rows, b.rows_out,
-                    b.start_of, b.temp, b.status, b.val, b.out, b.B, b.flag, b.bb, b.mx, b.coords,
-                    b.levels};
+    void *ptrs[] = {b.in, b.seg, b.keys, b.keys_out, b.rows, b.rows_out,
+                    b.start_of, b.temp, b.val, b.out, b.B, b.flag, b.bb, b.mx, b.part};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     b = RcOrderBufs();
@@ -587,29 +930,37 @@ float rc_order_stat_score_batch(void *ctx, const unsigned int *prog, const unsig
     if (rc_rows_ensure_f64(c, r) != 0) return -1.0f;
     RcOrderBufs &b = c->order;
     StageInput in;
-    if (stage_inputs(c, prog, off, pcount, nsets, nsegs, kmax, c0, &in) != 0 ||
-        segment_offsets(c, nsegs, n) != 0 || sort_buffers(c, total, false) != 0 ||
-        rc_grow(c, (void **)&b.status, &b.status_cap, (size_t)nsegs, sizeof(int)) != 0 ||
-        rc_grow(c, (void **)&b.val, &b.val_cap, (size_t)nsegs, sizeof(double)) != 0)
+    stage_sets(c, prog, off, pcount, nsets, &in);
+    for (int g = 0; g < nsegs; ++g)
+        (in.sets[(size_t)(g / ntrials)].t_m > 0 ? in.fast : in.general).push_back(g);
+    const bool sorted = what == 1;
+    /* Values and statuses come back in one copy. */
+    const size_t ns = (size_t)nsegs, out_bytes = 12 * ns;
+    if (stage_inputs(c, prog, off, pcount, nsets, nsegs, kmax, c0, nullptr, nullptr, {}, &in) != 0 ||
+        (sorted && segment_offsets(c, nsegs, n) != 0) ||
+        sort_buffers(c, total, sorted, false) != 0 ||
+        rc_grow(c, (void **)&b.val, &b.val_cap, 2 * ns, sizeof(double)) != 0)
         return -1.0f;
-    if (hipMemsetAsync(b.status, 0, sizeof(int) * (size_t)nsegs, c->s_fit) != hipSuccess)
-        return -1.0f;
+    int *d_status = (int *)(b.val + ns);
+    if (hipMemsetAsync(d_status, 0, sizeof(int) * ns, c->s_fit) != hipSuccess) return -1.0f;
     (void)hipEventRecord(c->t0, c->s_fit);
-    os_keys_kernel<false><<<grid_for(total), 256, 0, c->s_fit>>>(
-        in.prog, in.off, in.c0, kmax, r->cols64, r->y64, n, nsegs, ntrials, b.keys, nullptr,
-        b.status);
-    if (hipGetLastError() != hipSuccess || segmented_sort(c, total, nsegs, false) != 0)
+    if (launch_keys(c, false, in, kmax, ntrials, d_status) != 0 ||
+        (sorted && segmented_sort(c, total, nsegs, false) != 0))
         return -1.0f;
-    os_pick_kernel<<<(unsigned)nsegs, 64, 0, c->s_fit>>>(b.keys_out, n, nsegs, what, b.val,
-                                                         b.status);
+    if (sorted)
+        os_mean_kernel<<<(unsigned)nsegs, 64, 0, c->s_fit>>>(b.keys_out, n, nsegs, b.val, d_status);
+    else
+        os_select_kernel<<<(unsigned)nsegs, SEL_THREADS, 0, c->s_fit>>>(b.keys, n, nsegs, b.val,
+                                                                      d_status);
     if (hipGetLastError() != hipSuccess) return -1.0f;
     (void)hipEventRecord(c->t1, c->s_fit);
-    if (hipMemcpyAsync(out_value, b.val, sizeof(double) * (size_t)nsegs, hipMemcpyDeviceToHost,
-                       c->s_fit) != hipSuccess ||
-        hipMemcpyAsync(out_status, b.status, sizeof(int) * (size_t)nsegs, hipMemcpyDeviceToHost,
-                       c->s_fit) != hipSuccess ||
+    b.h_out.resize(out_bytes);
+    if (hipMemcpyAsync(b.h_out.data(), b.val, out_bytes, hipMemcpyDeviceToHost, c->s_fit) !=
+            hipSuccess ||
         hipStreamSynchronize(c->s_fit) != hipSuccess)
         return -1.0f;
+    memcpy(out_value, b.h_out.data(), sizeof(double) * ns);
+    memcpy(out_status, b.h_out.data() + sizeof(double) * ns, sizeof(int) * ns);
     float ms = -1.0f;
     (void)hipEventElapsedTime(&ms, c->t0, c->t1);
     return ms;
@@ -631,18 +982,17 @@ float rc_rank_score_batch(void *ctx, const unsigned int *prog, const unsigned in
     if (rank_prepare(c) != 0) return -1.0f;
     RcOrderBufs &b = c->order;
     StageInput in;
-    if (stage_inputs(c, prog, off, pcount, nsets, nsegs, kmax, c0, &in) != 0 ||
-        segment_offsets(c, nsegs, n) != 0 || sort_buffers(c, total, true) != 0 ||
-        rc_grow(c, (void **)&b.status, &b.status_cap, (size_t)nsegs, sizeof(int)) != 0 ||
+    stage_sets(c, prog, off, pcount, nsets, &in);
+    for (int g = 0; g < nsegs; ++g)
+        (in.sets[(size_t)(g / ntrials)].t_m > 0 ? in.fast : in.general).push_back(g);
+    if (stage_inputs(c, prog, off, pcount, nsets, nsegs, kmax, c0, nullptr, nullptr,
+                     std::vector<int>((size_t)nsegs, 0), &in) != 0 ||
+        segment_offsets(c, nsegs, n) != 0 || sort_buffers(c, total, true, true) != 0 ||
         rc_grow(c, (void **)&b.out, &b.out_cap, 4 * (size_t)nsegs, sizeof(unsigned long long)) != 0)
         return -1.0f;
-    if (hipMemsetAsync(b.status, 0, sizeof(int) * (size_t)nsegs, c->s_fit) != hipSuccess)
-        return -1.0f;
     (void)hipEventRecord(c->t0, c->s_fit);
-    os_keys_kernel<true><<<grid_for(total), 256, 0, c->s_fit>>>(
-        in.prog, in.off, in.c0, kmax, r->cols64, r->y64, n, nsegs, ntrials, b.keys, b.rows,
-        b.status);
-    if (hipGetLastError() != hipSuccess || segmented_sort(c, total, nsegs, true) != 0)
+    if (launch_keys(c, true, in, kmax, ntrials, in.flags) != 0 ||
+        segmented_sort(c, total, nsegs, true) != 0)
         return -1.0f;
     rk_runs_kernel<false><<<(unsigned)nsegs, RK_THREADS, 0, c->s_fit>>>(
         b.keys_out, b.rows_out, n, nsegs, b.start_of, b.B, b.out);
@@ -650,7 +1000,7 @@ float rc_rank_score_batch(void *ctx, const unsigned int *prog, const unsigned in
     (void)hipEventRecord(c->t1, c->s_fit);
     if (hipMemcpyAsync(out, b.out, 4 * sizeof(unsigned long long) * (size_t)nsegs,
                        hipMemcpyDeviceToHost, c->s_fit) != hipSuccess ||
-        hipMemcpyAsync(out_status, b.status, sizeof(int) * (size_t)nsegs, hipMemcpyDeviceToHost,
+        hipMemcpyAsync(out_status, in.flags, sizeof(int) * (size_t)nsegs, hipMemcpyDeviceToHost,
                        c->s_fit) != hipSuccess ||
         hipStreamSynchronize(c->s_fit) != hipSuccess)
         return -1.0f;
@@ -687,25 +1037,61 @@ float rc_max_scan_batch(void *ctx, const unsigned int *prog, const unsigned int 
     RcOrderBufs &b = c->order;
     StageInput in;
     /* Null coords / levels: the maximum only (coordinate -1, level NaN). */
-    std::vector<int> &hc = b.h_coords;
-    std::vector<double> &hl = b.h_levels;
-    hc.assign((size_t)nsegs, -1);
-    hl.assign((size_t)nsegs, __builtin_nan(""));
+    std::vector<int> hc((size_t)nsegs, -1);
+    std::vector<double> hl((size_t)nsegs, __builtin_nan(""));
     if (coords && levels) {
-        for (int s = 0; s < nsegs; ++s) {
-            hc[s] = coords[s];
-            hl[s] = levels[s];
-        }
+        hc.assign(coords, coords + nsegs);
+        hl.assign(levels, levels + nsegs);
     }
-    if (stage_inputs(c, prog, off, pcount, nsets, nsegs, kmax, c0, &in) != 0 ||
-        upload(c, (void **)&b.coords, &b.coords_cap, hc.data(), sizeof(int) * hc.size()) != 0 ||
-        upload(c, (void **)&b.levels, &b.levels_cap, hl.data(), sizeof(double) * hl.size()) != 0 ||
+    stage_sets(c, prog, off, pcount, nsets, &in);
+    /* The record sweep serves a level where the program fits its stack and
+       the constant is one leaf (a sum over several is added in another order
+       than the adjoint sweep's), the value stream a plain maximum; the rest is
+       marked for the general kernel. */
+    std::vector<char> stack((size_t)nsets, 0);
+    for (int s = 0; s < nsets; ++s)
+        stack[(size_t)s] = n <= OR_MAX_ROWS && off[s] % 4 == 0 &&
+                           stack_tree(prog + off[s], in.sets[(size_t)s].m);
+    auto one_leaf = [&](int s, int slot) {
+        int leaves = 0;
+        for (int i = 0; i < in.sets[(size_t)s].m; ++i) {
+            const unsigned int *w = prog + off[s] + 4 * i;
+            leaves += w[0] == OP_CONST && (int)w[3] == slot;
+        }
+        return leaves == 1;
+    };
+    std::vector<int> redo((size_t)nsegs, 0), leveled;
+    for (int g = 0; g < nsegs; ++g) {
+        const int s = g / ntrials;
+        const bool want = pcount[s] > 0 && hc[g] >= 0 && hc[g] < pcount[s] && isfinite(hl[g]) &&
+                          hl[g] >= 0.0;
+        if (want && stack[(size_t)s] && one_leaf(s, hc[g])) leveled.push_back(g);
+        else if (!want && in.sets[(size_t)s].t_m > 0) in.fast.push_back(g);
+        else redo[(size_t)g] = 1;
+    }
+    const int nplain = (int)in.fast.size(), nlevel = (int)leveled.size(), nlist = nplain + nlevel;
+    in.fast.insert(in.fast.end(), leveled.begin(), leveled.end());
+    int tile_rows = 0;
+    const int tiles = or_max_tiles(n, std::max(nlist, 1), &tile_rows);
+    if (stage_inputs(c, prog, off, pcount, nsets, nsegs, kmax, c0, hc.data(), hl.data(), redo,
+                     &in) != 0 ||
+        rc_grow(c, (void **)&b.part, &b.part_cap, (size_t)nlist * (size_t)tiles + 1,
+                sizeof(OrMax)) != 0 ||
         rc_grow(c, (void **)&b.mx, &b.mx_cap, (size_t)nsegs, sizeof(RcMaxOut)) != 0)
         return -1.0f;
+    OrMax *part = (OrMax *)b.part;
+    const OrRows rows = {r->cols64, r->y64, n, r->v};
     (void)hipEventRecord(c->t0, c->s_fit);
+    or_launch_max(false, nplain, c->s_fit, in.lists, in.d_sets, in.d_code, in.prog, in.c0, kmax,
+                  ntrials, in.coords, in.levels, rows, part, tiles, tile_rows, in.flags);
+    or_launch_max(true, nlevel, c->s_fit, in.lists + nplain, in.d_sets, in.d_code, in.prog, in.c0,
+                  kmax, ntrials, in.coords, in.levels, rows,
+                  part + (size_t)nplain * (size_t)tiles, tiles, tile_rows, in.flags);
+    if (nlist > 0)
+        mx_finish_kernel<<<(unsigned)nlist, 64, 0, c->s_fit>>>(in.lists, nlist, part, tiles, b.mx);
     mx_scan_kernel<<<(unsigned)nsegs, MX_THREADS, 0, c->s_fit>>>(
-        in.prog, in.off, in.pcount, in.c0, kmax, b.coords, b.levels, r->cols64, r->y64, n, nsegs,
-        ntrials, b.mx);
+        in.prog, in.off, in.pcount, in.c0, kmax, in.coords, in.levels, r->cols64, r->y64, n, nsegs,
+        ntrials, in.flags, b.mx);
     if (hipGetLastError() != hipSuccess) return -1.0f;
     (void)hipEventRecord(c->t1, c->s_fit);
     if (hipMemcpyAsync(out, b.mx, sizeof(RcMaxOut) * (size_t)nsegs, hipMemcpyDeviceToHost,
