@@ -17,17 +17,24 @@
  * random program.  The reference runs this on the host.
  *
  * MI355X layout.  Every child is a pure function of its position except
- * for the dedup set, which is sequential in (island, slot) order.  So the
- * work is split into parallel passes and one ordered pass:
+ * for the dedup set, which is sequential in (island, slot) order: a child takes
+ * the first of its attempts that no earlier child and no parent has.  All
+ * hashes rank the children alike, so there is one assignment in which no child
+ * could have an earlier attempt, the sequential one, and children that propose
+ * side by side in any order end in it.  The work is split into passes:
  *   vy_meta     one lane per parent: hash and node count (the keys);
  *   vy_seed     the set of parent hashes (open addressing, 64-bit CAS);
- *   vy_try      one lane per child: its first VY_TRY attempts (validity and
- *               hash), independent of every other child;
- *   vy_resolve  one lane walks the children in order against the set and
- *               picks each child's first admissible attempt, generating
- *               later attempts itself only when the first VY_TRY fail;
+ *   vy_try      one lane per (child, attempt) of the first VY_TRY attempts
+ *               (validity and hash), independent of every other;
+ *   vy_resolve  one workgroup settles the dedup: every child proposes its
+ *               first admissible attempt, a hash keeps the first child in
+ *               order that proposes it, and a child that is refused or later
+ *               displaced goes on to its next attempt, generating those past
+ *               VY_TRY itself;
+ *   vy_elite    one wave per island: its best parent;
  *   vy_write    one lane per slot: elites, restarted islands and the chosen
- *               attempt of every child, regenerated from its position.
+ *               attempt of every child, as vy_try kept it or regenerated from
+ *               its position.
  * Without dedup vy_try / vy_resolve are skipped and vy_write takes each
  * child's first valid attempt.  Programs are at most VY_WMAX words wide.
  */
@@ -45,6 +52,9 @@ namespace {
 constexpr int VY_WMAX = 128;  /* widest supported pool slot */
 constexpr int VY_TRY = 8;     /* attempts precomputed per child */
 constexpr int VY_ATTEMPTS = 64;
+/* The most memory for the programs of vy_try's attempts; a pool whose attempts
+   need more makes the chosen ones again. */
+constexpr size_t VY_KEPT_BYTES = (size_t)64 << 20;
 constexpr int VY_MAXOPS = 64;
 constexpr uint32_t VY_HALT = 255;
 
@@ -453,92 +463,137 @@ __global__ void vy_meta(const uint32_t *__restrict__ parents, int n, int width,
    of 0 is stored as 1). */
 __device__ __forceinline__ uint64_t vy_key(uint64_t h) { return h == 0 ? 1ull : h; }
 
-__global__ void vy_clear(uint64_t *__restrict__ table, int cap)
+/* The table: a key and its owner, the first child in order that has proposed
+   it (VY_PARENT for a parent's hash: before every child). */
+constexpr int VY_NOBODY = 0x7fffffff, VY_PARENT = -1;
+
+__global__ void vy_clear(uint64_t *__restrict__ table, int *__restrict__ owner, int cap)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < cap) table[i] = 0ull;
+    if (i >= cap) return;
+    table[i] = 0ull;
+    owner[i] = VY_NOBODY;
 }
 
-__global__ void vy_seed(const uint64_t *__restrict__ phash, int n, uint64_t *table, int cap)
+/* The entry of key k, taking an empty one if there is none: a table never
+   holds more than the parents' keys and one for each child (a key is always
+   its owner's proposal), a quarter of its entries. */
+__device__ __forceinline__ int vy_entry(uint64_t *table, int cap, uint64_t k)
+{
+    unsigned long long *t = (unsigned long long *)table;
+    int i = (int)(k & (uint64_t)(cap - 1));
+    for (int q = 0; q < cap; ++q, i = (i + 1) & (cap - 1)) {
+        const unsigned long long prev = atomicCAS(t + i, 0ull, (unsigned long long)k);
+        if (prev == 0ull || prev == k) return i;
+    }
+    return -1;
+}
+
+__global__ void vy_seed(const uint64_t *__restrict__ phash, int n, uint64_t *table, int *owner,
+                        int cap)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
-    const uint64_t k = vy_key(phash[s]);
-    unsigned long long *t = (unsigned long long *)table;
-    for (int q = 0, i = (int)(k & (uint64_t)(cap - 1)); q < cap; ++q, i = (i + 1) & (cap - 1)) {
-        const unsigned long long prev = atomicCAS(t + i, 0ull, (unsigned long long)k);
-        if (prev == 0ull || prev == k) return;
-    }
+    const int i = vy_entry(table, cap, vy_key(phash[s]));
+    if (i >= 0) atomicMin(owner + i, VY_PARENT);
 }
 
+/* One lane per (child, attempt): the attempts of a child run side by side, so
+   4096 children are 512 waves and not 64 that each make eight in a row. */
 __global__ void vy_try(VyCfg g, const uint32_t *__restrict__ parents, const double *__restrict__ err,
                        const uint32_t *__restrict__ pcost, const unsigned char *__restrict__ restart,
-                       uint64_t *__restrict__ thash, unsigned char *__restrict__ tok)
+                       uint64_t *__restrict__ thash, unsigned char *__restrict__ tok,
+                       uint32_t *__restrict__ kept)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= g.islands * g.pop) return;
-    const int island = c / g.pop, slot = c % g.pop;
+    const long long u = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = (int)(u % VY_TRY);
+    const long long c = u / VY_TRY;
+    if (c >= (long long)g.islands * g.pop) return;
+    const int island = (int)c / g.pop, slot = (int)c % g.pop;
     if (slot == 0 || (restart && restart[island])) return;
     VyProg p;
-    for (int a = 0; a < VY_TRY; ++a) {
-        const bool ok = vy_attempt(g, parents, err, pcost, island, slot, a, p);
-        tok[(size_t)c * VY_TRY + a] = ok ? 1 : 0;
-        thash[(size_t)c * VY_TRY + a] = ok ? vy_hash(p.w, p.len) : 0ull;
+    const bool ok = vy_attempt(g, parents, err, pcost, island, slot, a, p);
+    tok[(size_t)c * VY_TRY + a] = ok ? 1 : 0;
+    thash[(size_t)c * VY_TRY + a] = ok ? vy_hash(p.w, p.len) : 0ull;
+    if (kept && ok) {
+        uint32_t *dst = kept + ((size_t)c * VY_TRY + a) * (size_t)g.width;
+        for (int i = 0; i < g.width; ++i) dst[i] = i < p.len ? p.w[i] : VY_HALT;
     }
 }
 
-/* The ordered pass: one lane, children in (island, slot) order.  Table
-   accesses are volatile (coherent with the atomic inserts of vy_seed). */
-__global__ void vy_resolve(VyCfg g, const uint32_t *__restrict__ parents,
-                           const double *__restrict__ err, const uint32_t *__restrict__ pcost,
-                           const unsigned char *__restrict__ restart,
-                           const uint64_t *__restrict__ thash, const unsigned char *__restrict__ tok,
-                           uint64_t *table, int cap, int *__restrict__ chosen)
+/* The dedup by rounds of proposals in one workgroup.  chosen[c] is child c's
+   current attempt (-1: none is left), entry[c] the table entry it proposed
+   for.  A child's attempt only grows, so the rounds end; the walk in order by
+   one lane that this replaces took 1.4 us a child, the wait for a table entry
+   (4096 children: 5.7 ms, now 0.06). */
+constexpr int VY_THREADS = 1024;
+__global__ __launch_bounds__(VY_THREADS) void vy_resolve(
+    VyCfg g, const uint32_t *__restrict__ parents, const double *__restrict__ err,
+    const uint32_t *__restrict__ pcost, const unsigned char *__restrict__ restart,
+    const uint64_t *__restrict__ thash, const unsigned char *__restrict__ tok, uint64_t *table,
+    int *owner, int cap, int *__restrict__ chosen, int *__restrict__ entry)
 {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    volatile uint64_t *t = table;
-    auto find = [&](uint64_t k, int &at) {
-        int i = (int)(k & (uint64_t)(cap - 1));
-        for (int q = 0; q < cap; ++q, i = (i + 1) & (cap - 1)) {
-            const uint64_t v = t[i];
-            if (v == k) return true;
-            if (v == 0ull) {
-                at = i;
-                return false;
-            }
-        }
-        at = -1;
-        return false;
-    };
-    VyProg p;
-    for (int c = 0; c < g.islands * g.pop; ++c) {
-        const int island = c / g.pop, slot = c % g.pop;
-        if (slot == 0 || (restart && restart[island])) continue;
-        int pick = -1;
-        for (int a = 0; a < VY_ATTEMPTS && pick < 0; ++a) {
-            bool ok;
-            uint64_t h;
-            if (a < VY_TRY) {
-                ok = tok[(size_t)c * VY_TRY + a] != 0;
-                h = thash[(size_t)c * VY_TRY + a];
-            } else {
-                ok = vy_attempt(g, parents, err, pcost, island, slot, a, p);
-                h = ok ? vy_hash(p.w, p.len) : 0ull;
-            }
-            if (!ok) continue;
+    const int n = g.islands * g.pop;
+    bool first = true;
+    for (;;) {
+        int moved = 0;
+        for (int c = threadIdx.x; c < n; c += VY_THREADS) {
+            const int island = c / g.pop, slot = c % g.pop;
+            if (slot == 0 || (restart && restart[island])) continue;
+            int a = first ? -1 : chosen[c];
+            if (!first && (a < 0 || __hip_atomic_load(owner + entry[c], __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT) == c))
+                continue;
             int at = -1;
-            if (find(vy_key(h), at)) continue;
-            if (at >= 0) t[at] = vy_key(h);
-            pick = a;
+            for (++a; a < VY_ATTEMPTS && at < 0; ++a) {
+                bool ok;
+                uint64_t h;
+                if (a < VY_TRY) {
+                    ok = tok[(size_t)c * VY_TRY + a] != 0;
+                    h = thash[(size_t)c * VY_TRY + a];
+                } else {
+                    VyProg p;
+                    ok = vy_attempt(g, parents, err, pcost, island, slot, a, p);
+                    h = ok ? vy_hash(p.w, p.len) : 0ull;
+                }
+                if (!ok) continue;
+                const int i = vy_entry(table, cap, vy_key(h));
+                if (i >= 0 && atomicMin(owner + i, c) > c) at = i;
+            }
+            /* The loop has stepped past the attempt it found. */
+            chosen[c] = at >= 0 ? a - 1 : -1;
+            entry[c] = at;
+            moved = 1;
         }
-        chosen[c] = pick;
+        first = false;
+        if (!__syncthreads_or(moved)) break;
     }
+}
+
+/* Each island's best parent: one wave per island over its slots (the keys are
+   a strict order, so any reduction finds the same one). */
+__global__ __launch_bounds__(64) void vy_elite(VyCfg g, const double *__restrict__ err,
+                                               const uint32_t *__restrict__ pcost,
+                                               int *__restrict__ best)
+{
+    const int base = blockIdx.x * g.pop;
+    int b = base + (int)threadIdx.x;
+    if ((int)threadIdx.x >= g.pop) b = base;
+    for (int s = base + (int)threadIdx.x + 64; s < base + g.pop; s += 64)
+        if (vy_less(err, pcost, s, b)) b = s;
+    for (int o = 32; o > 0; o >>= 1) {
+        const int x = __shfl_xor(b, o, 64);
+        if (vy_less(err, pcost, x, b)) b = x;
+    }
+    if (threadIdx.x == 0) best[blockIdx.x] = b;
 }
 
 __global__ void vy_write(VyCfg g, const uint32_t *__restrict__ parents,
                          const double *__restrict__ err, const uint32_t *__restrict__ pcost,
                          const uint64_t *__restrict__ phash, const unsigned char *__restrict__ restart,
-                         const int *__restrict__ chosen, uint32_t *__restrict__ kids,
+                         const int *__restrict__ chosen, const int *__restrict__ elite,
+                         const uint32_t *__restrict__ kept, const uint64_t *__restrict__ thash,
+                         uint32_t *__restrict__ kids,
                          unsigned short *__restrict__ klen, unsigned short *__restrict__ kcost,
                          uint64_t *__restrict__ khash, double *__restrict__ kerr)
 {
@@ -547,16 +602,27 @@ __global__ void vy_write(VyCfg g, const uint32_t *__restrict__ parents,
     const int island = c / g.pop, slot = c % g.pop;
     uint32_t *dst = kids + (size_t)c * g.width;
     if (!(restart && restart[island]) && slot == 0) {
-        const int base = island * g.pop;
-        int best = base;
-        for (int s = base + 1; s < base + g.pop; ++s)
-            if (vy_less(err, pcost, s, best)) best = s;
+        const int best = elite[island];
         const uint32_t *src = parents + (size_t)best * g.width;
         for (int i = 0; i < g.width; ++i) dst[i] = src[i];
         klen[c] = (unsigned short)vy_logical_len(src, g.width);
         kcost[c] = (unsigned short)pcost[best];
         khash[c] = phash[best];
         kerr[c] = err[best];
+        return;
+    }
+    /* An attempt that vy_try kept is copied (its words from the length on are
+       HALT, and an admissible program ends at its first HALT); any other is
+       made again from its position. */
+    if (kept && !(restart && restart[island]) && chosen[c] >= 0 && chosen[c] < VY_TRY) {
+        const size_t at = (size_t)c * VY_TRY + (size_t)chosen[c];
+        const uint32_t *src = kept + at * (size_t)g.width;
+        for (int i = 0; i < g.width; ++i) dst[i] = src[i];
+        const int len = vy_logical_len(src, g.width);
+        klen[c] = (unsigned short)len;
+        kcost[c] = (unsigned short)max(vy_parse(src, len), 0);
+        khash[c] = thash[at];
+        kerr[c] = __builtin_nan("");
         return;
     }
     VyProg p;
@@ -659,7 +725,13 @@ extern "C" int rc_pool_vary(void *ctx, int from, int islands, int pop, unsigned 
     const size_t o_thash = vy_take(cur, (size_t)n * VY_TRY * 8);
     const size_t o_tok = vy_take(cur, (size_t)n * VY_TRY);
     const size_t o_table = vy_take(cur, (size_t)tcap * 8);
+    const size_t o_owner = vy_take(cur, (size_t)tcap * 4);
     const size_t o_chosen = vy_take(cur, (size_t)n * 4);
+    const size_t o_entry = vy_take(cur, (size_t)n * 4);
+    const size_t o_elite = vy_take(cur, (size_t)islands * 4);
+    const size_t kept_bytes = (size_t)n * VY_TRY * (size_t)width * 4;
+    const bool keep = g.dedup && kept_bytes <= VY_KEPT_BYTES;
+    const size_t o_kept = vy_take(cur, keep ? kept_bytes : 0);
     const size_t o_klen = vy_take(cur, (size_t)n * 2);
     const size_t o_kcost = vy_take(cur, (size_t)n * 2);
     const size_t o_khash = vy_take(cur, (size_t)n * 8);
@@ -696,15 +768,20 @@ extern "C" int rc_pool_vary(void *ctx, int from, int islands, int pop, unsigned 
         return -1;
     const unsigned blocks = (unsigned)((n + 63) / 64);
     vy_meta<<<blocks, 64, 0, s>>>(parents, n, width, d_phash, d_pcost);
+    uint32_t *d_kept = keep ? (uint32_t *)(D + o_kept) : nullptr;
     if (g.dedup) {
-        vy_clear<<<(unsigned)((tcap + 255) / 256), 256, 0, s>>>(d_table, tcap);
-        vy_seed<<<blocks, 64, 0, s>>>(d_phash, n, d_table, tcap);
-        vy_try<<<blocks, 64, 0, s>>>(g, parents, d_err, d_pcost, d_rs, d_thash, d_tok);
-        vy_resolve<<<1, 64, 0, s>>>(g, parents, d_err, d_pcost, d_rs, d_thash, d_tok, d_table, tcap,
-                                    d_chosen);
+        int *d_owner = (int *)(D + o_owner);
+        vy_clear<<<(unsigned)((tcap + 255) / 256), 256, 0, s>>>(d_table, d_owner, tcap);
+        vy_seed<<<blocks, 64, 0, s>>>(d_phash, n, d_table, d_owner, tcap);
+        vy_try<<<(unsigned)(((long long)n * VY_TRY + 63) / 64), 64, 0, s>>>(
+            g, parents, d_err, d_pcost, d_rs, d_thash, d_tok, d_kept);
+        vy_resolve<<<1, VY_THREADS, 0, s>>>(g, parents, d_err, d_pcost, d_rs, d_thash, d_tok,
+                                            d_table, d_owner, tcap, d_chosen, (int *)(D + o_entry));
     }
-    vy_write<<<blocks, 64, 0, s>>>(g, parents, d_err, d_pcost, d_phash, d_rs, d_chosen, kids,
-                                   d_klen, d_kcost, d_khash, d_kerr);
+    int *d_elite = (int *)(D + o_elite);
+    vy_elite<<<(unsigned)islands, 64, 0, s>>>(g, d_err, d_pcost, d_elite);
+    vy_write<<<blocks, 64, 0, s>>>(g, parents, d_err, d_pcost, d_phash, d_rs, d_chosen, d_elite,
+                                   d_kept, d_thash, kids, d_klen, d_kcost, d_khash, d_kerr);
     if (hipGetLastError() != hipSuccess) return -1;
     /* The evaluator translates the pool from its host mirror. */
     std::vector<uint32_t> &mirror = c->pool_host[(from & 1) ^ 1];
