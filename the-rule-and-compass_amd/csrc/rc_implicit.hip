@@ -29,7 +29,7 @@
  * +-1e6, implicit.rs:215-253, 277-409) runs on the host between batched
  * passes: one JAC and one RSS launch per iteration for the whole batch.
  */
-#include "rc_device.h"
+#include "rc_implicit_dev.h"
 #include "rc_internal.h"
 
 #include <math.h>
@@ -39,69 +39,6 @@
 #include <vector>
 
 namespace {
-
-constexpr int IM_MAX_NODES = 96;
-constexpr int IM_KMAX = 20;
-constexpr int IM_STATS = (IM_KMAX + 1) * (IM_KMAX + 2) / 2; /* [J | r] lower triangle */
-constexpr double IM_INV_SQRT_PI = 0.5641895835477563;
-
-enum { IM_SCORE = 0, IM_RSS = 1, IM_JAC = 2 };
-
-struct ImCand {
-    uint32_t off; /* first record word */
-    int m;        /* nodes */
-    int k;        /* constants */
-    int fast;     /* 1: runs the register-stack sweep (im_fast_kernel) */
-    int sub;      /* rows of a sub-tile, items of a group (RcSplit) */
-    int group;
-};
-
-/* The register-stack sweep's limits: values below the top of the stack
-   (the post-order evaluation's depth less one) and input columns. */
-constexpr int IM_SDEPTH = 8;
-constexpr int IM_NVMAX = 4;
-/* A stack file: two components of the 8 stack entries, one in elements
-   0..7 and one in 8..15 (a 16-element vector is indexed with one register
-   move per access; shorter ones are lowered to select chains). */
-typedef double im_d16 __attribute__((ext_vector_type(16)));
-typedef double im_d4 __attribute__((ext_vector_type(4)));
-
-struct ImItem {
-    int cand;
-    int row0;
-    int rows;
-    int pad;
-};
-
-/* value_of (fit.rs:1211-1365) for the fit operator set. */
-__device__ __forceinline__ double im_value(uint32_t op, double a, double b)
-{
-    switch (op) {
-        case OP_ADD: return a + b;
-        case OP_SUB: return a - b;
-        case OP_MUL: return a * b;
-        case OP_DIV: return fabs(b) < 1e-12 ? RC_F64_NAN : a / b;
-        case OP_POW: return pow(a, b);
-        case OP_NEG: return -a;
-        case OP_EXP: return a > 700.0 ? __builtin_inf() : exp(a);
-        case OP_LOG: return log(a);
-        case OP_ABS: return fabs(a);
-        case OP_SQRT: return sqrt(a);
-        case OP_SIN: return sin(a);
-        case OP_COS: return cos(a);
-        case OP_TAN: return tan(a);
-        case OP_SINH: return sinh(a);
-        case OP_COSH: return cosh(a);
-        case OP_TANH: return tanh(a);
-        case OP_SIG: return 1.0 / (1.0 + exp(-a));
-        case OP_GAUSS: return exp(-a * a);
-        case OP_SQUARE: return a * a;
-        case OP_CUBE: return a * a * a;
-        case OP_ERF: return erf(a);
-        case OP_ERFC: return erfc(a);
-        default: return RC_F64_NAN;
-    }
-}
 
 /* Whether expr::eval's guard fires where value_of does not (LOG of a
    non-positive, SQRT of a negative, a non-finite TAN, POW of a negative base
@@ -126,11 +63,6 @@ __device__ __forceinline__ double im_guarded(uint32_t op, double a, double b)
         case OP_POW: return (a < 0.0 && fabs(b - round(b)) > 1e-9) ? RC_F64_NAN : pow(a, b);
         default: return im_value(op, a, b);
     }
-}
-
-__device__ __forceinline__ bool im_is_bin(uint32_t op)
-{
-    return op == OP_ADD || op == OP_SUB || op == OP_MUL || op == OP_DIV || op == OP_POW;
 }
 
 /* Signed distance (metric 0) or f itself (metric 1) of one row at constants
@@ -389,12 +321,6 @@ __global__ __launch_bounds__(64) void im_pass_kernel(
    an exactly cancelling pair of adjoints (which the adjoint sweep skips)
    sits above an infinite partial, the two may differ, and both then flag
    the row in every case the tests hold. */
-__device__ __forceinline__ double im_lm(double p, double t)
-{
-    return (p == 0.0 || t == 0.0) ? 0.0 : p * t;
-}
-__device__ __forceinline__ double im_ld(double t, double x) { return t == 0.0 ? 0.0 : t / x; }
-
 /* A unary node of value_of argument a and guarded argument ga: its value,
    guarded value, whether a guard fires, and its local partial p (the
    tangent is t / p when div, else p * t, both under the zero rule).  Out
@@ -586,7 +512,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void im
     const ImItem it = items[it_i];
     if (run && !run[it.cand]) return;
     const ImCand d = cands[it.cand];
-    if (!d.fast) return;
+    if (d.fast != 1) return;
     const int lane = threadIdx.x;
     const uint32_t *r4 = rec + d.off;
     const double *c = cs + (size_t)it.cand * (size_t)kmax;
@@ -931,7 +857,7 @@ struct ImBatch {
     std::vector<double> h_part;
     std::vector<int> h_bad;
     float ms = 0.0f;
-    bool any_fast = false, any_general = false;
+    bool any_wide = false, any_fast = false, any_general = false;
 
     /* One pass over ni items of mode MODE on stream s: the register-stack
        kernel for the fast candidates, the node-array kernel for the rest. */
@@ -940,6 +866,9 @@ struct ImBatch {
     {
         if (ni <= 0) return;
         RcRows &R = c->sets[0];
+        if (any_wide)
+            im_launch_wide(MODE, R.v, ni, s, d_items, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64,
+                           R.n, metric, d_part, stride, d_bad, run);
         if (any_fast) {
             switch (R.v) {
                 case 1: im_fast_kernel<MODE, 1><<<ni, 64, 0, s>>>(d_items, ni, d_cand, d_rec, d_cs, kmax, R.cols64, R.w64, R.n, metric, d_part, stride, d_bad, run); break;
@@ -984,6 +913,7 @@ struct ImBatch {
                       p <= IM_KMAX;
             std::vector<int> st;
             size_t depth = 0;
+            bool guards = false; /* an operator whose guarded value may differ */
             for (int q = 0; ok && q < m; ++q) {
                 const uint32_t op = w[4 * q], k0 = w[4 * q + 1], k1 = w[4 * q + 2], slot = w[4 * q + 3];
                 if (op == OP_CONST) {
@@ -996,6 +926,7 @@ struct ImBatch {
                            op == OP_POW) {
                     ok = st.size() >= 2 && st.back() == (int)k1 && st[st.size() - 2] == (int)k0;
                     if (ok) { st.pop_back(); st.pop_back(); st.push_back(q); }
+                    guards = guards || op == OP_POW;
                 } else {
                     const bool known = op == OP_SIN || op == OP_COS || op == OP_TAN || op == OP_EXP ||
                                        op == OP_LOG || op == OP_SQRT || op == OP_ABS ||
@@ -1005,6 +936,7 @@ struct ImBatch {
                                        op == OP_ERFC;
                     ok = known && !st.empty() && st.back() == (int)k0;
                     if (ok) { st.pop_back(); st.push_back(q); }
+                    guards = guards || op == OP_LOG || op == OP_SQRT || op == OP_TAN;
                 }
                 depth = std::max(depth, st.size());
             }
@@ -1017,7 +949,9 @@ struct ImBatch {
             cands[i].m = m;
             cands[i].k = p;
             cands[i].fast = (depth <= (size_t)IM_SDEPTH + 1 && R.v >= 1 && R.v <= IM_NVMAX) ? 1 : 0;
-            (cands[i].fast ? any_fast : any_general) = true;
+            if (!guards && depth <= (size_t)IM_WDEPTH + 1 && R.v >= 1 && R.v <= IM_WNV)
+                cands[i].fast = 2;
+            (cands[i].fast == 2 ? any_wide : cands[i].fast == 1 ? any_fast : any_general) = true;
             rec.insert(rec.end(), w, w + words);
         }
         if (rec.empty()) rec.push_back(0);
