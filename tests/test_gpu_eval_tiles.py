@@ -1,0 +1,91 @@
+"""The evaluator's row tiles over small and odd tables, the allocation-free
+entry point where its partial sums take several parts, the one-pass
+correlation score, and the rare operators' shared call, against f64
+reductions of the device's own predictions."""
+import numpy as np
+import pytest
+
+from rcsr_hip import host, lib
+from rcsr_hip.expr import (ADD, ATAN2, CUBE, DIV, ERF, IF, LOG, MAX, MOD, MUL, POW, SIN, SQRT, SUB,
+                           TAN, TANH, const, node, var)
+
+pytestmark = pytest.mark.gpu
+
+TREES = [node(ADD, node(MUL, const(1.3), var(0)), const(0.2)),
+         node(TANH, node(ADD, var(0), node(SIN, var(1)))),
+         node(ERF, node(CUBE, var(0))),
+         node(ADD, node(TAN, var(0)), node(SQRT, node(MUL, var(1), var(1)))),
+         node(MAX, node(MOD, var(0), const(0.7)), node(ATAN2, var(1), var(0))),
+         node(POW, node(MUL, var(0), var(0)), const(0.6)),
+         node(IF, var(0), node(TANH, var(1)), node(DIV, var(0), const(3.0))),
+         node(ADD, const(2.0e4), var(0))]
+
+
+def _evaluator(n):
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((2, n)).astype(np.float32)
+    y = (x[0] + 0.3 * rng.standard_normal(n)).astype(np.float32)
+    return y, host.GpuEvaluator(x.reshape(-1), n, 2, y)
+
+
+def _words(trees):
+    pop = host.Population()
+    assert all(pop.add(t) for t in trees)
+    return pop.arrays()
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 1000, 4096, 4097, 5000, 32768, 32769])
+def test_losses_and_correlation_scores_of_every_tile_size(n):
+    y, ev = _evaluator(n)
+    prog, off = _words(TREES)
+    print(f"eval tiles: {n} rows", flush=True)
+    pred = ev.predict_words(prog, off)
+    assert np.isfinite(pred).all()
+    out, ms = ev.eval_words(prog, off, 0)
+    rr = (pred - y).astype(np.float32)
+    want = np.sum((rr * rr).astype(np.float64), 1)
+    assert ms >= 0 and np.allclose(out, want, rtol=1.2e-7, atol=0)   # one f32 rounding
+    p, dy = pred.astype(np.float64), y.astype(np.float64) - y.astype(np.float64).mean()
+    dp = p - p.mean(1, keepdims=True)
+    ss, yy = np.sum(dp * dp, 1), np.sum(dy * dy)
+    rho = np.zeros(len(TREES)) if n == 1 else (dp @ dy) / np.sqrt(ss * yy)
+    for kind, want in ((5, 1.0 - np.abs(rho)), (6, 1.0 - rho)):
+        score, st, ms = ev.score_words(prog, off, kind)
+        assert ms >= 0 and not st.any()
+        # f64 sums of n terms on both sides; the last program's mean is 2e4 of its
+        # spread, which costs the f64 mean that many of its digits.
+        assert np.allclose(score, want, rtol=0, atol=1e-11)
+    ev.close()
+
+
+def test_correlation_flags_a_row_that_is_not_finite_wherever_it_is():
+    n = 9000
+    x = np.ones((1, n), np.float32)
+    for bad in (0, 1, 4095, 4096, n - 1):
+        x[0, bad] = -1.0
+        ev = host.GpuEvaluator(x.reshape(-1), n, 1, np.arange(n, dtype=np.float32))
+        prog, off = _words([node(LOG, var(0)), var(0)])
+        score, st, ms = ev.score_words(prog, off, 5)
+        assert ms >= 0 and list(st) == [2, 0] and np.isinf(score[0]) and np.isfinite(score[1])
+        x[0, bad] = 1.0
+        ev.close()
+
+
+def test_static_evaluation_in_several_parts():
+    n, copies = 4000, 19000
+    y, ev = _evaluator(n)
+    prog, off = _words(TREES)
+    lens = np.tile(np.diff(off), copies)
+    big = np.tile(prog, copies).astype(np.uint32)
+    boff = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    nprog = len(boff) - 1
+    out = np.zeros(nprog, np.float32)
+    print(f"static evaluation: {nprog} programs x {n} rows", flush=True)
+    ms = ev._L.rc_eval_static(ev.ctx, lib.ptr(big, lib.u32p), lib.ptr(boff, lib.u32p), nprog,
+                              lib.ptr(out, lib.f32p), 0)
+    assert ms >= 0
+    want, ms = ev.eval_words(prog, off, 0)
+    assert ms >= 0
+    assert np.array_equal(out.reshape(copies, -1).view(np.uint32),
+                          np.tile(want, (copies, 1)).view(np.uint32))
+    ev.close()

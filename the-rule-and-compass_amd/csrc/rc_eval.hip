@@ -57,10 +57,6 @@ constexpr uint32_t RC_OP_NAN = 254;
    input column (w >> 16) (var = 1) or the f32 word that follows (var = 0). */
 constexpr uint32_t RC_OP_FUSED = 64;
 
-/* Internal score pass: the per-program mean prediction that the correlation
-   scores centre on (their first pass, eval.cu:930-960). */
-constexpr int RC_SCORE_CORR_MEAN = 100;
-
 constexpr int MODE_EVAL = 0;    /* sum of rho with 1e30 hard failures (rc_eval) */
 constexpr int MODE_SCORE = 1;   /* f64 score objectives + bad flag */
 constexpr int MODE_PREDICT = 2; /* raw predictions */
@@ -621,15 +617,18 @@ __device__ __forceinline__ void rc_fused(uint32_t bop, float *tos, Leaf leaf)
 
 /* Evaluate the program at `pc` for R rows of this lane: rows row0 +
    loff[r] / 4 (clamped in range by the caller). */
-/* Score inputs beyond the rows: score weights (may be null), label signs,
-   per-program mean predictions, the target mean, second per-item sums. */
+/* Score inputs beyond the rows: score weights (may be null), label signs, the
+   target mean, and where an item's further sums go: the classification
+   scores' weights, or RC_CORR_SUMS of the correlation scores. */
 struct RcScoreArgs {
     const double *w;
     const float *tsign;
-    const double *pbar;
     double ybar;
     double *part2;
 };
+/* A tile's mean prediction, its sum of (pred - mean) (y - ybar) and its sum of
+   y - ybar; the sum of (pred - mean)^2 is the item's partial itself. */
+constexpr int RC_CORR_SUMS = 3;
 
 /* Column c of the evaluator's rows: an input (c < nv) or a derived column. */
 __device__ __forceinline__ const float *rc_col(const float *cols, const float *dcols, int n, int nv,
@@ -811,7 +810,12 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
                       (kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED);
     const bool classif = MODE == MODE_SCORE && kind >= RC_SCORE_LOG_LOSS &&
                          kind <= RC_SCORE_HINGE_SQUARED;
-    const double pb = corr ? sa.pbar[p] : 0.0;
+    /* The correlation scores need the moments about the mean (two passes in
+       eval.cu:930-1008).  A tile takes them about its first prediction, shifts
+       them to its own mean at its end, and the finish combines the tiles'
+       means: one pass, with at most a tile's rows between pivot and mean (512
+       programs x 154 001 rows: 1.74 -> 1.15 ms). */
+    double pivot = 0.0, sp = 0.0, sy = 0.0;
     for (int base = row0; base < row1; base += 64 * R) {
         uint32_t loff[R];
         bool ok[R];
@@ -828,6 +832,9 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
         }
         float res[R];
         rc_run<S, R>(pc, cols, dcols, n, nv, row0, loff, res);
+        if (corr && base == row0)
+            pivot = (double)__uint_as_float(
+                (unsigned)__builtin_amdgcn_readfirstlane((int)__float_as_uint(res[0])));
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if (!ok[r]) continue;
@@ -880,15 +887,13 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
                     bad = 1;
                     continue;
                 }
-                if (kind == RC_SCORE_CORR_MEAN) {
-                    acc += (double)pred;
-                    continue;
-                }
                 if (corr) {
-                    const double dp = (double)pred - pb;
+                    const double dp = (double)pred - pivot;
                     const double dy = (double)yv[r] - sa.ybar;
                     acc += dp * dp;
                     acc2 += dp * dy;
+                    sp += dp;
+                    sy += dy;
                     continue;
                 }
                 const double rr = (double)pred - (double)yv[r];
@@ -918,11 +923,21 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
     const int anybad = __any(bad) ? 1 : 0;
     const bool two = corr || classif;
     const double tot2 = two ? rc_wave_sum_f64(acc2) : 0.0;
+    const double totp = corr ? rc_wave_sum_f64(sp) : 0.0;
+    const double toty = corr ? rc_wave_sum_f64(sy) : 0.0;
     if (lane == 0) {
         const size_t item = (size_t)p * (size_t)tiles + (size_t)t;
-        part[item] = tot;
+        const double shift = totp / (double)(row1 - row0);
+        part[item] = corr ? fmax(tot - totp * shift, 0.0) : tot;
         part_bad[item] = anybad;
-        if (two) sa.part2[item] = tot2;
+        if (corr) {
+            double *q = sa.part2 + RC_CORR_SUMS * item;
+            q[0] = pivot + shift;
+            q[1] = tot2 - shift * toty;
+            q[2] = toty;
+        } else if (two) {
+            sa.part2[item] = tot2;
+        }
     }
 }
 
@@ -955,23 +970,41 @@ __global__ __launch_bounds__(256) void rc_derive_kernel(const float *__restrict_
 
 /* Per-program finish in tile order (deterministic). */
 __global__ void rc_eval_finish(const double *__restrict__ part, const int *__restrict__ part_bad,
-                               const double *__restrict__ part2, int nprog, int tiles, int n,
-                               int mode, int kind, double syy, float *__restrict__ out32,
-                               double *__restrict__ out64, int *__restrict__ status,
-                               double *__restrict__ pbar)
+                               const double *__restrict__ part2, int nprog, int tiles,
+                               int tile_rows, int n, int mode, int kind, double syy,
+                               float *__restrict__ out32, double *__restrict__ out64,
+                               int *__restrict__ status)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= nprog) return;
-    const bool two = mode == MODE_SCORE &&
-                     (kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED ||
-                      (kind >= RC_SCORE_LOG_LOSS && kind <= RC_SCORE_HINGE_SQUARED));
-    double s = 0.0, s2 = 0.0;
+    const bool corr = mode == MODE_SCORE &&
+                      (kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED);
+    const bool classif =
+        mode == MODE_SCORE && kind >= RC_SCORE_LOG_LOSS && kind <= RC_SCORE_HINGE_SQUARED;
+    double s = 0.0, s2 = 0.0, pbar = 0.0;
     int bad = 0;
+    const size_t item0 = (size_t)p * (size_t)tiles;
+    auto rows_of = [&](int t) { return (double)min(tile_rows, n - t * tile_rows); };
+    if (corr) {
+#pragma unroll 8
+        for (int t = 0; t < tiles; ++t)
+            pbar += rows_of(t) * part2[RC_CORR_SUMS * (item0 + (size_t)t)];
+        pbar /= (double)n;
+    }
+#pragma unroll 4
     for (int t = 0; t < tiles; ++t) {
-        const size_t item = (size_t)p * (size_t)tiles + (size_t)t;
-        if (mode == MODE_SCORE && kind == RC_SCORE_MAXIMUM) s = fmax(s, part[item]);
-        else s += part[item];
-        if (two) s2 += part2[item];
+        const size_t item = item0 + (size_t)t;
+        if (corr) {
+            const double *q = part2 + RC_CORR_SUMS * item;
+            const double d = q[0] - pbar;
+            s += part[item] + rows_of(t) * d * d;
+            s2 += q[1] + d * q[2];
+        } else if (mode == MODE_SCORE && kind == RC_SCORE_MAXIMUM) {
+            s = fmax(s, part[item]);
+        } else {
+            s += part[item];
+        }
+        if (classif) s2 += part2[item];
         bad |= part_bad[item];
     }
     if (mode == MODE_EVAL) {
@@ -984,9 +1017,7 @@ __global__ void rc_eval_finish(const double *__restrict__ part, const int *__res
         return;
     }
     status[p] = 0;
-    if (kind == RC_SCORE_CORR_MEAN) {
-        pbar[p] = s / (double)n;
-    } else if (kind >= RC_SCORE_LOG_LOSS && kind <= RC_SCORE_HINGE_SQUARED) {
+    if (kind >= RC_SCORE_LOG_LOSS && kind <= RC_SCORE_HINGE_SQUARED) {
         /* Weighted mean; no positive weight is status 4 (eval.cu:917-925). */
         if (!(s2 > 0.0)) {
             out64[p] = __builtin_inf();
@@ -1034,11 +1065,15 @@ namespace {
 
 /* Row tiles are a multiple of 256 rows so every class (R = 4, 2, 1) walks
    whole passes; tiles depend only on n, so a program's sums never depend on
-   the batch it came in. */
+   the batch it came in.  A small table is cut into single passes: 200 programs
+   over 1000 rows are then 800 waves of one pass and not 200 of four (the kernel
+   44 -> 12 us), 4096 programs over 5000 rows have no wave of 904 rows beside
+   one of 4096 (197 -> 84 us), and a generation that fills the card anyway loses
+   nothing (4096 programs over 4096 rows: 0.98 ms a batch either way). */
 int tile_rows_for(int n, int tuned)
 {
     const int whole = ((n + 255) / 256) * 256 > 0 ? ((n + 255) / 256) * 256 : 256;
-    const int t = tuned > 0 ? tuned : 4096;
+    const int t = tuned > 0 ? tuned : n <= 4096 ? 256 : n <= 32768 ? 1024 : 4096;
     return whole < t ? whole : t;
 }
 
@@ -1048,7 +1083,7 @@ void launch_class(int mode, dim3 grid, hipStream_t s, const RcCtx *c, const uint
                   int kind, float *pred, double *part, int *part_bad)
 {
     const RcRows *r = &c->sets[0];
-    const RcScoreArgs sa = {r->w64, c->d_tsign, c->d_pbar, r->ybar, c->d_part2};
+    const RcScoreArgs sa = {r->w64, c->d_tsign, r->ybar, c->d_part2};
     if (mode == MODE_EVAL)
         rc_eval_kernel<S, R, MODE_EVAL><<<grid, 64, 0, s>>>(
             r->cols, c->d_derived, r->v, r->y, r->n, code, meta, plist, ncls, tiles, tile_rows, kind,
@@ -1063,17 +1098,17 @@ void launch_class(int mode, dim3 grid, hipStream_t s, const RcCtx *c, const uint
             part, part_bad, pred, sa);
 }
 
-/* The class launches of one row pass over a translated batch whose class
-   starts are cls[0..4], with explicit partial-sum buffers (nprog * tiles
+/* The class launches of one row pass over a translated batch, class q being
+   the programs lo[q] .. hi[q] of its list, with explicit partial-sum buffers (nprog * tiles
    items each). */
 int launch_classes(const RcCtx *c, int mode, int kind, int nprog, const uint32_t *code,
-                   const uint32_t *meta, const int *cls, int tiles, int tile_rows, hipStream_t s,
+                   const uint32_t *meta, const int *lo, const int *hi, int tiles, int tile_rows, hipStream_t s,
                    float *pred, double *part, int *part_bad)
 {
     for (int q = 0; q < 4; ++q) {
-        const int ncls = cls[q + 1] - cls[q];
+        const int ncls = hi[q] - lo[q];
         if (ncls <= 0) continue;
-        const uint32_t *plist = meta + nprog + cls[q];
+        const uint32_t *plist = meta + nprog + lo[q];
         size_t grid;
         if (tiles < 8) grid = (size_t)ncls * (size_t)tiles;
         else grid = ((size_t)(tiles + 7) / 8) * (size_t)ncls * 8;
@@ -1108,16 +1143,15 @@ int launch_rows(RcCtx *c, int mode, int kind, int nprog, const uint32_t *code,
     if (rc_grow(c, (void **)&c->d_part, &c->part_cap, items, sizeof(double)) != 0) return -1;
     if (rc_grow(c, (void **)&c->d_part_bad, &c->part_bad_cap, items, sizeof(int)) != 0) return -1;
     if (mode == MODE_SCORE &&
-        (rc_grow(c, (void **)&c->d_part2, &c->part2_cap, items, sizeof(double)) != 0 ||
-         rc_grow(c, (void **)&c->d_pbar, &c->pbar_cap, (size_t)nprog, sizeof(double)) != 0))
+        rc_grow(c, (void **)&c->d_part2, &c->part2_cap, RC_CORR_SUMS * items, sizeof(double)) != 0)
         return -1;
-    if (launch_classes(c, mode, kind, nprog, code, meta, c->cls_start, tiles, tile_rows, s, pred,
+    if (launch_classes(c, mode, kind, nprog, code, meta, c->cls_start, c->cls_start + 1, tiles, tile_rows, s, pred,
                        c->d_part, c->d_part_bad) != 0)
         return -1;
     if (mode == MODE_PREDICT) return 0;
     rc_eval_finish<<<(nprog + 127) / 128, 128, 0, s>>>(c->d_part, c->d_part_bad, c->d_part2, nprog,
-                                                       tiles, n, mode, kind, r->syy, c->d_out,
-                                                       c->d_score, c->d_status, c->d_pbar);
+                                                       tiles, tile_rows, n, mode, kind, r->syy,
+                                                       c->d_out, c->d_score, c->d_status);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1279,10 +1313,7 @@ float score_current(RcCtx *c, int nprog, int kind, const int *pcount, double *ou
     if (ensure_outputs(c, nprog) != 0) return -1.0f;
     double t = rc_now_ms();
     (void)hipEventRecord(c->t0, c->s_eval);
-    const bool corr = kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED;
-    if ((corr && launch_rows(c, MODE_SCORE, RC_SCORE_CORR_MEAN, nprog, c->arena_code[c->arena_slot],
-                             c->arena_meta[c->arena_slot], c->s_eval, nullptr) != 0) ||
-        launch_rows(c, MODE_SCORE, kind, nprog, c->arena_code[c->arena_slot],
+    if (launch_rows(c, MODE_SCORE, kind, nprog, c->arena_code[c->arena_slot],
                     c->arena_meta[c->arena_slot], c->s_eval, nullptr) != 0) {
         st->failed = 1;
         return -1.0f;
@@ -1350,7 +1381,9 @@ float score_current(RcCtx *c, int nprog, int kind, const int *pcount, double *ou
    before it is read. */
 constexpr size_t RC_STATIC_BYTES = (size_t)32 << 20;
 constexpr int RC_STATIC_MAX_DEVICES = 64;
-static __device__ __align__(256) unsigned char scratch[RC_STATIC_BYTES];
+/* Room for some programs' partial sums beside the largest streams. */
+constexpr size_t RC_STATIC_SPARE = 4096;
+static __device__ __align__(256) unsigned char scratch[RC_STATIC_BYTES + RC_STATIC_SPARE];
 void *g_static_ptr[RC_STATIC_MAX_DEVICES];
 std::mutex g_static_mu;
 
@@ -1404,14 +1437,26 @@ float rc_eval_static(void *ctx, const unsigned int *prog, const unsigned int *of
     (void)rc_translate_programs(prog, off, nprog, r->v, code, meta, cls, &derived, c->derived_cols);
     const int tile_rows = tile_rows_for(n, c->tune_eval_tile);
     const int tiles = (n + tile_rows - 1) / tile_rows;
-    const size_t items = (size_t)nprog * (size_t)tiles;
     size_t cur = 0;
     const size_t o_code = static_take(cur, code.size() * 4);
     const size_t o_meta = static_take(cur, meta.size() * 4);
+    const size_t o_out = static_take(cur, (size_t)nprog * sizeof(float));
+    /* A batch fits with partial sums of 4096-row tiles (or the tuned ones)
+       beside its streams.  A small table's tiles are smaller: its programs then
+       run in as many parts as their partial sums need. */
+    const size_t wide = c->tune_eval_tile > 0 ? (size_t)tile_rows : 4096;
+    size_t whole = cur;
+    const size_t wide_items = (size_t)nprog * (((size_t)n + wide - 1) / wide);
+    (void)static_take(whole, wide_items * sizeof(double));
+    (void)static_take(whole, wide_items * sizeof(int));
+    if (whole > RC_STATIC_BYTES) return -2.0f; /* the batch does not fit the static array */
+    /* (two alignments; at most 32 tiles are smaller than the ones above) */
+    const size_t left = RC_STATIC_BYTES + RC_STATIC_SPARE - static_take(cur, 0) - 512;
+    const int per = (int)std::min<size_t>(left / (12 * (size_t)tiles), (size_t)nprog);
+    if (per < 1) return -2.0f;
+    const size_t items = (size_t)per * (size_t)tiles;
     const size_t o_part = static_take(cur, items * sizeof(double));
     const size_t o_bad = static_take(cur, items * sizeof(int));
-    const size_t o_out = static_take(cur, (size_t)nprog * sizeof(float));
-    if (cur > RC_STATIC_BYTES) return -2.0f; /* the batch does not fit the static array */
     uint32_t *d_code = (uint32_t *)(base + o_code);
     uint32_t *d_meta = (uint32_t *)(base + o_meta);
     double *d_part = (double *)(base + o_part);
@@ -1430,12 +1475,24 @@ float rc_eval_static(void *ctx, const unsigned int *prog, const unsigned int *of
                                                         (int)nhoist);
         if (hipGetLastError() != hipSuccess) return -1.0f;
     }
-    if (launch_classes(c, MODE_EVAL, loss, nprog, d_code, d_meta, cls, tiles, tile_rows, s, nullptr,
-                       d_part, d_bad) != 0)
-        return -1.0f;
-    rc_eval_finish<<<(nprog + 127) / 128, 128, 0, s>>>(d_part, d_bad, nullptr, nprog, tiles, n,
-                                                       MODE_EVAL, loss, r->syy, d_out, nullptr,
-                                                       nullptr, nullptr);
+    const uint32_t *plist = meta.data() + nprog;
+    for (int p0 = 0; p0 < nprog; p0 += per) {
+        const int p1 = std::min(nprog, p0 + per);
+        /* Each class lists its programs in increasing order. */
+        int lo[4], hi[4];
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t *a = plist + cls[q], *b = plist + cls[q + 1];
+            lo[q] = (int)(std::lower_bound(a, b, (uint32_t)p0) - plist);
+            hi[q] = (int)(std::lower_bound(a, b, (uint32_t)p1) - plist);
+        }
+        const ptrdiff_t back = (ptrdiff_t)p0 * (ptrdiff_t)tiles;
+        if (launch_classes(c, MODE_EVAL, loss, nprog, d_code, d_meta, lo, hi, tiles, tile_rows, s,
+                           nullptr, d_part - back, d_bad - back) != 0)
+            return -1.0f;
+        rc_eval_finish<<<(p1 - p0 + 127) / 128, 128, 0, s>>>(d_part, d_bad, nullptr, p1 - p0, tiles,
+                                                             tile_rows, n, MODE_EVAL, loss, r->syy,
+                                                             d_out + p0, nullptr, nullptr);
+    }
     (void)hipEventRecord(c->t1, s);
     if (hipGetLastError() != hipSuccess ||
         hipMemcpyAsync(out, d_out, (size_t)nprog * sizeof(float), hipMemcpyDeviceToHost, s) !=
