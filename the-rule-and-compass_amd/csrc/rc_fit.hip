@@ -1291,6 +1291,8 @@ static FtProg translate_fit(const uint32_t *w, int words, int p, int nvars, bool
     return out;
 }
 
+constexpr int FT_SIDES = 3;
+
 /* Device-resident state of the fit arm (grown at the high-water mark). */
 struct RcFitState {
     unsigned char *dev = nullptr;
@@ -1307,10 +1309,10 @@ struct RcFitState {
     int n_pass[4] = {0, 0, 0, 0};
     FtState *last_state = nullptr;
     int last_nprog = 0;
-    /* A second stream with its fork / join events: the small class
-       kernels of a pass run on it beside the large ones. */
-    hipStream_t side = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    /* Side streams with their fork / join events: class kernels of a pass
+       run on them beside those on the fit stream. */
+    hipStream_t side[FT_SIDES] = {};
+    hipEvent_t ev_fork = nullptr, ev_join[FT_SIDES] = {};
 };
 
 void rc_fit_state_free(RcCtx *c)
@@ -1320,9 +1322,11 @@ void rc_fit_state_free(RcCtx *c)
     if (c->fit->graph) (void)hipGraphDestroy(c->fit->graph);
     if (c->fit->dev) (void)hipFree(c->fit->dev);
     if (c->fit->host) (void)hipHostFree(c->fit->host);
-    if (c->fit->side) (void)hipStreamDestroy(c->fit->side);
+    for (int q = 0; q < FT_SIDES; ++q) {
+        if (c->fit->side[q]) (void)hipStreamDestroy(c->fit->side[q]);
+        if (c->fit->ev_join[q]) (void)hipEventDestroy(c->fit->ev_join[q]);
+    }
     if (c->fit->ev_fork) (void)hipEventDestroy(c->fit->ev_fork);
-    if (c->fit->ev_join) (void)hipEventDestroy(c->fit->ev_join);
     delete c->fit;
     c->fit = nullptr;
 }
@@ -1777,9 +1781,15 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
     int *d_pbad = (int *)(D + o_pbad);
     int *d_pskip = (int *)(D + o_pskip);
 
-    if ((!f->side && hipStreamCreateWithFlags(&f->side, hipStreamNonBlocking) != hipSuccess) ||
-        (!f->ev_fork && hipEventCreateWithFlags(&f->ev_fork, hipEventDisableTiming) != hipSuccess) ||
-        (!f->ev_join && hipEventCreateWithFlags(&f->ev_join, hipEventDisableTiming) != hipSuccess)) {
+    auto event = [](hipEvent_t &e) {
+        return e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    };
+    bool have = event(f->ev_fork);
+    for (int q = 0; q < FT_SIDES; ++q)
+        have = have && event(f->ev_join[q]) &&
+               (f->side[q] ||
+                hipStreamCreateWithFlags(&f->side[q], hipStreamNonBlocking) == hipSuccess);
+    if (!have) {
         (void)hipGetLastError();
         return -1.0f;
     }
@@ -1801,97 +1811,120 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
                                             d_pskip, d_outc, d_sse, d_st, all64 ? 1 : 0);
     };
     auto ctrl = [&](int op) { mark(3, [&]() { ctrl0(op); }); };
-    /* The classes of a pass write disjoint items: the large ones run on
-       the fit stream, the small ones on the side stream between a fork and
-       a join, so the small classes fill the slots the large ones leave. */
-    hipStream_t &sd = f->side;
-    auto fork = [&]() {
-        (void)hipEventRecord(f->ev_fork, s);
-        (void)hipStreamWaitEvent(sd, f->ev_fork, 0);
+    /* The classes of a pass write disjoint items, so their kernels may run side
+       by side between a fork and a join.  Where the pass fills the card, the
+       4-row classes run in order on the fit stream (beside each other they
+       measured slower: 154 ms against 143 for 1024 fits x 262 144 rows) and
+       the small ones on one side stream, in the slots those leave; where it
+       does not, a class is as long as one of its waves, and the classes are
+       dealt out over all streams (64 fits x 100 003 rows in four classes:
+       10.1 -> 7.1 ms). */
+    const bool filled = nitems >= RC_ITEMS_WANTED;
+    hipStream_t on[NA];
+    int used = 0; /* side streams */
+    for (int q = 0, dealt = 0; q < NA; ++q) {
+        const bool large = q < 2 || q >= 8 || (all64 && q < 4);
+        int at = filled ? (large ? 0 : 1) : dealt % (FT_SIDES + 1);
+        if (lofs[q + 1] > lofs[q]) ++dealt;
+        else at = 0;
+        on[q] = at == 0 ? nullptr : f->side[at - 1];
+        used = std::max(used, at);
+    }
+    auto fork = [&](int sides) {
+        if (sides > 0) (void)hipEventRecord(f->ev_fork, s);
+        for (int q = 0; q < sides; ++q) (void)hipStreamWaitEvent(f->side[q], f->ev_fork, 0);
     };
-    auto join = [&]() {
-        (void)hipEventRecord(f->ev_join, sd);
-        (void)hipStreamWaitEvent(s, f->ev_join, 0);
+    auto join = [&](int sides) {
+        for (int q = 0; q < sides; ++q) {
+            (void)hipEventRecord(f->ev_join[q], f->side[q]);
+            (void)hipStreamWaitEvent(s, f->ev_join[q], 0);
+        }
     };
-    auto asm_launch = [&](auto kern, int q, hipStream_t st) {
+    auto stream_of = [&](int q) { return on[q] ? on[q] : s; };
+    auto asm_launch = [&](auto kern, int q) {
+        const hipStream_t st = stream_of(q);
         const int nl = lofs[q + 1] - lofs[q];
         if (nl <= 0) return;
         kern<<<nl, 64, 0, st>>>(d_items, d_lists + lofs[q], nl, d_cand, d_rows, d_code, d_run_a,
                                 d_cp32, d_cp64, d_pgram, tri_stride, d_ploss, d_pbad, d_pskip);
     };
-    auto vm_asm = [&](int kc, int r, bool polish, int q, hipStream_t st) {
+    auto vm_asm = [&](int kc, int r, bool polish, int q) {
+        const hipStream_t st = stream_of(q);
         vm_launch_asm(kc, r, q >= 8 ? q / 2 - 3 : 0, lslots[q & 1], polish, lofs[q + 1] - lofs[q], st, d_items, d_lists + lofs[q], d_cand,
                       d_rows, d_code, d_run_a, d_cp32, d_cp64, d_pgram, tri_stride, d_ploss,
                       d_pbad, d_pskip, d_p64);
     };
-    auto asm64_launch = [&](auto kern, int q, hipStream_t st) {
+    auto asm64_launch = [&](auto kern, int q) {
+        const hipStream_t st = stream_of(q);
         const int nl = lofs[q + 1] - lofs[q];
         if (nl <= 0) return;
         kern<<<nl, 64, 0, st>>>(d_items, d_lists + lofs[q], nl, d_cand, d_rows, d_code, d_run_a,
                                 d_cp64, d_pgram, tri_stride, d_ploss, d_pbad, d_pskip);
     };
-    auto vm_asm64 = [&](int kc, bool polish, int q, hipStream_t st) {
+    auto vm_asm64 = [&](int kc, bool polish, int q) {
+        const hipStream_t st = stream_of(q);
         vm_launch_asm64(kc, polish, lofs[q + 1] - lofs[q], st, d_items, d_lists + lofs[q], d_cand,
                         d_rows, d_code, d_run_a, d_cp64, d_pgram, tri_stride, d_ploss, d_pbad,
                         d_pskip);
     };
     auto asm_pass0 = [&](int polish) {
-        fork();
+        fork(used);
         if (all64) {
             /* The classes of 4 f32 rows per lane (0, 1, 8..11) are empty here. */
-            vm_asm64(16, polish != 0, 2, s);
-            vm_asm64(32, polish != 0, 3, s);
+            vm_asm64(16, polish != 0, 2);
+            vm_asm64(32, polish != 0, 3);
             if (polish) {
-                asm64_launch(ft_asm64_kernel<16, false, true>, 4, sd);
-                asm64_launch(ft_asm64_kernel<32, false, true>, 5, sd);
-                asm64_launch(ft_asm64_kernel<16, true, true>, 6, sd);
-                asm64_launch(ft_asm64_kernel<32, true, true>, 7, sd);
+                asm64_launch(ft_asm64_kernel<16, false, true>, 4);
+                asm64_launch(ft_asm64_kernel<32, false, true>, 5);
+                asm64_launch(ft_asm64_kernel<16, true, true>, 6);
+                asm64_launch(ft_asm64_kernel<32, true, true>, 7);
             } else {
-                asm64_launch(ft_asm64_kernel<16, false, false>, 4, sd);
-                asm64_launch(ft_asm64_kernel<32, false, false>, 5, sd);
-                asm64_launch(ft_asm64_kernel<16, true, false>, 6, sd);
-                asm64_launch(ft_asm64_kernel<32, true, false>, 7, sd);
+                asm64_launch(ft_asm64_kernel<16, false, false>, 4);
+                asm64_launch(ft_asm64_kernel<32, false, false>, 5);
+                asm64_launch(ft_asm64_kernel<16, true, false>, 6);
+                asm64_launch(ft_asm64_kernel<32, true, false>, 7);
             }
         } else if (polish) {
-            vm_asm(16, 4, true, 0, s);
-            vm_asm(32, 4, true, 1, s);
-            vm_asm(16, 4, true, 8, s);
-            vm_asm(32, 4, true, 9, s);
-            vm_asm(16, 4, true, 10, s);
-            vm_asm(32, 4, true, 11, s);
-            vm_asm(16, 2, true, 2, sd);
-            vm_asm(32, 2, true, 3, sd);
-            asm_launch(ft_asm_kernel<16, false, true>, 4, sd);
-            asm_launch(ft_asm_kernel<32, false, true>, 5, sd);
-            asm_launch(ft_asm_kernel<16, true, true>, 6, sd);
-            asm_launch(ft_asm_kernel<32, true, true>, 7, sd);
+            vm_asm(16, 4, true, 0);
+            vm_asm(32, 4, true, 1);
+            vm_asm(16, 4, true, 8);
+            vm_asm(32, 4, true, 9);
+            vm_asm(16, 4, true, 10);
+            vm_asm(32, 4, true, 11);
+            vm_asm(16, 2, true, 2);
+            vm_asm(32, 2, true, 3);
+            asm_launch(ft_asm_kernel<16, false, true>, 4);
+            asm_launch(ft_asm_kernel<32, false, true>, 5);
+            asm_launch(ft_asm_kernel<16, true, true>, 6);
+            asm_launch(ft_asm_kernel<32, true, true>, 7);
         } else {
-            vm_asm(16, 4, false, 0, s);
-            vm_asm(32, 4, false, 1, s);
-            vm_asm(16, 4, false, 8, s);
-            vm_asm(32, 4, false, 9, s);
-            vm_asm(16, 4, false, 10, s);
-            vm_asm(32, 4, false, 11, s);
-            vm_asm(16, 2, false, 2, sd);
-            vm_asm(32, 2, false, 3, sd);
-            asm_launch(ft_asm_kernel<16, false, false>, 4, sd);
-            asm_launch(ft_asm_kernel<32, false, false>, 5, sd);
-            asm_launch(ft_asm_kernel<16, true, false>, 6, sd);
-            asm_launch(ft_asm_kernel<32, true, false>, 7, sd);
+            vm_asm(16, 4, false, 0);
+            vm_asm(32, 4, false, 1);
+            vm_asm(16, 4, false, 8);
+            vm_asm(32, 4, false, 9);
+            vm_asm(16, 4, false, 10);
+            vm_asm(32, 4, false, 11);
+            vm_asm(16, 2, false, 2);
+            vm_asm(32, 2, false, 3);
+            asm_launch(ft_asm_kernel<16, false, false>, 4);
+            asm_launch(ft_asm_kernel<32, false, false>, 5);
+            asm_launch(ft_asm_kernel<16, true, false>, 6);
+            asm_launch(ft_asm_kernel<32, true, false>, 7);
         }
-        join();
+        join(used);
     };
     auto asm_pass = [&](int polish) { mark(0, [&]() { asm_pass0(polish); }); };
     /* One trial pass over the item lists at offsets of (full, first
        halves or second halves) with the run flags run. */
     auto trial_lists = [&](bool exact_, const int *of, const int *run) {
         const bool exact = exact_ || all64;
-        fork();
+        const int sides = of[NT] > of[1] ? 1 : 0; /* any outside the fit VM */
+        fork(sides);
         for (int q = 0; q < NT; ++q) {
             const int nl = of[q + 1] - of[q];
             if (nl <= 0) continue;
             const int *L = d_lists + of[q];
-            const hipStream_t st = q == 0 ? s : sd;
+            const hipStream_t st = q == 0 ? s : f->side[0];
             if (!exact) {
                 if (q == 0)
                     vm_launch_trial(false, nl, st, d_items, L, d_cand, d_rows, d_code, run, d_cp32, d_cp64, d_ploss,
@@ -1910,13 +1943,20 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
                     ft_trial_kernel<double, true><<<nl, 64, 0, st>>>(d_items, L, nl, d_cand, d_rows, d_code, run, d_cp64, d_ploss);
             }
         }
-        join();
+        join(sides);
     };
 
     auto trial_pass0 = [&](bool exact) { trial_lists(exact, tofs, d_run_t); };
     /* An LM trial pass: the first halves, the prune, the second halves of
-       the candidates not yet rejected. */
+       the candidates not yet rejected.  Where the whole pass does not fill the
+       card twice, the halves would only take one after the other what runs
+       side by side: it is one pass then (the pruned flags stay clear). */
+    const bool halves = nitems >= RC_ITEMS_WANTED;
     auto trial_lm0 = [&]() {
+        if (!halves) {
+            trial_lists(false, tofs, d_run_t);
+            return;
+        }
         trial_lists(false, tofs_a, d_run_t);
         ft_trial_prune<<<(nprog + 63) / 64, 64, 0, s>>>(nprog, d_state, d_cand, d_ploss, d_run_t,
                                                          d_run_b);
