@@ -54,10 +54,13 @@ constexpr size_t FT_P64_CAP = (size_t)32 << 30;
 constexpr int SMALL_S = 8, SMALL_AS = 8, SMALL_TAPE = 32;
 constexpr int BIG_S = 100, BIG_AS = 100, BIG_TAPE = 100;
 
+constexpr int FT_TOLD = 4;
+
 /* Candidate stages of the device state machine. */
 enum {
     ST_NEED_ASM = 1, ST_NEED_TRIAL = 2, ST_LM_DONE = 3, ST_P_NEED_ASM = 4, ST_P_NEED_TRIAL = 5,
-    ST_DONE = 6
+    ST_DONE = 6,
+    ST_KNOWN = 7 /* an LM trial that is rejected without its pass (told_rejected) */
 };
 
 /* Control operations. */
@@ -79,7 +82,11 @@ struct FtState {
     int halvings, polish_it, pre_status, acc_bits; /* acc_bits: LM decision q accepted (bit q) */
     int n_asm, n_trial, n_exact, n_decided; /* passes consumed, LM decisions (telemetry) */
     int pruned; /* this LM trial was rejected on its first half (ft_trial_prune) */
-    int pad_[2];
+    int ntold;  /* entries of told that hold a vector, and the next to take */
+    int told_at;
+    /* f32 constants (bits) whose loss is known not to be below `best`: those
+       `best` was measured at and trials rejected since (told_rejected). */
+    unsigned told[FT_TOLD][FT_KMAX];
 };
 static_assert(sizeof(FtState) % 16 == 0, "FtState is copied in 16-byte words");
 
@@ -732,8 +739,9 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
                                        double *__restrict__ outc, double *__restrict__ outsse,
                                        int *__restrict__ outstatus, int all64);
 __device__ __forceinline__ void ctrl_after_solve(int kind, int rc, int cand, FtState *s, int k,
-                                              const double *delta, float *__restrict__ cp32,
-                                              double *__restrict__ cp64, int all64);
+                                              const double *delta, bool known,
+                                              float *__restrict__ cp32, double *__restrict__ cp64,
+                                              int all64);
 __device__ __forceinline__ void ctrl_flags(int op, int cand, const FtState *s,
                                         int *__restrict__ run_asm, int *__restrict__ run_trial);
 
@@ -832,7 +840,21 @@ __global__ __launch_bounds__(64) void ft_ctrl_kernel(
     if (solve != CT_SOLVE_NONE) {
         const int rc = ft_solve_wave(s->jtj, s->jtr, sh_lambda, k, sh_delta, L, sh_dsc, sh_rhs,
                                      lane);
-        if (lane == 0) ctrl_after_solve(solve, rc, cand, s, k, sh_delta, cp32, cp64, all64);
+        /* Whether the step's constants are told, by the wave: two vectors at a
+           time, a constant a lane. */
+        bool known = false;
+        if (solve == CT_SOLVE_LM && s->ntold > 0) {
+            const int j = lane & 31;
+            const unsigned t =
+                j < k ? __float_as_uint((float)clamp_step(s->c[j] + sh_delta[j])) : 0u;
+            for (int q0 = 0; q0 < s->ntold; q0 += 2) {
+                const int q = q0 + (lane >> 5);
+                const unsigned long long ne =
+                    __ballot(q >= s->ntold || (j < k && s->told[q][j] != t));
+                known = known || (unsigned)ne == 0u || (unsigned)(ne >> 32) == 0u;
+            }
+        }
+        if (lane == 0) ctrl_after_solve(solve, rc, cand, s, k, sh_delta, known, cp32, cp64, all64);
     }
     if (lane == 0) ctrl_flags(op, cand, s, run_asm, run_trial);
     __syncthreads();
@@ -854,6 +876,50 @@ __device__ __forceinline__ void ctrl_set_pass64(double *__restrict__ cp64, int c
                                              const double *v)
 {
     for (int j = 0; j < FT_KMAX; ++j) cp64[(size_t)cand * FT_KMAX + j] = j < k ? v[j] : 0.0;
+}
+
+/* An LM trial's loss is a function of its f32 constants alone: the same rows,
+   stream, items and order of sums.  Near the optimum the solves at growing
+   lambda keep giving the step that was just rejected, or none that f32 can
+   see, so most trials there would measure a loss that is known: that of the
+   constants `best` was measured at, or of a trial rejected since.  Such a
+   trial is rejected without its pass (1024 fits x 262 144 rows: 198 -> 182 ms). */
+__device__ __forceinline__ bool told_rejected(const FtState *s, int k)
+{
+    for (int q = 0; q < s->ntold; ++q) {
+        bool same = true;
+        for (int j = 0; j < k; ++j)
+            same = same && s->told[q][j] == __float_as_uint((float)s->trial[j]);
+        if (same) return true;
+    }
+    return false;
+}
+__device__ __forceinline__ void tell(FtState *s, int k)
+{
+    for (int j = 0; j < k; ++j) s->told[s->told_at][j] = __float_as_uint((float)s->trial[j]);
+    s->told_at = (s->told_at + 1) % FT_TOLD;
+    if (s->ntold < FT_TOLD) s->ntold += 1;
+}
+
+/* The end of an LM iteration's inner loop (count or break): the next IRLS
+   round, or the end of the LM loop. */
+__device__ __forceinline__ void ctrl_end_inner(FtState *s)
+{
+    s->round += 1;
+    s->it = 0;
+    if (s->round >= s->rounds || s->best == 0.0 || s->status != 0) {
+        s->stage = ST_LM_DONE;
+    } else {
+        s->assembled = 0; /* new IRLS weights, new Gram */
+    }
+}
+
+/* A rejected LM iteration: the next lambda, or the end of the inner loop. */
+__device__ __forceinline__ void ctrl_reject(FtState *s)
+{
+    s->lambda *= 6.0;
+    s->it += 1;
+    if (s->lambda > 1e9 || s->it >= s->inner) ctrl_end_inner(s);
 }
 
 /* The serial part of a control step (one lane): LM / IRLS / polish state
@@ -897,16 +963,6 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
             s->stage = ST_NEED_ASM;
         }
     };
-    auto end_inner = [&]() {
-        /* The inner loop of this round ended (count or break). */
-        s->round += 1;
-        s->it = 0;
-        if (s->round >= s->rounds || s->best == 0.0 || s->status != 0) {
-            s->stage = ST_LM_DONE;
-        } else {
-            s->assembled = 0; /* new IRLS weights, new Gram */
-        }
-    };
 
     switch (op) {
         case CT_INIT: {
@@ -935,6 +991,8 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
             s->n_exact = 0;
             s->acc_bits = 0;
             s->n_decided = 0;
+            s->ntold = 0;
+            s->told_at = 0;
             if (s->pre_status >= 0) {
                 s->stage = ST_DONE;
             } else if (s->iters > 0) {
@@ -965,17 +1023,29 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
             break;
         }
         case CT_AFTER_TRIAL: {
+            if (s->stage == ST_KNOWN) {
+                s->n_decided += 1;
+                ctrl_reject(s);
+                lm_next();
+                break;
+            }
             if (!ran_trial || s->stage != ST_NEED_TRIAL) break;
             const double tsse = s->pruned ? __builtin_inf() : sh_loss;
             s->pruned = 0;
+            if (tsse < s->best) s->ntold = s->told_at = 0; /* a new best */
+            if (!all64) tell(s, k);
             if (!(tsse < s->best) && s->halvings > 0) {
-                /* True-metric Armijo halving for the L1 arm (eval.cu:2496-2509). */
-                s->halvings -= 1;
-                for (int j = 0; j < k; ++j) s->trial[j] = cc[j] + 0.5 * (s->trial[j] - cc[j]);
-                set_pass32(s->trial);
-                break;
+                /* True-metric Armijo halving for the L1 arm (eval.cu:2496-2509),
+                   past the halved steps known to be rejected. */
+                do {
+                    s->halvings -= 1;
+                    for (int j = 0; j < k; ++j) s->trial[j] = cc[j] + 0.5 * (s->trial[j] - cc[j]);
+                } while (s->halvings > 0 && told_rejected(s, k));
+                if (!told_rejected(s, k)) {
+                    set_pass32(s->trial);
+                    break;
+                }
             }
-            bool brk = false;
             if (tsse < s->best && s->n_decided < 31) s->acc_bits |= 1 << s->n_decided;
             s->n_decided += 1;
             if (tsse < s->best) {
@@ -984,13 +1054,11 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
                 s->lambda = fmax(s->lambda / 8.0, 1e-12);
                 s->improved = 1;
                 s->assembled = 0;
-                if (s->best == 0.0) brk = true;
+                s->it += 1;
+                if (s->best == 0.0 || s->it >= s->inner) ctrl_end_inner(s);
             } else {
-                s->lambda *= 6.0;
-                if (s->lambda > 1e9) brk = true;
+                ctrl_reject(s);
             }
-            s->it += 1;
-            if (brk || s->it >= s->inner) end_inner();
             lm_next();
             break;
         }
@@ -1071,10 +1139,12 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
 }
 
 /* The end of a control step that solved: stage the trial (clamped step from
-   the current constants) or record the failed solve. */
+   the current constants; known: its constants are told), or record the failed
+   solve. */
 __device__ __forceinline__ void ctrl_after_solve(int kind, int rc, int cand, FtState *s, int k,
-                                              const double *delta, float *__restrict__ cp32,
-                                              double *__restrict__ cp64, int all64)
+                                              const double *delta, bool known,
+                                              float *__restrict__ cp32, double *__restrict__ cp64,
+                                              int all64)
 {
     if (rc == 1) {
         if (kind == CT_SOLVE_LM) {
@@ -1088,10 +1158,16 @@ __device__ __forceinline__ void ctrl_after_solve(int kind, int rc, int cand, FtS
     if (rc == 4) s->srank = 1;
     for (int j = 0; j < k; ++j) s->trial[j] = clamp_step(s->c[j] + delta[j]);
     if (kind == CT_SOLVE_LM) {
+        s->halvings = s->irls ? 2 : 0;
+        while (known && s->halvings > 0) {
+            s->halvings -= 1;
+            for (int j = 0; j < k; ++j) s->trial[j] = s->c[j] + 0.5 * (s->trial[j] - s->c[j]);
+            known = told_rejected(s, k);
+        }
+        s->stage = known ? ST_KNOWN : ST_NEED_TRIAL;
+        if (known) return;
         if (all64) ctrl_set_pass64(cp64, cand, k, s->trial);
         else ctrl_set_pass32(cp32, cand, k, s->trial);
-        s->halvings = s->irls ? 2 : 0;
-        s->stage = ST_NEED_TRIAL;
     } else {
         ctrl_set_pass64(cp64, cand, k, s->trial);
         s->halvings = s->irls ? 1 : 0;
