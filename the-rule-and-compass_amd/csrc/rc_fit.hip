@@ -1857,19 +1857,6 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
     int *d_pbad = (int *)(D + o_pbad);
     int *d_pskip = (int *)(D + o_pskip);
 
-    auto event = [](hipEvent_t &e) {
-        return e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-    };
-    bool have = event(f->ev_fork);
-    for (int q = 0; q < FT_SIDES; ++q)
-        have = have && event(f->ev_join[q]) &&
-               (f->side[q] ||
-                hipStreamCreateWithFlags(&f->side[q], hipStreamNonBlocking) == hipSuccess);
-    if (!have) {
-        (void)hipGetLastError();
-        return -1.0f;
-    }
-
     std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> marks;
     auto mark = [&](int kind, auto &&fn) {
         if (!f->profile) { fn(); return; }
@@ -1896,15 +1883,31 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
        dealt out over all streams (64 fits x 100 003 rows in four classes:
        10.1 -> 7.1 ms). */
     const bool filled = nitems >= RC_ITEMS_WANTED;
-    hipStream_t on[NA];
+    int on[NA];   /* 0: the fit stream, else the side stream */
     int used = 0; /* side streams */
     for (int q = 0, dealt = 0; q < NA; ++q) {
         const bool large = q < 2 || q >= 8 || (all64 && q < 4);
         int at = filled ? (large ? 0 : 1) : dealt % (FT_SIDES + 1);
         if (lofs[q + 1] > lofs[q]) ++dealt;
         else at = 0;
-        on[q] = at == 0 ? nullptr : f->side[at - 1];
+        on[q] = at;
         used = std::max(used, at);
+    }
+    /* Streams are made when a batch first needs them (a stream costs a tenth of
+       a millisecond): the assembly's, and one for the trial passes' general
+       kernels. */
+    auto event = [](hipEvent_t &e) {
+        return e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    };
+    const int nsides = std::max(used, tofs[NT] > tofs[1] ? 1 : 0);
+    bool have = nsides == 0 || event(f->ev_fork);
+    for (int q = 0; q < nsides; ++q)
+        have = have && event(f->ev_join[q]) &&
+               (f->side[q] ||
+                hipStreamCreateWithFlags(&f->side[q], hipStreamNonBlocking) == hipSuccess);
+    if (!have) {
+        (void)hipGetLastError();
+        return -1.0f;
     }
     auto fork = [&](int sides) {
         if (sides > 0) (void)hipEventRecord(f->ev_fork, s);
@@ -1916,7 +1919,7 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
             (void)hipStreamWaitEvent(s, f->ev_join[q], 0);
         }
     };
-    auto stream_of = [&](int q) { return on[q] ? on[q] : s; };
+    auto stream_of = [&](int q) { return on[q] ? f->side[on[q] - 1] : s; };
     auto asm_launch = [&](auto kern, int q) {
         const hipStream_t st = stream_of(q);
         const int nl = lofs[q + 1] - lofs[q];
