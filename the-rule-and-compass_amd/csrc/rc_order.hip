@@ -473,8 +473,8 @@ __global__ __launch_bounds__(RK_THREADS) void rk_runs_kernel(
 /* ---- the exact maximum-error scan ----------------------------------------- */
 
 /* One workgroup per segment marked in redo, those that the row kernels do not
-   run and those in which they met a row that is not finite
-   (eval.cu:4505-4600): max |r| as an integer
+   run and those in which they met a row or a derivative that is not finite or
+   may have left the range of f64 on its way (eval.cu:4505-4600): max |r| as an integer
    max of bit patterns with the lowest row on ties; with a constant `coord`
    and a finite level t >= 0, the intersection of the per-row intervals
    {delta : |r_i + b_i delta| <= t}, b_i = d pred_i / d c_coord from the f64

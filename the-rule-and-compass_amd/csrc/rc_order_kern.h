@@ -50,7 +50,8 @@ int or_max_tiles(int n, int nsegs, int *tile_rows);
 /* Maximum scan of the segments segs[0 .. nlist): level false, the maximum by
    the value stream; true, the maximum and the level's interval by the record
    sweep.  part holds nlist * tiles entries; redo[seg] is set where a row is
-   not finite or a derivative's product left the range of f64. */
+   not finite, or a partial of its derivative is not or leads out of the range of
+   f64. */
 void or_launch_max(bool level, int nlist, hipStream_t s, const int *segs, const OrSet *sets,
                    const uint32_t *code, const uint32_t *prog, const double *c0, int kmax,
                    int ntrials, const int *coords, const double *levels, OrRows rows, OrMax *part,

@@ -89,68 +89,125 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void or
     if (bad) status[seg] = 2;
 }
 
-/* A tangent's product under the adjoint sweep's zero rule; `off` is set where
-   two nonzero factors leave the range of f64. */
-__device__ __forceinline__ double or_tan(double p, double t, int &off)
-{
-    if (p == 0.0 || t == 0.0) return 0.0;
-    const double r = p * t;
-    off |= r == 0.0 || !isfinite(r);
-    return r;
-}
-
 /* Prediction and its derivative by constant slot j for two rows a lane, in one
    forward sweep over the post-order records: a value and a tangent per stack
    entry, the top in fixed registers, the entries below in a 16-element vector
    a row (values in 0..7, tangents in 8..15) indexed by the wave-uniform depth.
-   The local partials are ft_rec_hand_down's.  The product of the partials on
-   the constant's way to the root is taken from the leaf up, the adjoint
-   sweep's from the root down: the same up to rounding while it stays in range
-   (off). */
+   The local partials are ft_rec_hand_down's.
+
+   The constant is one leaf, so its derivative is the product of the partials on
+   one path, which the adjoint sweep takes from the root down and this one from
+   the leaf up.  The sweep from the root ends at the first partial of zero (the
+   derivative is zero, whatever is below it) or that is not finite (neither is
+   the derivative).  Seen from the leaf that is the last such partial: it is
+   noted, in place of one noted before, and the product starts again from 1
+   above it.  The adjoint of a node above that is the last of these products
+   over the node's own, so the least and the greatest binary exponent of the
+   products say whether any adjoint left 2^+-800; while none did, and no product
+   leaves 2^+-1000, both sweeps stay in the normal range at every step and agree
+   to rounding.  Any other row, and one that ends in a partial that is not
+   finite, sends its segment to the general kernel. */
+enum { OR_ZERO = 1, OR_WILD = 4, OR_REDO = 16 }; /* the first two shifted by the row */
+constexpr double OR_BIG = 0x1p1000, OR_SMALL = 0x1p-1000;
+constexpr int OR_ADJOINT = 800;
+/* A factor that an adjoint meets before another one. */
+constexpr double OR_FACTOR_BIG = 0x1p200, OR_FACTOR_SMALL = 0x1p-200;
+
+/* A node's values and tangents and what its partials were (OR_*). */
 struct OrDual {
     double v[2], t[2];
+    int ev;
 };
-__device__ __noinline__ OrDual or_unary(unsigned op_, OrDual a, int &off)
+
+__device__ __forceinline__ bool or_in_range(double u)
+{
+    return fabs(u) >= OR_SMALL && fabs(u) <= OR_BIG;
+}
+__device__ __forceinline__ bool or_mild(double f)
+{
+    return fabs(f) >= OR_FACTOR_SMALL && fabs(f) <= OR_FACTOR_BIG;
+}
+/* The tangent t through the partial p; off the path both stay zero. */
+__device__ __forceinline__ double or_tan(double p, double t, int r, int &ev)
+{
+    if (t == 0.0) return 0.0;
+    if (p == 0.0 || !isfinite(p)) {
+        ev |= (p == 0.0 ? OR_ZERO : OR_WILD) << r;
+        return 1.0;
+    }
+    const double u = p * t;
+    if (!or_in_range(u)) ev |= OR_REDO;
+    return u;
+}
+
+__device__ __noinline__ OrDual or_unary(unsigned op_, double v0, double v1, double t0, double t1)
 {
     const unsigned op = vm_uniform(op_);
+    const double v[2] = {v0, v1}, t[2] = {t0, t1};
     OrDual o;
+    o.ev = 0;
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-        o.v[r] = ft_unary(op, a.v[r]);
-        o.t[r] = a.t[r] == 0.0 ? 0.0
-                               : or_tan(ft_unary_partial<double>(op, a.v[r], o.v[r]), a.t[r], off);
+        o.v[r] = ft_unary(op, v[r]);
+        o.t[r] = t[r] == 0.0
+                     ? 0.0
+                     : or_tan(ft_unary_partial<double>(op, v[r], o.v[r]), t[r], r, o.ev);
     }
     return o;
 }
-__device__ __noinline__ OrDual or_divide_or_pow(unsigned op_, OrDual a, OrDual b, int &off)
+
+/* A division or a power with the path's tangent t on its left or right side:
+   t / d and -t l / (d d), t d pow(l, d - 1) and t pow(l, d) log(l) for l > 0,
+   else 0.  In the last three an adjoint meets the factors f and g one by one. */
+__device__ __noinline__ OrDual or_divide_or_pow(unsigned op_, double l0, double l1, double d0,
+                                                double d1, double t0, double t1, int left)
 {
     const unsigned op = vm_uniform(op_);
+    const double lv[2] = {l0, l1}, dv[2] = {d0, d1}, tv[2] = {t0, t1};
     OrDual o;
+    o.ev = 0;
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-        const double l = a.v[r], d = b.v[r];
-        double tl = 0.0, tr = 0.0;
+        const double l = lv[r], d = dv[r], t = tv[r];
         o.v[r] = ft_binary(op, l, d);
+        o.t[r] = 0.0;
+        if (t == 0.0) continue;
+        double u = 0.0, f = 1.0, g = 0.0;
+        bool mild = true;
         if (op == OP_DIV) {
-            if (a.t[r] != 0.0) tl = a.t[r] / d;
-            if (b.t[r] != 0.0) tr = -b.t[r] * l / (d * d);
-            off |= !isfinite(tl) || !isfinite(tr) || (a.t[r] != 0.0 && tl == 0.0) ||
-                   (b.t[r] != 0.0 && l != 0.0 && tr == 0.0);
+            const double q = left ? d : d * d;
+            if (!left) f = l;
+            g = isinf(q) ? 0.0 : q == 0.0 ? RC_F64_NAN : q;
+            u = left ? t / d : -t * l / q;
+            mild = left || or_mild(l);
         } else if (l > 0.0) {
-            if (a.t[r] != 0.0) tl = or_tan(d * pow(l, d - 1.0), a.t[r], off);
-            if (b.t[r] != 0.0) tr = or_tan(pow(l, d) * log(l), b.t[r], off);
+            f = left ? d : pow(l, d);
+            g = left ? pow(l, d - 1.0) : log(l);
+            u = t * f * g;
+            mild = or_mild(f);
         }
-        o.t[r] = tl + tr;
+        if (!isfinite(f) || !isfinite(g)) {
+            o.ev |= OR_WILD << r;
+            u = 1.0;
+        } else if (f == 0.0 || (g == 0.0 && mild)) {
+            o.ev |= OR_ZERO << r;
+            u = 1.0;
+        } else if (!mild || !or_in_range(u)) {
+            o.ev |= OR_REDO;
+        }
+        o.t[r] = u;
     }
     return o;
 }
 
 __device__ __forceinline__ OrDual or_dual(const uint32_t *__restrict__ rec, int m,
                                           const double *__restrict__ c, int j, const OrRows &R,
-                                          const int (&q)[2], int &off)
+                                          const int (&q)[2])
 {
     dv16 S0, S1;
-    OrDual t = {{0.0, 0.0}, {0.0, 0.0}};
+    OrDual t = {{0.0, 0.0}, {0.0, 0.0}, 0};
+    int ev = 0;                       /* of the path so far */
+    int least[2] = {0, 0}, most[2] = {0, 0}; /* exponents since the last start */
     int sp = -1; /* entries below the top; -1: empty */
     for (int i = 0; i < m; ++i) {
         const uint4 w = ((const uint4 *)rec)[i]; /* operator, children, slot */
@@ -172,28 +229,59 @@ __device__ __forceinline__ OrDual or_dual(const uint32_t *__restrict__ rec, int 
                 t.v[1] = col[q[1]];
                 t.t[0] = t.t[1] = 0.0;
             }
-        } else if (ft_is_binary(op)) {
+            continue;
+        }
+        if (op == OP_ADD || op == OP_SUB) { /* the tangent as it is */
             --sp;
-            const OrDual a = {{S0[sp], S1[sp]}, {S0[sp + 8], S1[sp + 8]}};
+            const double av[2] = {S0[sp], S1[sp]}, at[2] = {S0[sp + 8], S1[sp + 8]};
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                t.v[r] = op == OP_ADD ? av[r] + t.v[r] : av[r] - t.v[r];
+                t.t[r] = op == OP_ADD ? at[r] + t.t[r] : at[r] - t.t[r];
+            }
+            continue;
+        }
+        if (ft_is_binary(op)) {
+            --sp;
+            const double av[2] = {S0[sp], S1[sp]}, at[2] = {S0[sp + 8], S1[sp + 8]};
             if (op == OP_MUL) {
+                t.ev = 0;
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
-                    t.t[r] = or_tan(t.v[r], a.t[r], off) + or_tan(a.v[r], t.t[r], off);
-                    t.v[r] = a.v[r] * t.v[r];
-                }
-            } else if (op == OP_ADD || op == OP_SUB) {
-#pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    t.v[r] = op == OP_ADD ? a.v[r] + t.v[r] : a.v[r] - t.v[r];
-                    t.t[r] = op == OP_ADD ? a.t[r] + t.t[r] : a.t[r] - t.t[r];
+                    t.t[r] = or_tan(t.v[r], at[r], r, t.ev) + or_tan(av[r], t.t[r], r, t.ev);
+                    t.v[r] = av[r] * t.v[r];
                 }
             } else {
-                t = or_divide_or_pow(op, a, t, off);
+                const int left = at[0] != 0.0 || at[1] != 0.0;
+                t = or_divide_or_pow(op, av[0], av[1], t.v[0], t.v[1], left ? at[0] : t.t[0],
+                                     left ? at[1] : t.t[1], left);
             }
         } else {
-            t = or_unary(op, t, off);
+            t = or_unary(op, t.v[0], t.v[1], t.t[0], t.t[1]);
+        }
+        ev |= t.ev & OR_REDO;
+        if (t.t[0] == 0.0 && t.t[1] == 0.0) continue; /* off the path */
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const int what = t.ev & ((OR_ZERO | OR_WILD) << r);
+            const int e = __builtin_amdgcn_frexp_exp(t.t[r]); /* 0 off the path */
+            if (what) {
+                ev = (ev & ~((OR_ZERO | OR_WILD) << r)) | what;
+                least[r] = most[r] = 0;
+            } else {
+                least[r] = min(least[r], e);
+                most[r] = max(most[r], e);
+            }
         }
     }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int e = __builtin_amdgcn_frexp_exp(t.t[r]);
+        if (e - least[r] > OR_ADJOINT || most[r] - e > OR_ADJOINT) ev |= OR_REDO;
+        if (ev & (OR_ZERO << r)) t.t[r] = 0.0;
+        if (ev & (OR_WILD << r)) ev |= OR_REDO;
+    }
+    t.ev = ev & OR_REDO;
     return t;
 }
 
@@ -223,14 +311,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LEVEL ? 2 : 
 #pragma unroll
         for (int r = 0; r < RR; ++r) q[r] = min(base + 64 * r + lane, R.n - 1);
         double pred[RR], b[RR];
-        int off = 0;
         if constexpr (LEVEL) {
-            const OrDual o = or_dual(prog + d.r_off, d.m, cst, coord, R, q, off);
+            const OrDual o = or_dual(prog + d.r_off, d.m, cst, coord, R, q);
 #pragma unroll
             for (int r = 0; r < RR; ++r) {
                 pred[r] = o.v[r];
                 b[r] = o.t[r];
             }
+            bad |= o.ev;
         } else {
             const vm_d4 o = or_value((const uint2 *)(code + d.t_off), d.t_m, cst, R, q);
 #pragma unroll
@@ -239,13 +327,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LEVEL ? 2 : 
                 b[r] = 0.0;
             }
         }
-        bad |= off;
 #pragma unroll
         for (int r = 0; r < RR; ++r) {
             const int row = base + 64 * r + lane;
             if (row >= end) continue;
             const double rr = pred[r] - R.y64[row];
-            if (or_bad_row(pred[r], rr) || !isfinite(b[r])) {
+            if (or_bad_row(pred[r], rr)) {
                 bad = 1;
                 continue;
             }
