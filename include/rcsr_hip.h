@@ -245,7 +245,8 @@ int rc_set_fit_mode(void *ctx, int mode);
                                 the program fits the 4-row files (built-in) or 2
      RC_TUNE_EVAL_TILE_ROWS     rows per evaluation tile: a multiple of 256 in
                                 [256, 4194304] (built-in: 4096, 1024 up to
-                                32768 rows, 256 up to 4096)
+                                32768 rows, 256 up to 4096; the correlation
+                                scores take at most 4096)
    rc_set_tuning returns the previous value, or -1 for an unknown key or a
    value out of range; rc_get_tuning returns the current value or -1. */
 #define RC_TUNE_FIT_TILE_ROWS 1

@@ -71,6 +71,32 @@ def test_correlation_flags_a_row_that_is_not_finite_wherever_it_is():
         ev.close()
 
 
+# The first row's prediction is far from all others, over tiles of the built-in
+# size and of the largest that can be set: the moments about a pivot near it
+# would lose as many digits as a tile has rows.
+@pytest.mark.parametrize("n,tile", [(300, 0), (4096, 4096), (60000, 0), (1 << 20, 1 << 20)])
+@pytest.mark.parametrize("outliers", [1, 40])
+def test_correlation_of_predictions_with_an_outlier_in_the_first_row(n, tile, outliers):
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((1, n)).astype(np.float32)
+    y = (x[0] + 0.3 * rng.standard_normal(n)).astype(np.float32)
+    x[0, :outliers] = 1e6
+    ev = host.GpuEvaluator(x.reshape(-1), n, 1, y)
+    assert ev.set_tuning(host.TUNE_EVAL_TILE_ROWS, tile) == 0
+    prog, off = _words([var(0)])
+    print(f"correlation with {outliers} outliers: {n} rows, tile {tile}", flush=True)
+    p, q = x[0].astype(np.longdouble), y.astype(np.longdouble)
+    dp, dy = p - p.mean(), q - q.mean()
+    rho = float(np.sum(dp * dy) / np.sqrt(np.sum(dp * dp) * np.sum(dy * dy)))
+    score, st, ms = ev.score_words(prog, off, 6)
+    assert ms >= 0 and not st.any()
+    # 1 - r of an r near 0: sums of n / 64 terms a lane, their roundings of 2^-53
+    # adding up like a random walk, and up to 16 times that in the tile that the
+    # outliers are in.
+    assert abs(score[0] - (1.0 - rho)) <= 16 * 2.0 ** -53 * max(np.sqrt(n / 64), 8) * max(rho, 1e-3) + 4e-16
+    ev.close()
+
+
 def test_static_evaluation_in_several_parts():
     n, copies = 4000, 19000
     y, ev = _evaluator(n)

@@ -287,6 +287,31 @@ __device__ __forceinline__ double rc_wave_sum_f64(double v)
     return v;
 }
 
+/* The same sum in another fixed order by DPP moves, which wait for no LDS
+   permutes: pairs, quads, eights and rows of 16, then the rows one after the
+   other (a sum that each tile of a correlation score waits for, 16 000 programs
+   x 32 768 rows: 4.04 -> 3.96 ms, 3.95 without that sum).  All 64 lanes must be
+   active. */
+template <int CTRL, int ROWS> __device__ __forceinline__ double rc_dpp_f64(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double rc_wave_sum_dpp(double v)
+{
+    v += rc_dpp_f64<0xb1, 0xf>(v);  /* quad_perm 1 0 3 2 */
+    v += rc_dpp_f64<0x4e, 0xf>(v);  /* quad_perm 2 3 0 1 */
+    v += rc_dpp_f64<0x141, 0xf>(v); /* row_half_mirror */
+    v += rc_dpp_f64<0x140, 0xf>(v); /* row_mirror */
+    v += rc_dpp_f64<0x142, 0xa>(v); /* row_bcast15 into rows 1 and 3 */
+    v += rc_dpp_f64<0x143, 0xc>(v); /* row_bcast31 into rows 2 and 3 */
+    const long long b = __double_as_longlong(v);
+    return __hiloint2double(__builtin_amdgcn_readlane((int)(b >> 32), 63),
+                            __builtin_amdgcn_readlane((int)b, 63));
+}
+
 __device__ __forceinline__ int rc_wave_or(int v)
 {
     return __any(v) ? 1 : 0;

@@ -629,6 +629,9 @@ struct RcScoreArgs {
 /* A tile's mean prediction, its sum of (pred - mean) (y - ybar) and its sum of
    y - ybar; the sum of (pred - mean)^2 is the item's partial itself. */
 constexpr int RC_CORR_SUMS = 3;
+/* The most rows of a tile of the correlation scores: it bounds what the shift
+   to a tile's mean can cancel. */
+constexpr int RC_CORR_TILE = 4096;
 
 /* Column c of the evaluator's rows: an input (c < nv) or a derived column. */
 __device__ __forceinline__ const float *rc_col(const float *cols, const float *dcols, int n, int nv,
@@ -811,10 +814,13 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
     const bool classif = MODE == MODE_SCORE && kind >= RC_SCORE_LOG_LOSS &&
                          kind <= RC_SCORE_HINGE_SQUARED;
     /* The correlation scores need the moments about the mean (two passes in
-       eval.cu:930-1008).  A tile takes them about its first prediction, shifts
-       them to its own mean at its end, and the finish combines the tiles'
-       means: one pass, with at most a tile's rows between pivot and mean (512
-       programs x 154 001 rows: 1.74 -> 1.15 ms). */
+       eval.cu:930-1008).  A tile takes them about the mean of its first step's
+       predictions, shifts them to its own mean at its end, and the finish
+       combines the tiles' means: one pass (512 programs x 154 001 rows: 1.74 ->
+       1.15 ms).  The shift cancels at most tile / step of the squares, for the
+       step's own squares bound its mean: 64 where the tile has RC_CORR_TILE rows
+       and the step 64, whatever the rows are.  About a single prediction it
+       would be the tile's rows where that one is far from the others. */
     double pivot = 0.0, sp = 0.0, sy = 0.0;
     for (int base = row0; base < row1; base += 64 * R) {
         uint32_t loff[R];
@@ -832,9 +838,12 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
         }
         float res[R];
         rc_run<S, R>(pc, cols, dcols, n, nv, row0, loff, res);
-        if (corr && base == row0)
-            pivot = (double)__uint_as_float(
-                (unsigned)__builtin_amdgcn_readfirstlane((int)__float_as_uint(res[0])));
+        if (corr && base == row0) {
+            double first = 0.0;
+#pragma unroll
+            for (int r = 0; r < R; ++r) first += ok[r] ? (double)res[r] : 0.0;
+            pivot = rc_wave_sum_dpp(first) / (double)min(64 * R, row1 - row0);
+        }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if (!ok[r]) continue;
@@ -923,7 +932,8 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
     const int anybad = __any(bad) ? 1 : 0;
     const bool two = corr || classif;
     const double tot2 = two ? rc_wave_sum_f64(acc2) : 0.0;
-    const double totp = corr ? rc_wave_sum_f64(sp) : 0.0;
+    /* The pivot of a tile of one step is its mean already. */
+    const double totp = corr && row1 - row0 > 64 * R ? rc_wave_sum_f64(sp) : 0.0;
     const double toty = corr ? rc_wave_sum_f64(sy) : 0.0;
     if (lane == 0) {
         const size_t item = (size_t)p * (size_t)tiles + (size_t)t;
@@ -1137,7 +1147,10 @@ int launch_rows(RcCtx *c, int mode, int kind, int nprog, const uint32_t *code,
     RcRows *r = &c->sets[0];
     const int n = r->n;
     if (n <= 0) return -1;
-    const int tile_rows = tile_rows_for(n, c->tune_eval_tile);
+    const bool corr = mode == MODE_SCORE &&
+                      (kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED);
+    int tile_rows = tile_rows_for(n, c->tune_eval_tile);
+    if (corr) tile_rows = std::min(tile_rows, RC_CORR_TILE);
     const int tiles = (n + tile_rows - 1) / tile_rows;
     const size_t items = (size_t)nprog * (size_t)tiles;
     if (rc_grow(c, (void **)&c->d_part, &c->part_cap, items, sizeof(double)) != 0) return -1;
