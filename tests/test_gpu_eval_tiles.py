@@ -4,6 +4,7 @@ correlation score, and the rare operators' shared call, against f64
 reductions of the device's own predictions."""
 import numpy as np
 import pytest
+import torch
 
 from rcsr_hip import host, lib
 from rcsr_hip.expr import (ADD, ATAN2, CUBE, DIV, ERF, IF, LOG, MAX, MOD, MUL, POW, SIN, SQRT, SUB,
@@ -94,6 +95,24 @@ def test_correlation_of_predictions_with_an_outlier_in_the_first_row(n, tile, ou
     # adding up like a random walk, and up to 16 times that in the tile that the
     # outliers are in.
     assert abs(score[0] - (1.0 - rho)) <= 16 * 2.0 ** -53 * max(np.sqrt(n / 64), 8) * max(rho, 1e-3) + 4e-16
+    ev.close()
+
+
+def test_only_the_scores_with_further_sums_hold_memory_for_them():
+    n, copies = 4096, 7500
+    y, ev = _evaluator(n)
+    prog, off = _words(TREES)
+    lens = np.tile(np.diff(off), copies)
+    big = np.tile(prog, copies).astype(np.uint32)
+    boff = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    assert ev.eval_words(big, boff, 0)[1] >= 0    # grows the sums that every score has too
+    print(f"score memory: {len(boff) - 1} programs x {n} rows", flush=True)
+    free = torch.cuda.mem_get_info()[0]
+    score, st, ms = ev.score_words(big, boff, 0)
+    assert ms >= 0
+    # 960 000 items: 8 bytes each for a second sum would be 7.7 MB; the values and
+    # statuses of the call are 0.7 MB.
+    assert free - torch.cuda.mem_get_info()[0] <= 4 << 20
     ev.close()
 
 

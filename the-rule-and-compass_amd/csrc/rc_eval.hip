@@ -1155,8 +1155,11 @@ int launch_rows(RcCtx *c, int mode, int kind, int nprog, const uint32_t *code,
     const size_t items = (size_t)nprog * (size_t)tiles;
     if (rc_grow(c, (void **)&c->d_part, &c->part_cap, items, sizeof(double)) != 0) return -1;
     if (rc_grow(c, (void **)&c->d_part_bad, &c->part_bad_cap, items, sizeof(int)) != 0) return -1;
-    if (mode == MODE_SCORE &&
-        rc_grow(c, (void **)&c->d_part2, &c->part2_cap, RC_CORR_SUMS * items, sizeof(double)) != 0)
+    const bool classif =
+        mode == MODE_SCORE && kind >= RC_SCORE_LOG_LOSS && kind <= RC_SCORE_HINGE_SQUARED;
+    const size_t sums = corr ? RC_CORR_SUMS : classif ? 1 : 0; /* beside an item's partial */
+    if (sums > 0 &&
+        rc_grow(c, (void **)&c->d_part2, &c->part2_cap, sums * items, sizeof(double)) != 0)
         return -1;
     if (launch_classes(c, mode, kind, nprog, code, meta, c->cls_start, c->cls_start + 1, tiles, tile_rows, s, pred,
                        c->d_part, c->d_part_bad) != 0)
