@@ -2,8 +2,11 @@
 itself (small items, RcSplit) and in a batch large enough for whole groups of
 rows has the same constants, loss and status, for each arm that splits its
 rows this way and at row counts on either side of a sub-tile's edge."""
+import threading
+
 import numpy as np
 import pytest
+import torch
 
 from rcsr_hip import host
 from rcsr_hip.expr import ADD, COS, MUL, SIN, SQUARE, SUB, const, node, var
@@ -74,4 +77,29 @@ def test_implicit_scores_do_not_depend_on_the_batch(n):
     full, sf, mf = ev.implicit_score_batch(plans * 4200)
     assert ms >= 0 and mf >= 0 and not st.any() and not sf.any()
     assert np.all(full == alone[0])
+    ev.close()
+
+
+def test_implicit_scores_hold_two_sums_an_item():
+    """8000 candidates x 8192 rows are 128 000 items: 2 MB of sums, where the
+    fit's triangles would be 236 MB.  A second thread watches the free memory."""
+    n, copies = 8192, 8000
+    ev = _evaluator(n)
+    plans = [host.gpu_fit_plan(CURVE[0])] * copies
+    assert ev.implicit_score_batch(plans)[2] >= 0
+    print(f"split: implicit score memory, {copies} x {n}", flush=True)
+    before = torch.cuda.mem_get_info()[0]
+    least, stop = [before], threading.Event()
+
+    def watch():
+        while not stop.is_set():
+            least[0] = min(least[0], torch.cuda.mem_get_info()[0])
+
+    t = threading.Thread(target=watch)
+    t.start()
+    score, st, ms = ev.implicit_score_batch(plans)
+    stop.set()
+    t.join()
+    assert ms >= 0 and not st.any()
+    assert before - least[0] <= 32 << 20
     ev.close()

@@ -894,9 +894,9 @@ struct ImBatch {
     }
 
     /* Post-order validation as the fit path's (canonical children, supported
-       operators, slots in range). */
+       operators, slots in range); stride: doubles of an item's partial. */
     int setup(RcCtx *ctx, const unsigned *prog, const unsigned *off, const int *pcount, int np,
-              int km)
+              int km, int stride)
     {
         c = ctx;
         nprog = np;
@@ -968,7 +968,7 @@ struct ImBatch {
             hipMalloc((void **)&d_cand, sizeof(ImCand) * (size_t)np) != hipSuccess ||
             hipMalloc((void **)&d_items, sizeof(ImItem) * ni) != hipSuccess ||
             hipMalloc((void **)&d_cs, sizeof(double) * (size_t)np * (size_t)kmax) != hipSuccess ||
-            hipMalloc((void **)&d_part, sizeof(double) * ni * IM_STATS) != hipSuccess ||
+            hipMalloc((void **)&d_part, sizeof(double) * ni * (size_t)stride) != hipSuccess ||
             hipMalloc((void **)&d_bad, sizeof(int) * ni) != hipSuccess) {
             (void)hipGetLastError();
             return -1;
@@ -995,10 +995,10 @@ struct ImBatch {
                            hipMemcpyHostToDevice, s) != hipSuccess)
             return -1;
         (void)hipEventRecord(c->t0, s);
-        launch<IM_SCORE>(s, ni, metric, nullptr, 2);
+        launch<IM_SCORE>(s, ni, metric, nullptr, IM_SUMS);
         (void)hipEventRecord(c->t1, s);
         if (hipGetLastError() != hipSuccess) return -1;
-        h_part.resize(2 * (size_t)ni);
+        h_part.resize(IM_SUMS * (size_t)ni);
         h_bad.resize((size_t)ni);
         if (hipMemcpyAsync(h_part.data(), d_part, sizeof(double) * h_part.size(),
                            hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -1013,8 +1013,8 @@ struct ImBatch {
             double part[2] = {0.0, 0.0};
             for (int u = 0; u < cands[(size_t)cand].group && q < ni &&
                             h_items[(size_t)q].cand == cand; ++u, ++q) {
-                part[0] += h_part[2 * (size_t)q];
-                part[1] += h_part[2 * (size_t)q + 1];
+                part[0] += h_part[IM_SUMS * (size_t)q];
+                part[1] += h_part[IM_SUMS * (size_t)q + 1];
                 flags[(size_t)cand] |= h_bad[(size_t)q];
             }
             sums[2 * (size_t)cand] += part[0];
@@ -1042,7 +1042,7 @@ float rc_implicit_score_batch(void *ctx, const unsigned int *prog, const unsigne
         return -1.0f;
     if (rc_rows_ensure_f64(cx, &cx->sets[0]) != 0) return -1.0f;
     ImBatch B;
-    if (B.setup(cx, prog, off, pcount, nprog, kmax) != 0) return -1.0f;
+    if (B.setup(cx, prog, off, pcount, nprog, kmax, IM_SUMS) != 0) return -1.0f;
     std::vector<double> sums;
     std::vector<int> flags;
     if (B.score(metric, c, sums, flags) != 0) return -1.0f;
@@ -1070,7 +1070,7 @@ float rc_implicit_fit_batch(void *ctx, const unsigned int *prog, const unsigned 
         return -1.0f;
     if (rc_rows_ensure_f64(cx, &cx->sets[0]) != 0) return -1.0f;
     ImBatch B;
-    if (B.setup(cx, prog, off, pcount, nprog, kmax) != 0) return -1.0f;
+    if (B.setup(cx, prog, off, pcount, nprog, kmax, IM_STATS) != 0) return -1.0f;
     const size_t P = (size_t)nprog, KM = (size_t)kmax;
     /* Each candidate's items are consecutive in row order. */
     std::vector<int> item0(P, 0), nitem(P, 0);

@@ -14,6 +14,7 @@
 constexpr int IM_MAX_NODES = 96;
 constexpr int IM_KMAX = 20;
 constexpr int IM_STATS = (IM_KMAX + 1) * (IM_KMAX + 2) / 2; /* [J | r] lower triangle */
+constexpr int IM_SUMS = 2; /* a score's sums: weighted distances, weights */
 constexpr double IM_INV_SQRT_PI = 0.5641895835477563;
 
 enum { IM_SCORE = 0, IM_RSS = 1, IM_JAC = 2 };
