@@ -499,9 +499,15 @@ __device__ __forceinline__ bool im_fast_distance(const uint32_t *__restrict__ r4
 
 /* im_pass_kernel on the register-stack sweep for the candidates marked
    fast (the general kernel skips them, this one skips the others); NV is
-   the row set's input count. */
+   the row set's input count.  The value passes of up to two inputs fit the 168
+   registers of three waves per SIMD (one input: with 32 bytes of scratch) and
+   are held to them: scores of 9000 relations with LOG x 5000 rows 7.2 -> 5.5 ms
+   with two inputs, 7.8 -> 6.1 with one.  The others are held to two waves, the
+   Jacobian pass so that it takes the registers of two (2000 fits x 8192 rows
+   23.2 -> 22.9 ms). */
+constexpr int im_fast_waves(int mode, int nv) { return mode != IM_JAC && nv <= 2 ? 3 : 2; }
 template <int MODE, int NV>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void im_fast_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(im_fast_waves(MODE, NV)))) void im_fast_kernel(
     const ImItem *__restrict__ items, int nitems, const ImCand *__restrict__ cands,
     const uint32_t *__restrict__ rec, const double *__restrict__ cs, int kmax,
     const double *__restrict__ cols64, const double *__restrict__ w64, int n, int metric,
