@@ -41,9 +41,10 @@ __device__ __forceinline__ bool cr_row_ok(double f, double y)
    SIMD, and the interpreter's chain of dependent instructions is what they
    wait for.  Held to two waves they keep 392 bytes of scratch and are faster
    all the same, with the same bits: 128 fits x 50 021 rows 11.3 -> 9.4 ms,
-   256 x 262 144 126.7 -> 115.1 ms. */
+   256 x 262 144 126.7 -> 115.1 ms.  The record sweeps need two waves as much:
+   without the bound 32 columns take 258 registers. */
 template <int KC, bool VM>
-__global__ __launch_bounds__(64, VM ? 2 : 1) void cr_asm_kernel(
+__global__ __launch_bounds__(64, 2) void cr_asm_kernel(
     const FtItem *__restrict__ items, const int *__restrict__ list, int nlist,
     const CrCand *__restrict__ cands, FtRows Rw, const uint32_t *__restrict__ code,
     const int *__restrict__ run, const double *__restrict__ cp, double *__restrict__ pgram,
@@ -174,10 +175,11 @@ __global__ __launch_bounds__(64, VM ? 2 : 1) void cr_asm_kernel(
            16x16 block. */
         if (base + BLOCK >= sub_end || base + BLOCK >= row_end) {
             const bool add = sub_end != it.row0 + d.sub;
-            const int j = lane & 15;
+            const int at = rc_here(lane);
+            const int j = at & 15;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int i = (lane >> 4) + 4 * r;
+                const int i = (at >> 4) + 4 * r;
                 if (KC == 16 && i >= j && i < q) rc_put(pg + i * (i + 1) / 2 + j, acc00[r], add);
                 if (KC == 32) ft_pair_store<PS>(pg, i, j, q, acc00[r], acc10[r], add);
                 acc00[r] = 0.0;
@@ -213,12 +215,13 @@ __global__ __launch_bounds__(64) void cr_score_kernel(
     int bad = 0;
     dv8 U0 = (dv8)(0.0), U1 = U0, U2 = U0, U3 = U0, Bd = U0;
     const int row_end = it.row0 + it.rows;
-    double out[CR_NMOM] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    double out = 0.0; /* lane qd < CR_NMOM: the item's sum qd */
     int sub_end = it.row0 + d.sub;
     auto take = [&]() {
 #pragma unroll
         for (int qd = 0; qd < CR_NMOM; ++qd) {
-            out[qd] += rc_wave_sum_f64(mo[qd]);
+            const double sum = rc_wave_sum_f64(mo[qd]);
+            out = lane == qd ? out + sum : out;
             mo[qd] = 0.0;
         }
     };
@@ -273,11 +276,8 @@ __global__ __launch_bounds__(64) void cr_score_kernel(
     }
     if (sub_end - d.sub < row_end) take();
     const int anybad = __any(bad) ? 1 : 0;
-    if (lane == 0) {
-#pragma unroll
-        for (int qd = 0; qd < CR_NMOM; ++qd) pmom[(size_t)item * CR_NMOM + qd] = out[qd];
-        pbad[item] = anybad;
-    }
+    if (lane < CR_NMOM) pmom[(size_t)item * CR_NMOM + lane] = out;
+    if (lane == 0) pbad[item] = anybad;
 }
 
 } /* namespace */

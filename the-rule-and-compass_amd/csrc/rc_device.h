@@ -280,36 +280,43 @@ __device__ __forceinline__ RcRowFit rc_row_fit(double wb, double p, double y, in
 }
 
 /* ---- Wave-level helpers (wave64). */
+/* v of the lane with bit 32, 16, 8, 4, 2 or 1 of its number flipped, added to
+   this lane's: register moves, where __shfl_xor takes two LDS permutes. */
+template <int BIT> __device__ __forceinline__ double rc_xor_sum_f64(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned w[2] = {(unsigned)b, (unsigned)(b >> 32)};
+    unsigned x[2], y[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        x[h] = w[h];
+        if (BIT == 32 || BIT == 16) {
+            /* The two halves (rows of 16, pairwise) of v, in both halves each. */
+            const auto p = BIT == 32 ? __builtin_amdgcn_permlane32_swap(w[h], w[h], false, false)
+                                     : __builtin_amdgcn_permlane16_swap(w[h], w[h], false, false);
+            x[h] = p[0];
+            y[h] = p[1];
+        } else if (BIT == 4) {
+            const int up = __builtin_amdgcn_update_dpp(0, (int)w[h], 0x104, 0xf, 0x5, false);
+            y[h] = (unsigned)__builtin_amdgcn_update_dpp(up, (int)w[h], 0x114, 0xf, 0xa, false);
+        } else { /* row_ror:8, quad_perm 2 3 0 1, quad_perm 1 0 3 2 */
+            constexpr int ctrl = BIT == 8 ? 0x128 : BIT == 2 ? 0x4e : 0xb1;
+            y[h] = (unsigned)__builtin_amdgcn_update_dpp(0, (int)w[h], ctrl, 0xf, 0xf, true);
+        }
+    }
+    return __hiloint2double((int)x[1], (int)x[0]) + __hiloint2double((int)y[1], (int)y[0]);
+}
+/* The wave's sum in every lane, in a fixed butterfly order (independent of
+   scheduling).  All 64 lanes must be active.  Correlation scores of 16 000
+   programs x 32 768 rows, four sums a tile: 4.04 ms with LDS permutes, 3.89. */
 __device__ __forceinline__ double rc_wave_sum_f64(double v)
 {
-    /* Fixed butterfly order: the result is independent of scheduling. */
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-/* The same sum in another fixed order by DPP moves, which wait for no LDS
-   permutes: pairs, quads, eights and rows of 16, then the rows one after the
-   other (a sum that each tile of a correlation score waits for, 16 000 programs
-   x 32 768 rows: 4.04 -> 3.96 ms, 3.95 without that sum).  All 64 lanes must be
-   active. */
-template <int CTRL, int ROWS> __device__ __forceinline__ double rc_dpp_f64(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, true);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double rc_wave_sum_dpp(double v)
-{
-    v += rc_dpp_f64<0xb1, 0xf>(v);  /* quad_perm 1 0 3 2 */
-    v += rc_dpp_f64<0x4e, 0xf>(v);  /* quad_perm 2 3 0 1 */
-    v += rc_dpp_f64<0x141, 0xf>(v); /* row_half_mirror */
-    v += rc_dpp_f64<0x140, 0xf>(v); /* row_mirror */
-    v += rc_dpp_f64<0x142, 0xa>(v); /* row_bcast15 into rows 1 and 3 */
-    v += rc_dpp_f64<0x143, 0xc>(v); /* row_bcast31 into rows 2 and 3 */
-    const long long b = __double_as_longlong(v);
-    return __hiloint2double(__builtin_amdgcn_readlane((int)(b >> 32), 63),
-                            __builtin_amdgcn_readlane((int)b, 63));
+    v = rc_xor_sum_f64<32>(v);
+    v = rc_xor_sum_f64<16>(v);
+    v = rc_xor_sum_f64<8>(v);
+    v = rc_xor_sum_f64<4>(v);
+    v = rc_xor_sum_f64<2>(v);
+    return rc_xor_sum_f64<1>(v);
 }
 
 __device__ __forceinline__ int rc_wave_or(int v)
@@ -362,8 +369,36 @@ __device__ __forceinline__ double rc_grouped_sum(const double *__restrict__ p, s
     return left < group ? acc + part : acc;
 }
 
-/* A sub-tile's sum into an item's partial: the first stores, the others add. */
-__device__ __forceinline__ void rc_put(double *p, double v, bool add) { *p = add ? *p + v : v; }
+/* A sub-tile's sum into an item's partial: the first stores, the others add.
+   One lane owns an entry, so its operations on it are in order, and nothing
+   waits for the sum (9000 fits x 5000 rows, a sub-tile every two steps: 10.12 ms
+   with a load and a store, 9.97 so). */
+__device__ __forceinline__ void rc_put(double *p, double v, bool add)
+{
+    if (add) unsafeAtomicAdd(p, v);
+    else *p = v;
+}
+
+/* The same number, but not to the compiler: what is computed from it stays
+   where it stands.  Addresses that a kernel needs once in a sub-tile would
+   otherwise be computed before its row loop and held in registers through it,
+   which cost the interpreters of scratch and register stacks a wave per SIMD
+   (2000 FP64 fits x 20 000 rows 72.6 -> 48.6 ms, the same in f32 107.7 -> 105.4).
+   The 4-row VM kernels have the registers and keep the addresses (640 fits x
+   131 072 rows 14.24 ms, 14.34 so). */
+__device__ __forceinline__ int rc_here(int x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
+
+/* A wave-uniform value in scalar registers. */
+__device__ __forceinline__ double rc_scalar(double v)
+{
+    const long long b = __double_as_longlong(v);
+    return __hiloint2double(__builtin_amdgcn_readfirstlane((int)(b >> 32)),
+                            __builtin_amdgcn_readfirstlane((int)b));
+}
 
 /* p[0] | p[1] | ... | p[n - 1], n >= 0, loads issued eight at a time. */
 __device__ __forceinline__ int rc_batched_or(const int *__restrict__ p, int n)

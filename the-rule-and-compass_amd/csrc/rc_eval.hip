@@ -842,7 +842,7 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
             double first = 0.0;
 #pragma unroll
             for (int r = 0; r < R; ++r) first += ok[r] ? (double)res[r] : 0.0;
-            pivot = rc_wave_sum_dpp(first) / (double)min(64 * R, row1 - row0);
+            pivot = rc_wave_sum_f64(first) / (double)min(64 * R, row1 - row0);
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {

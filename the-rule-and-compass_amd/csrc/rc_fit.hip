@@ -474,10 +474,11 @@ __global__ __launch_bounds__(64) void ft_asm_kernel(
            register r holds D[4*(l/16) + r][l % 16] of each 16x16 block. */
         if (base + 64 >= sub_end || base + 64 >= row_end) {
             const bool add = sub_end != it.row0 + d.sub;
-            const int j = lane & 15;
+            const int at = rc_here(lane);
+            const int j = at & 15;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int i = 4 * (lane >> 4) + r;
+                const int i = 4 * (at >> 4) + r;
                 g00[r] += (double)acc00[r];
                 acc00[r] = 0.0f;
                 if (i >= j && i < K) rc_put(pg + i * (i + 1) / 2 + j, g00[r], add);
@@ -494,7 +495,7 @@ __global__ __launch_bounds__(64) void ft_asm_kernel(
                     g11[r] = 0.0;
                 }
             }
-            ltot += rc_wave_sum_f64(lsum);
+            ltot = rc_scalar(ltot + rc_wave_sum_f64(lsum));
             lsum = 0.0;
             sub_end += d.sub;
         }
@@ -515,8 +516,11 @@ __global__ __launch_bounds__(64) void ft_asm_kernel(
    on FP64 MFMA (v_mfma_f64_16x16x4f64), accumulated in f64.  A row is usable
    when its f64 prediction and residual are finite. */
 constexpr int XS64 = 68; /* f64 column stride: 64 rows + 4 */
+/* 16 columns over the scratch stores take 257 registers: held to the 256 of two
+   waves per SIMD (2000 fits x 20 000 rows, one wave 72.6 ms). */
+constexpr int ft_asm64_waves(int kc, bool big) { return big && kc == 16 ? 2 : 1; }
 template <int KC, bool BIG, bool POLISH>
-__global__ __launch_bounds__(64) void ft_asm64_kernel(
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(ft_asm64_waves(KC, BIG)))) void ft_asm64_kernel(
     const FtItem *__restrict__ items, const int *__restrict__ list, int nlist,
     const FtCand *__restrict__ cands, const FtRows *__restrict__ rowsd,
     const uint32_t *__restrict__ code, const int *__restrict__ run,
@@ -599,10 +603,11 @@ __global__ __launch_bounds__(64) void ft_asm64_kernel(
            output: lane l, register r holds D[l/16 + 4 r][l % 16]. */
         if (base + 64 >= sub_end || base + 64 >= row_end) {
             const bool add = sub_end != it.row0 + d.sub;
-            const int j = lane & 15;
+            const int at = rc_here(lane);
+            const int j = at & 15;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int i = (lane >> 4) + 4 * r;
+                const int i = (at >> 4) + 4 * r;
                 if (i >= j && i < K) rc_put(pg + i * (i + 1) / 2 + j, acc00[r], add);
                 acc00[r] = 0.0;
                 if (KC == 32) {
@@ -613,7 +618,7 @@ __global__ __launch_bounds__(64) void ft_asm64_kernel(
                     acc11[r] = 0.0;
                 }
             }
-            ltot += rc_wave_sum_f64(lsum);
+            ltot = rc_scalar(ltot + rc_wave_sum_f64(lsum));
             lsum = 0.0;
             sub_end += d.sub;
         }
@@ -681,12 +686,12 @@ __global__ __launch_bounds__(64) void ft_trial_kernel(
             lsum += hard ? 1e30 : wb * rc_row_stat((double)pred[r], yr, d.metric);
         }
         if (base + 64 * R >= sub_end) {
-            ltot += rc_wave_sum_f64(lsum);
+            ltot = rc_scalar(ltot + rc_wave_sum_f64(lsum));
             lsum = 0.0;
             sub_end += d.sub;
         }
     }
-    if (sub_end - d.sub < row_end) ltot += rc_wave_sum_f64(lsum);
+    if (sub_end - d.sub < row_end) ltot = rc_scalar(ltot + rc_wave_sum_f64(lsum));
     if (lane == 0) ploss[item] = ltot;
 }
 

@@ -321,7 +321,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(PM != 0 ? 2 
                 g00[r] = 0.0;
                 if (KC == 32) g10[r] = 0.0;
             }
-            ltot += rc_wave_sum_f64(lsum);
+            ltot = rc_scalar(ltot + rc_wave_sum_f64(lsum));
             lsum = 0.0;
             sub_end += d.sub;
         }
@@ -478,16 +478,17 @@ __global__ __launch_bounds__(64, 2) void vm_asm64_kernel(
            16x16 block (not the FP32 form's 4 (l/16) + r). */
         if (base + BLOCK >= sub_end || base + BLOCK >= row_end) {
             const bool add = sub_end != it.row0 + d.sub;
-            const int j = lane & 15;
+            const int at = rc_here(lane);
+            const int j = at & 15;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int i = (lane >> 4) + 4 * r;
+                const int i = (at >> 4) + 4 * r;
                 if (KC == 16 && i >= j && i < K) rc_put(pg + i * (i + 1) / 2 + j, acc00[r], add);
                 if (KC == 32) ft_pair_store<6>(pg, i, j, K, acc00[r], acc10[r], add);
                 acc00[r] = 0.0;
                 if (KC == 32) acc10[r] = 0.0;
             }
-            ltot += rc_wave_sum_f64(lsum);
+            ltot = rc_scalar(ltot + rc_wave_sum_f64(lsum));
             lsum = 0.0;
             sub_end += d.sub;
         }
@@ -596,12 +597,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void vm
             }
         }
         if (base + 64 * RR >= sub_end) {
-            ltot += rc_wave_sum_f64(lsum);
+            ltot = rc_scalar(ltot + rc_wave_sum_f64(lsum));
             lsum = 0.0;
             sub_end += d.sub;
         }
     }
-    if (sub_end - d.sub < row_end) ltot += rc_wave_sum_f64(lsum);
+    if (sub_end - d.sub < row_end) ltot = rc_scalar(ltot + rc_wave_sum_f64(lsum));
     if (lane == 0) ploss[item] = ltot;
 }
 

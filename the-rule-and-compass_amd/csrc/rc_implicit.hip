@@ -278,15 +278,16 @@ __global__ __launch_bounds__(64) void im_pass_kernel(
         /* The end of a sub-tile: its sums go onto the item's. */
         if (base + 64 >= sub_end || base + 64 >= row_end) {
             const bool add = sub_end != it.row0 + d.sub;
+            const int at = rc_here(lane);
             if (MODE == IM_JAC) {
                 for (int q = 0; q < 4; ++q) {
-                    const int s = lane + 64 * q;
+                    const int s = at + 64 * q;
                     if (s < nstats) rc_put(p + s, acc[q], add);
                     acc[q] = 0.0;
                 }
             } else {
-                t0 += rc_wave_sum_f64(s0);
-                t1 += rc_wave_sum_f64(s1);
+                t0 = rc_scalar(t0 + rc_wave_sum_f64(s0));
+                t1 = rc_scalar(t1 + rc_wave_sum_f64(s1));
                 s0 = s1 = 0.0;
             }
             sub_end += d.sub;
@@ -632,8 +633,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(im_fast_wave
                     acc00[r] = acc10[r] = acc11[r] = 0.0;
                 }
             } else {
-                t0 += rc_wave_sum_f64(s0);
-                t1 += rc_wave_sum_f64(s1);
+                t0 = rc_scalar(t0 + rc_wave_sum_f64(s0));
+                t1 = rc_scalar(t1 + rc_wave_sum_f64(s1));
                 s0 = s1 = 0.0;
             }
             sub_end += d.sub;

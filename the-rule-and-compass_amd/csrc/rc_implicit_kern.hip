@@ -315,19 +315,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void im
            im_fast_kernel). */
         if (base + ROWS >= sub_end || base + ROWS >= row_end) {
             const bool add = sub_end != it.row0 + d.sub;
+            /* rc_here: 640 Jacobian fits x 131 072 rows of two inputs 114.4 ->
+               112.8 ms; three inputs keep 112 bytes of scratch less but take
+               133.2 ms for 130.4. */
+            const int at = NV < 3 ? rc_here(lane) : lane;
             if (MODE == IM_JAC) {
-                const int jj = lane & 15;
+                const int jj = at & 15;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int ii = (lane >> 4) + 4 * r, i1 = 16 + ii;
+                    const int ii = (at >> 4) + 4 * r, i1 = 16 + ii;
                     if (ii >= jj && ii < K1) rc_put(p + ii * (ii + 1) / 2 + jj, acc00[r], add);
                     if (i1 < K1) rc_put(p + i1 * (i1 + 1) / 2 + jj, acc10[r], add);
                     if (ii >= jj && i1 < K1) rc_put(p + i1 * (i1 + 1) / 2 + 16 + jj, acc11[r], add);
                     acc00[r] = acc10[r] = acc11[r] = 0.0;
                 }
             } else {
-                t0 += rc_wave_sum_f64(s0);
-                t1 += rc_wave_sum_f64(s1);
+                t0 = rc_scalar(t0 + rc_wave_sum_f64(s0));
+                t1 = rc_scalar(t1 + rc_wave_sum_f64(s1));
                 s0 = s1 = 0.0;
             }
             sub_end += d.sub;
