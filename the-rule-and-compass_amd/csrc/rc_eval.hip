@@ -59,6 +59,10 @@ constexpr uint32_t RC_OP_FUSED = 64;
 
 constexpr int MODE_EVAL = 0;    /* sum of rho with 1e30 hard failures (rc_eval) */
 constexpr int MODE_SCORE = 1;   /* f64 score objectives + bad flag */
+constexpr int MODE_CORR = 3;    /* the correlation scores, a kernel of their own:
+                                   their moments cost the others the 128 registers
+                                   of four waves per SIMD (4096 programs of 9 to 13
+                                   stack entries x 32 768 rows 3.83 -> 3.23 ms) */
 constexpr int MODE_PREDICT = 2; /* raw predictions */
 
 bool is_binary_op(uint32_t op)
@@ -626,6 +630,10 @@ struct RcScoreArgs {
     double ybar;
     double *part2;
 };
+__host__ __device__ __forceinline__ bool rc_score_is_corr(int kind)
+{
+    return kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED;
+}
 /* A tile's mean prediction, its sum of (pred - mean) (y - ybar) and its sum of
    y - ybar; the sum of (pred - mean)^2 is the item's partial itself. */
 constexpr int RC_CORR_SUMS = 3;
@@ -809,8 +817,7 @@ __global__ __launch_bounds__(64) void rc_eval_kernel(
     const int row1 = min(n, row0 + tile_rows);
     double acc = 0.0, acc2 = 0.0;
     int bad = 0;
-    const bool corr = MODE == MODE_SCORE &&
-                      (kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED);
+    constexpr bool corr = MODE == MODE_CORR;
     const bool classif = MODE == MODE_SCORE && kind >= RC_SCORE_LOG_LOSS &&
                          kind <= RC_SCORE_HINGE_SQUARED;
     /* The correlation scores need the moments about the mean (two passes in
@@ -987,8 +994,7 @@ __global__ void rc_eval_finish(const double *__restrict__ part, const int *__res
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= nprog) return;
-    const bool corr = mode == MODE_SCORE &&
-                      (kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED);
+    const bool corr = mode == MODE_SCORE && rc_score_is_corr(kind);
     const bool classif =
         mode == MODE_SCORE && kind >= RC_SCORE_LOG_LOSS && kind <= RC_SCORE_HINGE_SQUARED;
     double s = 0.0, s2 = 0.0, pbar = 0.0;
@@ -1098,6 +1104,10 @@ void launch_class(int mode, dim3 grid, hipStream_t s, const RcCtx *c, const uint
         rc_eval_kernel<S, R, MODE_EVAL><<<grid, 64, 0, s>>>(
             r->cols, c->d_derived, r->v, r->y, r->n, code, meta, plist, ncls, tiles, tile_rows, kind,
             part, part_bad, pred, sa);
+    else if (mode == MODE_SCORE && rc_score_is_corr(kind))
+        rc_eval_kernel<S, R, MODE_CORR><<<grid, 64, 0, s>>>(
+            r->cols, c->d_derived, r->v, r->y, r->n, code, meta, plist, ncls, tiles, tile_rows, kind,
+            part, part_bad, pred, sa);
     else if (mode == MODE_SCORE)
         rc_eval_kernel<S, R, MODE_SCORE><<<grid, 64, 0, s>>>(
             r->cols, c->d_derived, r->v, r->y, r->n, code, meta, plist, ncls, tiles, tile_rows, kind,
@@ -1147,8 +1157,7 @@ int launch_rows(RcCtx *c, int mode, int kind, int nprog, const uint32_t *code,
     RcRows *r = &c->sets[0];
     const int n = r->n;
     if (n <= 0) return -1;
-    const bool corr = mode == MODE_SCORE &&
-                      (kind == RC_SCORE_CORRELATION || kind == RC_SCORE_CORRELATION_SIGNED);
+    const bool corr = mode == MODE_SCORE && rc_score_is_corr(kind);
     int tile_rows = tile_rows_for(n, c->tune_eval_tile);
     if (corr) tile_rows = std::min(tile_rows, RC_CORR_TILE);
     const int tiles = (n + tile_rows - 1) / tile_rows;
