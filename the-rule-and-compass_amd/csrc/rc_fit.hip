@@ -60,7 +60,7 @@ constexpr int FT_TOLD = 4;
 enum {
     ST_NEED_ASM = 1, ST_NEED_TRIAL = 2, ST_LM_DONE = 3, ST_P_NEED_ASM = 4, ST_P_NEED_TRIAL = 5,
     ST_DONE = 6,
-    ST_KNOWN = 7 /* an LM trial that is rejected without its pass (told_rejected) */
+    ST_KNOWN = 7 /* an LM trial that is rejected without its pass (told_has) */
 };
 
 /* Control operations. */
@@ -82,13 +82,20 @@ struct FtState {
     int halvings, polish_it, pre_status, acc_bits; /* acc_bits: LM decision q accepted (bit q) */
     int n_asm, n_trial, n_exact, n_decided; /* passes consumed, LM decisions (telemetry) */
     int pruned; /* this LM trial was rejected on its first half (ft_trial_prune) */
-    int ntold;  /* entries of told that hold a vector, and the next to take */
+    int ntold;  /* vectors of FtTold in use, and the next to take */
     int told_at;
-    /* f32 constants (bits) whose loss is known not to be below `best`: those
-       `best` was measured at and trials rejected since (told_rejected). */
-    unsigned told[FT_TOLD][FT_KMAX];
 };
 static_assert(sizeof(FtState) % 16 == 0, "FtState is copied in 16-byte words");
+
+/* f32 constants (bits) whose loss is known not to be below `best`: those `best`
+   was measured at and trials rejected since (told_has), k words each.
+   Beside the state, which every control step reads and writes whole: the LM
+   steps read these and write the one vector that is told (9000 candidates, a
+   launch: 24.5 us without them, 26.4 in the state, 25.6 so). */
+struct FtTold {
+    unsigned v[FT_TOLD * FT_KMAX];
+};
+constexpr int FT_TOLD_WORDS = (FT_TOLD * FT_KMAX + 63) / 64; /* of a lane */
 
 /* Wave-uniform storage for the interpreter: an LLVM vector (registers,
    indexed through s_set_gpr_idx) for the common sizes, a plain array for the
@@ -732,6 +739,27 @@ __global__ __launch_bounds__(64) void ft_probe_kernel(const FtCand *__restrict__
 
 __device__ __forceinline__ double clamp_step(double t) { return fmin(1e6, fmax(-1e6, t)); }
 
+/* An LM trial's loss is a function of its f32 constants alone: the same rows,
+   stream, items and order of sums.  Near the optimum the solves at growing
+   lambda keep giving the step that was just rejected, or none that f32 can
+   see, so most trials there would measure a loss that is known: that of the
+   constants `best` was measured at, or of a trial rejected since.  Such a
+   trial is rejected without its pass (1024 fits x 262 144 rows: 198 -> 182 ms). */
+__device__ __forceinline__ unsigned told_bits(double c) { return __float_as_uint((float)c); }
+/* Whether one of the first nt vectors is the one whose constant lane & 31 has
+   the bits t in each lane (any for the lanes past k): two vectors at a time. */
+__device__ __forceinline__ bool told_has(const FtTold &told, int nt, int k, unsigned t, int lane)
+{
+    const int j = lane & 31;
+    bool has = false;
+    for (int q0 = 0; q0 < nt; q0 += 2) {
+        const int q = q0 + (lane >> 5);
+        const unsigned long long ne = __ballot(q >= nt || (j < k && told.v[q * k + j] != t));
+        has = has || (unsigned)ne == 0u || (unsigned)(ne >> 32) == 0u;
+    }
+    return has;
+}
+
 /* A solve the serial control step leaves to the whole wave: the LM step at
    the cached normal equations or the polish's Gauss-Newton step. */
 enum { CT_SOLVE_NONE = 0, CT_SOLVE_LM = 1, CT_SOLVE_POLISH = 2 };
@@ -742,9 +770,9 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
                                        const double *G, double sh_loss, int sh_bad, int sh_skip,
                                        int ran_trial, bool want_gram, double &solve_lambda,
                                        double *__restrict__ outc, double *__restrict__ outsse,
-                                       int *__restrict__ outstatus, int all64);
+                                       int *__restrict__ outstatus, int all64, unsigned halved);
 __device__ __forceinline__ void ctrl_after_solve(int kind, int rc, int cand, FtState *s, int k,
-                                              const double *delta, bool known,
+                                              const double *delta, unsigned known,
                                               float *__restrict__ cp32, double *__restrict__ cp64,
                                               int all64);
 __device__ __forceinline__ void ctrl_flags(int op, int cand, const FtState *s,
@@ -756,12 +784,16 @@ __global__ __launch_bounds__(64) void ft_ctrl_kernel(
     float *__restrict__ cp32, double *__restrict__ cp64, const double *__restrict__ pgram,
     int tri_stride, const double *__restrict__ ploss, const int *__restrict__ pbad,
     const int *__restrict__ pskip, double *__restrict__ outc, double *__restrict__ outsse,
-    int *__restrict__ outstatus, int all64)
+    int *__restrict__ outstatus, int all64, unsigned *__restrict__ told)
 {
     const int cand = blockIdx.x;
     if (cand >= ncand) return;
     const int lane = threadIdx.x;
     const FtCand d = cands[cand];
+    const int k = d.k;
+    __shared__ FtTold sT;
+    unsigned *gT = told + (size_t)cand * (FT_TOLD * FT_KMAX);
+    const bool lm_step = !all64 && (op == CT_AFTER_ASM || op == CT_AFTER_TRIAL);
     __shared__ double G[FT_TRI_MAX];
     __shared__ double L[FT_KMAX * FT_KMAX];
     __shared__ double sh_loss;
@@ -780,15 +812,25 @@ __global__ __launch_bounds__(64) void ft_ctrl_kernel(
         int4 v[SU];
 #pragma unroll
         for (int u = 0; u < SU; ++u) v[u] = src[min(lane + 64 * u, SW - 1)];
+        unsigned t[FT_TOLD_WORDS];
+        if (lm_step) {
+#pragma unroll
+            for (int u = 0; u < FT_TOLD_WORDS; ++u)
+                t[u] = gT[min(lane + 64 * u, FT_TOLD * FT_KMAX - 1)];
+        }
 #pragma unroll
         for (int u = 0; u < SU; ++u) dst[min(lane + 64 * u, SW - 1)] = v[u];
+        if (lm_step) {
+#pragma unroll
+            for (int u = 0; u < FT_TOLD_WORDS; ++u)
+                sT.v[min(lane + 64 * u, FT_TOLD * FT_KMAX - 1)] = t[u];
+        }
     }
     __syncthreads();
     FtState *s = &sS;
 
     const int ran_asm = run_asm[cand];
     const int ran_trial = run_trial[cand];
-    const int k = d.k;
     const int K = k + 2;
     const int tri = K * (K + 1) / 2;
 
@@ -834,10 +876,32 @@ __global__ __launch_bounds__(64) void ft_ctrl_kernel(
     __shared__ double sh_lambda;
     __shared__ double sh_delta[FT_KMAX], sh_dsc[FT_KMAX], sh_rhs[FT_KMAX];
     __syncthreads();
+    /* A measured LM trial is told, by the wave, and whether the steps that
+       halving it would try are. */
+    const int tj = min(lane & 31, k - 1); /* a constant a lane; no lane's where k = 0 */
+    unsigned halved = 0u;
+    if (lm_step && op == CT_AFTER_TRIAL && ran_trial && s->stage == ST_NEED_TRIAL && k > 0) {
+        const double tsse = s->pruned ? __builtin_inf() : sh_loss;
+        const bool better = tsse < s->best;
+        double t = s->trial[tj];
+        const int q = better ? 0 : s->told_at;
+        if (lane < k) {
+            sT.v[q * k + lane] = told_bits(t);
+            gT[q * k + lane] = told_bits(t);
+        }
+        __syncthreads();
+        if (!better && s->halvings > 0) {
+            const int nt = min(s->ntold + 1, FT_TOLD);
+            for (int h = 0; h < 2; ++h) {
+                t = s->c[tj] + 0.5 * (t - s->c[tj]);
+                halved |= told_has(sT, nt, k, told_bits(t), lane) ? 1u << h : 0u;
+            }
+        }
+    }
     if (lane == 0) {
         double lam = 0.0;
         sh_solve = ctrl_lane0(op, cand, s, d, c0, kmax, cp32, cp64, G, sh_loss, sh_bad, sh_skip,
-                              ran_trial, want_gram, lam, outc, outsse, outstatus, all64);
+                              ran_trial, want_gram, lam, outc, outsse, outstatus, all64, halved);
         sh_lambda = lam;
     }
     __syncthreads();
@@ -845,18 +909,14 @@ __global__ __launch_bounds__(64) void ft_ctrl_kernel(
     if (solve != CT_SOLVE_NONE) {
         const int rc = ft_solve_wave(s->jtj, s->jtr, sh_lambda, k, sh_delta, L, sh_dsc, sh_rhs,
                                      lane);
-        /* Whether the step's constants are told, by the wave: two vectors at a
-           time, a constant a lane. */
-        bool known = false;
-        if (solve == CT_SOLVE_LM && s->ntold > 0) {
-            const int j = lane & 31;
-            const unsigned t =
-                j < k ? __float_as_uint((float)clamp_step(s->c[j] + sh_delta[j])) : 0u;
-            for (int q0 = 0; q0 < s->ntold; q0 += 2) {
-                const int q = q0 + (lane >> 5);
-                const unsigned long long ne =
-                    __ballot(q >= s->ntold || (j < k && s->told[q][j] != t));
-                known = known || (unsigned)ne == 0u || (unsigned)(ne >> 32) == 0u;
+        /* Whether the step's constants are told (bit 0), and those of the
+           steps that halve it. */
+        unsigned known = 0u;
+        if (solve == CT_SOLVE_LM && lm_step && s->ntold > 0 && k > 0) {
+            double t = clamp_step(s->c[tj] + sh_delta[tj]);
+            for (int h = 0; h < (s->irls ? 3 : 1); ++h) {
+                known |= told_has(sT, s->ntold, k, told_bits(t), lane) ? 1u << h : 0u;
+                t = s->c[tj] + 0.5 * (t - s->c[tj]);
             }
         }
         if (lane == 0) ctrl_after_solve(solve, rc, cand, s, k, sh_delta, known, cp32, cp64, all64);
@@ -881,29 +941,6 @@ __device__ __forceinline__ void ctrl_set_pass64(double *__restrict__ cp64, int c
                                              const double *v)
 {
     for (int j = 0; j < FT_KMAX; ++j) cp64[(size_t)cand * FT_KMAX + j] = j < k ? v[j] : 0.0;
-}
-
-/* An LM trial's loss is a function of its f32 constants alone: the same rows,
-   stream, items and order of sums.  Near the optimum the solves at growing
-   lambda keep giving the step that was just rejected, or none that f32 can
-   see, so most trials there would measure a loss that is known: that of the
-   constants `best` was measured at, or of a trial rejected since.  Such a
-   trial is rejected without its pass (1024 fits x 262 144 rows: 198 -> 182 ms). */
-__device__ __forceinline__ bool told_rejected(const FtState *s, int k)
-{
-    for (int q = 0; q < s->ntold; ++q) {
-        bool same = true;
-        for (int j = 0; j < k; ++j)
-            same = same && s->told[q][j] == __float_as_uint((float)s->trial[j]);
-        if (same) return true;
-    }
-    return false;
-}
-__device__ __forceinline__ void tell(FtState *s, int k)
-{
-    for (int j = 0; j < k; ++j) s->told[s->told_at][j] = __float_as_uint((float)s->trial[j]);
-    s->told_at = (s->told_at + 1) % FT_TOLD;
-    if (s->ntold < FT_TOLD) s->ntold += 1;
 }
 
 /* The end of an LM iteration's inner loop (count or break): the next IRLS
@@ -937,7 +974,7 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
                                        const double *G, double sh_loss, int sh_bad, int sh_skip,
                                        int ran_trial, bool want_gram, double &solve_lambda,
                                        double *__restrict__ outc, double *__restrict__ outsse,
-                                       int *__restrict__ outstatus, int all64)
+                                       int *__restrict__ outstatus, int all64, unsigned halved)
 {
     const int k = d.k;
     double *cc = s->c;
@@ -1038,15 +1075,21 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
             const double tsse = s->pruned ? __builtin_inf() : sh_loss;
             s->pruned = 0;
             if (tsse < s->best) s->ntold = s->told_at = 0; /* a new best */
-            if (!all64) tell(s, k);
+            if (!all64) { /* the trial was told */
+                s->told_at = (s->told_at + 1) % FT_TOLD;
+                if (s->ntold < FT_TOLD) s->ntold += 1;
+            }
             if (!(tsse < s->best) && s->halvings > 0) {
                 /* True-metric Armijo halving for the L1 arm (eval.cu:2496-2509),
                    past the halved steps known to be rejected. */
+                bool known;
                 do {
                     s->halvings -= 1;
                     for (int j = 0; j < k; ++j) s->trial[j] = cc[j] + 0.5 * (s->trial[j] - cc[j]);
-                } while (s->halvings > 0 && told_rejected(s, k));
-                if (!told_rejected(s, k)) {
+                    known = (halved & 1u) != 0u;
+                    halved >>= 1;
+                } while (s->halvings > 0 && known);
+                if (!known) {
                     set_pass32(s->trial);
                     break;
                 }
@@ -1147,7 +1190,7 @@ __device__ __forceinline__ int ctrl_lane0(int op, int cand, FtState *s, const Ft
    the current constants; known: its constants are told), or record the failed
    solve. */
 __device__ __forceinline__ void ctrl_after_solve(int kind, int rc, int cand, FtState *s, int k,
-                                              const double *delta, bool known,
+                                              const double *delta, unsigned known,
                                               float *__restrict__ cp32, double *__restrict__ cp64,
                                               int all64)
 {
@@ -1164,13 +1207,13 @@ __device__ __forceinline__ void ctrl_after_solve(int kind, int rc, int cand, FtS
     for (int j = 0; j < k; ++j) s->trial[j] = clamp_step(s->c[j] + delta[j]);
     if (kind == CT_SOLVE_LM) {
         s->halvings = s->irls ? 2 : 0;
-        while (known && s->halvings > 0) {
+        while ((known & 1u) && s->halvings > 0) {
             s->halvings -= 1;
             for (int j = 0; j < k; ++j) s->trial[j] = s->c[j] + 0.5 * (s->trial[j] - s->c[j]);
-            known = told_rejected(s, k);
+            known >>= 1;
         }
-        s->stage = known ? ST_KNOWN : ST_NEED_TRIAL;
-        if (known) return;
+        s->stage = (known & 1u) ? ST_KNOWN : ST_NEED_TRIAL;
+        if (known & 1u) return;
         if (all64) ctrl_set_pass64(cp64, cand, k, s->trial);
         else ctrl_set_pass32(cp32, cand, k, s->trial);
     } else {
@@ -1430,7 +1473,7 @@ static size_t take(size_t &cur, size_t bytes)
 struct FtRegion {
     size_t o_code, o_cand, o_rows, o_items, o_lists, o_pre, o_c0, in_end;
     size_t o_outc, o_sse, o_st, io_end;
-    size_t o_state, o_run_a, o_run_t, o_run_b, o_cp32, o_cp64, o_pgram, o_ploss, o_pbad, o_pskip,
+    size_t o_state, o_told, o_run_a, o_run_t, o_run_b, o_cp32, o_cp64, o_pgram, o_ploss, o_pbad, o_pskip,
         o_p64, dev_end;
 };
 static const int FT_REGION_FIELDS = (int)(sizeof(FtRegion) / sizeof(size_t));
@@ -1455,6 +1498,7 @@ static FtRegion ft_region(size_t code_words, size_t ncands, size_t nrowsets, siz
     g.o_st = take(cur, np * 4);
     g.io_end = take(cur, 0);
     g.o_state = take(cur, np * sizeof(FtState));
+    g.o_told = take(cur, np * FT_TOLD * FT_KMAX * 4);
     g.o_run_a = take(cur, np * 4);
     g.o_run_t = take(cur, np * 4);
     g.o_run_b = take(cur, np * 4);
@@ -1876,7 +1920,8 @@ static float fit_run(RcCtx *c, const uint32_t *prog, const uint32_t *off, const 
     auto ctrl0 = [&](int op) {
         ft_ctrl_kernel<<<nprog, 64, 0, s>>>(op, nprog, d_state, d_cand, d_c0, kmax, d_run_a, d_run_t,
                                             d_cp32, d_cp64, d_pgram, tri_stride, d_ploss, d_pbad,
-                                            d_pskip, d_outc, d_sse, d_st, all64 ? 1 : 0);
+                                            d_pskip, d_outc, d_sse, d_st, all64 ? 1 : 0,
+                                            (unsigned *)(D + rg.o_told));
     };
     auto ctrl = [&](int op) { mark(3, [&]() { ctrl0(op); }); };
     /* The classes of a pass write disjoint items, so their kernels may run side
