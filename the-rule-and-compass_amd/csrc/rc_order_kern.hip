@@ -244,15 +244,17 @@ __device__ __forceinline__ OrDual or_dual(const uint32_t *__restrict__ rec, int 
         if (ft_is_binary(op)) {
             --sp;
             const double av[2] = {S0[sp], S1[sp]}, at[2] = {S0[sp + 8], S1[sp + 8]};
+            const int left = at[0] != 0.0 || at[1] != 0.0; /* the path's side */
             if (op == OP_MUL) {
                 t.ev = 0;
+                if (left || t.t[0] != 0.0 || t.t[1] != 0.0) {
 #pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    t.t[r] = or_tan(t.v[r], at[r], r, t.ev) + or_tan(av[r], t.t[r], r, t.ev);
-                    t.v[r] = av[r] * t.v[r];
+                    for (int r = 0; r < 2; ++r)
+                        t.t[r] = or_tan(left ? t.v[r] : av[r], left ? at[r] : t.t[r], r, t.ev);
                 }
+#pragma unroll
+                for (int r = 0; r < 2; ++r) t.v[r] = av[r] * t.v[r];
             } else {
-                const int left = at[0] != 0.0 || at[1] != 0.0;
                 t = or_divide_or_pow(op, av[0], av[1], t.v[0], t.v[1], left ? at[0] : t.t[0],
                                      left ? at[1] : t.t[1], left);
             }
