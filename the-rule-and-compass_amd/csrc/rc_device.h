@@ -297,11 +297,12 @@ template <int BIT> __device__ __forceinline__ double rc_xor_sum_f64(double v)
             x[h] = p[0];
             y[h] = p[1];
         } else if (BIT == 4) {
-            const int up = __builtin_amdgcn_update_dpp(0, (int)w[h], 0x104, 0xf, 0x5, false);
+            const int up =
+                __builtin_amdgcn_update_dpp((int)w[h], (int)w[h], 0x104, 0xf, 0x5, false);
             y[h] = (unsigned)__builtin_amdgcn_update_dpp(up, (int)w[h], 0x114, 0xf, 0xa, false);
         } else { /* row_ror:8, quad_perm 2 3 0 1, quad_perm 1 0 3 2 */
             constexpr int ctrl = BIT == 8 ? 0x128 : BIT == 2 ? 0x4e : 0xb1;
-            y[h] = (unsigned)__builtin_amdgcn_update_dpp(0, (int)w[h], ctrl, 0xf, 0xf, true);
+            y[h] = (unsigned)__builtin_amdgcn_update_dpp((int)w[h], (int)w[h], ctrl, 0xf, 0xf, true);
         }
     }
     return __hiloint2double((int)x[1], (int)x[0]) + __hiloint2double((int)y[1], (int)y[0]);
