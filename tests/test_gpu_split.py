@@ -8,8 +8,9 @@ import numpy as np
 import pytest
 import torch
 
-from rcsr_hip import host
-from rcsr_hip.expr import ADD, COS, MUL, SIN, SQUARE, SUB, const, node, var
+from rcsr_hip import host, workloads
+from rcsr_hip.expr import ADD, COS, LOG, MUL, SIN, SQUARE, SUB, const, node, var
+from test_gpu_fit_tape import _basis, _tree
 
 pytestmark = pytest.mark.gpu
 
@@ -77,6 +78,78 @@ def test_implicit_scores_do_not_depend_on_the_batch(n):
     full, sf, mf = ev.implicit_score_batch(plans * 4200)
     assert ms >= 0 and mf >= 0 and not st.any() and not sf.any()
     assert np.all(full == alone[0])
+    ev.close()
+
+
+def _nested(levels):
+    """A right-deep tree over two inputs: it keeps `levels` values below its top."""
+    t = node(MUL, const(0.5), var(0))
+    for i in range(levels):
+        t = node(ADD if i % 2 else SUB, node(MUL, const(0.1 * (i + 1)), _basis(i, 2)), t)
+    return t
+
+
+# One program for every assembly kernel and value pass: 4-row streams with the
+# tape in U, B and LDS (and their 2-row or general kernels with 2 rows per lane),
+# 16 and 32 columns, and two programs outside the fit VM, of a small and of a
+# large evaluation stack.
+KERNELS = {"16 columns": FIT[0],
+           "32 columns": workloads.structured_candidate(workloads.rng_for(3), 2, 18), "tape in B": _tree(16, 2, 0),
+           "tape in LDS": _tree(20, 2, 2), "small stack": _nested(8), "large stack": _nested(11)}
+
+
+@pytest.mark.parametrize("rows", [4, 2])
+@pytest.mark.parametrize("metric", [0, 4])
+@pytest.mark.parametrize("n", [8193, 20001])
+def test_sub_tiles_and_whole_groups_of_every_kernel(n, metric, rows):
+    """An item size of 8192 rows set by hand makes one item of each group: the
+    kernels add its sub-tiles themselves."""
+    ev = _evaluator(n)
+    plans = [host.gpu_fit_plan(t) for t in KERNELS.values()]
+    assert ev.set_tuning(host.TUNE_FIT_ROWS_PER_LANE, rows) == 0
+    for mode in (host.FIT_MODE_MIXED, host.FIT_MODE_FP64) if metric == 0 else (host.FIT_MODE_MIXED,):
+        ev.set_fit_mode(mode)
+        print(f"split: {n} rows, metric {metric}, {rows} rows a lane, mode {mode}", flush=True)
+        ev.set_tuning(host.TUNE_FIT_TILE_ROWS, 0)
+        small, ms = ev.fit_batch(plans, 5, metric)
+        assert ms >= 0 and all(np.isfinite(o.sse) for o in small)
+        ev.set_tuning(host.TUNE_FIT_TILE_ROWS, 8192)
+        whole, ms = ev.fit_batch(plans, 5, metric)
+        assert ms >= 0
+        _same(whole, small)
+    ev.close()
+
+
+@pytest.mark.parametrize("n", [8193, 20001])
+def test_sub_tiles_and_whole_groups_of_the_correlation_kernels(n):
+    ev = _evaluator(n)
+    trees = [SHAPE[0], KERNELS["32 columns"], _nested(8), _nested(15)]
+    plans = [host.gpu_fit_plan(t) for t in trees]
+    small, ms = ev.fit_batch(plans, 5, 2)
+    assert ms >= 0
+    ev.set_tuning(host.TUNE_FIT_TILE_ROWS, 8192)
+    whole, ms = ev.fit_batch(plans, 5, 2)
+    assert ms >= 0
+    _same(whole, small)
+    ev.close()
+
+
+# Relations for the sweeps beside the four-wide one: a guarded operator, and a
+# stack beyond the register sweep's.
+@pytest.mark.parametrize("n,copies", [(700, 8400), (8193, 4200)])
+def test_implicit_relations_of_every_sweep(n, copies):
+    trees = [node(SUB, node(ADD, node(SQUARE, var(0)), node(MUL, const(0.9), node(SQUARE, var(1)))),
+                  node(SUB, const(1.1), node(LOG, node(ADD, const(3.0), var(0))))),
+             node(ADD, _nested(10), node(SUB, node(SQUARE, var(1)), const(0.6)))]
+    ev = _evaluator(n)
+    plans = [host.gpu_fit_plan(t) for t in trees]
+    print(f"split: implicit sweeps, {n} rows, {copies} copies", flush=True)
+    alone, ms = ev.implicit_fit_batch(plans, 1)
+    assert ms >= 0
+    full, ms = ev.implicit_fit_batch(plans * (copies // len(plans)), 1)
+    assert ms >= 0
+    _same(full[:len(plans)], alone)
+    _same(full[-len(plans):], alone)
     ev.close()
 
 
