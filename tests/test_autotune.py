@@ -4,6 +4,7 @@ function of the shapes."""
 import math
 
 import numpy as np
+import pytest
 
 from rcsr_hip import autotune as at
 from rcsr_hip.host import TUNE_EVAL_TILE_ROWS, TUNE_FIT_ROWS_PER_LANE, TUNE_FIT_TILE_ROWS
@@ -153,3 +154,55 @@ def test_tune_fit_confirms_a_sample_winner_on_the_whole_batch():
         conf = {s[TUNE_FIT_TILE_ROWS]: ms for s, ms in res.confirm_table}
         assert conf == {8192: 40.0, 4096: 44.0 if full_prefers_builtin else 36.0}
         assert len(res.to_json()["confirm_table"]) == 2
+
+
+# The built-in choice (setting 0) follows the batch: its cost differs from that
+# of every size set by hand, also of those it is made of.
+def _adaptive(cost0, explicit):
+    def cost(t):
+        tile = t[TUNE_FIT_TILE_ROWS]
+        base = cost0 if tile == 0 else explicit.get(tile, 30.0)
+        return base * (1.5 if t[TUNE_FIT_ROWS_PER_LANE] == 2 else 1.0)
+    return cost
+
+
+def _tuned(cost, rows, **kw):
+    ev = FakeEv(cost)
+    ev.fit_batch = lambda plans, iters, metric: ([], ev.run())
+    ev.set_tuning(TUNE_FIT_TILE_ROWS, 2048)  # whatever an earlier batch chose
+    res = at.tune_fit(ev, [Plan(3)] * len(rows), 8, 0, rows=rows, reps=1, **kw)
+    return ev, res
+
+
+@pytest.mark.parametrize("confirm", [False, True])
+@pytest.mark.parametrize("rows", [1000, 100000])
+def test_a_fit_tuner_measures_the_built_in_choice_and_returns_to_it(rows, confirm):
+    ev, res = _tuned(_adaptive(10.0, {8192: 14.0, 2048: 10.1}), [rows] * 48, confirm=confirm)
+    assert ev.t == {TUNE_FIT_TILE_ROWS: 0, TUNE_FIT_ROWS_PER_LANE: 0, TUNE_EVAL_TILE_ROWS: 0}
+    assert (res.best_ms, res.builtin_ms, res.speedup) == (10.0, 10.0, 1.0)
+    assert all(v == 0 for v in res.best.values())
+    assert 8192 in {s[TUNE_FIT_TILE_ROWS] for s, _ in res.table}
+
+
+@pytest.mark.parametrize("confirm", [False, True])
+def test_a_size_that_beats_the_built_in_choice_is_compared_with_it(confirm):
+    ev, res = _tuned(_adaptive(10.0, {8192: 9.9, 4096: 8.0}), [100000] * 48, confirm=confirm)
+    assert ev.t[TUNE_FIT_TILE_ROWS] == 4096 and (res.best_ms, res.builtin_ms) == (8.0, 10.0)
+    if confirm:
+        assert [s[TUNE_FIT_TILE_ROWS] for s, _ in res.confirm_table] == [0, 4096]
+
+
+def test_an_eval_tuner_measures_the_built_in_choice_and_returns_to_it():
+    for explicit, want in ((12.0, 0), (5.0, 1024)):
+        ev = FakeEv(lambda t, e=explicit: {0: 10.0, 1024: e}.get(t[TUNE_EVAL_TILE_ROWS], 20.0))
+        ev.eval_words = lambda prog, off, loss: (None, ev.run())
+        res = at.tune_eval(ev, None, [0] * 9, 1000, reps=1)
+        assert ev.t[TUNE_EVAL_TILE_ROWS] == want and res.builtin_ms == 10.0
+
+
+def test_choices_cached_under_the_earlier_meaning_are_not_applied(tmp_path):
+    cache = at.TuningCache(str(tmp_path / "t.json"))
+    # What a tuner without the built-in choice in its grid wrote for it.
+    cache.put("fit:P5:med9:max9:k2:sq", {TUNE_FIT_TILE_ROWS: 8192, TUNE_FIT_ROWS_PER_LANE: 4})
+    ev, res = _tuned(_adaptive(10.0, {8192: 14.0}), [1000] * 48, cache=cache)
+    assert ev.t[TUNE_FIT_TILE_ROWS] == 0 and res.best_ms == 10.0

@@ -12,10 +12,14 @@ The shapes (rc_set_tuning, include/rcsr_hip.h):
     the LDS block (more waves per SIMD);
   - rows per evaluation tile (TUNE_EVAL_TILE_ROWS).
 
+A shape of 0 is the built-in choice, which follows the batch and the row
+count: no size set by hand stands for it.
+
 The tuner times the caller's own work (a fit batch, a sample of it, or an
-evaluation batch) under each shape of a small grid on the device, keeps the
-fastest, and leaves the built-in shape in place unless another is faster by
-more than `margin` (timing noise never flips a choice).  Choices can be kept
+evaluation batch) under the built-in choice and each shape of a small grid on
+the device, keeps the fastest, and leaves the built-in choice in place unless a
+shape is faster by more than `margin` (timing noise never flips a choice).
+Choices can be kept
 in a JSON cache keyed by a workload signature (row counts, batch size,
 constants, metrics in power-of-two buckets), so a search loop tunes once per
 shape of work.  A candidate's results depend on its program, its rows and
@@ -37,8 +41,12 @@ from .host import TUNE_EVAL_TILE_ROWS, TUNE_FIT_ROWS_PER_LANE, TUNE_FIT_TILE_ROW
 FIT_TILES = (2048, 4096, 8192, 16384, 32768, 65536)
 FIT_ROWS = (4, 2)
 EVAL_TILES = (1024, 2048, 4096, 8192, 16384)
-BUILTIN = {TUNE_FIT_TILE_ROWS: 8192, TUNE_FIT_ROWS_PER_LANE: 4, TUNE_EVAL_TILE_ROWS: 4096}
-BUILTIN_FIT = {TUNE_FIT_TILE_ROWS: 8192, TUNE_FIT_ROWS_PER_LANE: 4}
+# The built-in choices (0), and for a grid of a caller's own without them the
+# sizes they take for large batches, as what the others have to beat.
+BUILTIN = {TUNE_FIT_TILE_ROWS: 0, TUNE_FIT_ROWS_PER_LANE: 0, TUNE_EVAL_TILE_ROWS: 0}
+BUILTIN_FIT = {k: BUILTIN[k] for k in (TUNE_FIT_TILE_ROWS, TUNE_FIT_ROWS_PER_LANE)}
+BUILTIN_EVAL = {TUNE_EVAL_TILE_ROWS: BUILTIN[TUNE_EVAL_TILE_ROWS]}
+LARGE_BATCH = {TUNE_FIT_TILE_ROWS: 8192, TUNE_FIT_ROWS_PER_LANE: 4, TUNE_EVAL_TILE_ROWS: 4096}
 
 Setting = Dict[int, int]
 
@@ -70,15 +78,25 @@ class TuneResult:
         }
 
 
-def _is_builtin(setting: Setting) -> bool:
-    return all(BUILTIN.get(k) == v for k, v in setting.items())
+def _reference(space: Sequence[Setting]) -> Optional[Setting]:
+    """What the other settings of a grid have to beat: the built-in choice, else
+    the large batch's sizes, if it has them."""
+    for s in space:
+        if all(BUILTIN.get(k) == v for k, v in s.items()):
+            return s
+    for s in space:
+        if all(LARGE_BATCH.get(k) == v for k, v in s.items()):
+            return s
+    return None
 
 
 def tune(ev, run: Callable[[], float], space: Sequence[Setting], reps: int = 2,
          margin: float = 0.02) -> Optional[TuneResult]:
     """Time run() (device ms of one call, < 0 = failed) under every setting of
-    `space` on evaluator `ev`, apply the fastest (the built-in setting unless
-    another beats it by more than `margin`) and return the timings.  Settings
+    `space` on evaluator `ev`, apply the fastest (the built-in choice, if it is
+    among them, unless another beats it by more than `margin`) and return the
+    timings; builtin_ms is the built-in choice's, or in a grid without it that of
+    the sizes it takes for large batches.  Settings
     the library refuses, and runs that fail, are skipped; with no successful
     run the previous shapes are restored and None is returned."""
     keys = sorted({k for s in space for k in s})
@@ -96,10 +114,10 @@ def tune(ev, run: Callable[[], float], space: Sequence[Setting], reps: int = 2,
             ev.set_tuning(k, v)
         return None
     best, best_ms = min(table, key=lambda e: e[1])
-    builtin = [ms for s, ms in table if _is_builtin(s)]
-    builtin_ms = builtin[0] if builtin else float("nan")
-    if builtin and builtin_ms <= best_ms * (1.0 + margin):
-        best, best_ms = next(s for s, ms in table if _is_builtin(s)), builtin_ms
+    ref = _reference([s for s, _ in table])
+    builtin_ms = next(ms for s, ms in table if s == ref) if ref is not None else float("nan")
+    if ref is not None and builtin_ms <= best_ms * (1.0 + margin):
+        best, best_ms = ref, builtin_ms
     for k, v in best.items():
         ev.set_tuning(k, v)
     return TuneResult(dict(best), best_ms, builtin_ms, table)
@@ -107,22 +125,25 @@ def tune(ev, run: Callable[[], float], space: Sequence[Setting], reps: int = 2,
 
 def fit_space(max_rows: int, tiles: Sequence[int] = FIT_TILES,
               rows: Sequence[int] = FIT_ROWS) -> List[Setting]:
-    """Tile sizes up to the next one covering the largest candidate (larger
-    tiles are the same work items), crossed with the rows-per-lane choices."""
+    """Tile sizes set by hand, up to the next one covering the largest candidate
+    (larger tiles are the same work items), crossed with the rows-per-lane
+    choices.  tune_fit times the built-in choice beside them."""
     cover = [t for t in tiles if t < max_rows]
     bigger = [t for t in tiles if t >= max_rows]
     if bigger:
         cover.append(min(bigger))
-    if BUILTIN[TUNE_FIT_TILE_ROWS] not in cover and BUILTIN[TUNE_FIT_TILE_ROWS] in tiles:
-        cover.append(BUILTIN[TUNE_FIT_TILE_ROWS])
+    if LARGE_BATCH[TUNE_FIT_TILE_ROWS] not in cover and LARGE_BATCH[TUNE_FIT_TILE_ROWS] in tiles:
+        cover.append(LARGE_BATCH[TUNE_FIT_TILE_ROWS])
     return [{TUNE_FIT_TILE_ROWS: t, TUNE_FIT_ROWS_PER_LANE: r} for t in sorted(set(cover))
             for r in rows]
 
 
 def eval_space(n: int, tiles: Sequence[int] = EVAL_TILES) -> List[Setting]:
+    """Tiles set by hand for n rows; tune_eval times the built-in choice beside
+    them."""
     cover = [t for t in tiles if t < n] + [t for t in tiles if t >= n][:1]
-    if BUILTIN[TUNE_EVAL_TILE_ROWS] not in cover and BUILTIN[TUNE_EVAL_TILE_ROWS] in tiles:
-        cover.append(BUILTIN[TUNE_EVAL_TILE_ROWS])
+    if LARGE_BATCH[TUNE_EVAL_TILE_ROWS] not in cover and LARGE_BATCH[TUNE_EVAL_TILE_ROWS] in tiles:
+        cover.append(LARGE_BATCH[TUNE_EVAL_TILE_ROWS])
     return [{TUNE_EVAL_TILE_ROWS: t} for t in sorted(set(cover))]
 
 
@@ -134,7 +155,8 @@ def signature(kind: str, rows: Sequence[int], ks: Sequence[int] = (),
               metrics: Sequence[int] = ()) -> str:
     """Power-of-two buckets of what sets the best shape: the batch size, the
     median and largest row counts, the mean constant count and the metric
-    mix."""
+    mix.  The 2 keeps apart choices of when sizes set by hand stood for the
+    built-in choice."""
     rows = sorted(int(r) for r in rows)
     med = rows[len(rows) // 2] if rows else 0
     mx = rows[-1] if rows else 0
@@ -143,7 +165,7 @@ def signature(kind: str, rows: Sequence[int], ks: Sequence[int] = (),
     if metrics:
         l1 = sum(1 for m in metrics if m == 4) / len(metrics)
         mix = "sq" if l1 == 0 else ("l1" if l1 == 1 else "mixed")
-    return f"{kind}:P{_b(len(rows))}:med{_b(med)}:max{_b(mx)}:k{_b(km + 1)}:{mix}"
+    return f"{kind}2:P{_b(len(rows))}:med{_b(med)}:max{_b(mx)}:k{_b(km + 1)}:{mix}"
 
 
 class TuningCache:
@@ -183,11 +205,12 @@ def tune_fit(ev, plans, iters: int, metric: int = 0, rows: Optional[Sequence[int
     """Tune the fit shapes for a batch: `rows` are the candidates' row counts
     (one per candidate); a heterogeneous batch passes its rowset and metrics
     (rc_fit_batch_hetero).  The timing runs on an evenly spread sample of at
-    most `sample` candidates.  With `confirm`, a sample winner other than the
-    built-in shape is timed against the built-in shape on the whole batch and
-    kept only if it is faster there by more than `margin` (a sample can rank
-    shapes differently from the batch it stands for).  With a cache, a known
-    signature is applied without timing (best_ms is then NaN)."""
+    most `sample` candidates, over the built-in choice and the grid of
+    fit_space (or `space` alone).  With `confirm`, a sample winner other than the
+    built-in choice is timed against it on the whole batch and kept only if it is
+    faster there by more than `margin` (a sample can rank shapes differently from
+    the batch it stands for).  With a cache, a known signature is applied without
+    timing (best_ms is then NaN)."""
     n = len(plans)
     rows = list(rows) if rows is not None else [0] * n
     step = max(1, n // max(sample, 1))
@@ -209,9 +232,12 @@ def tune_fit(ev, plans, iters: int, metric: int = 0, rows: Optional[Sequence[int
     else:
         def run():
             return ev.fit_batch(sub, iters, metric)[1]
-    res = tune(ev, run, space if space is not None else fit_space(max(rows) if rows else 0),
-               reps=reps, margin=margin)
-    if res is not None and confirm and not _is_builtin(res.best):
+    if space is None:
+        space = [dict(BUILTIN_FIT), {**BUILTIN_FIT, TUNE_FIT_ROWS_PER_LANE: 2}]
+        space += fit_space(max(rows) if rows else 0)
+    res = tune(ev, run, space, reps=reps, margin=margin)
+    ref = _reference(space) or BUILTIN_FIT
+    if res is not None and confirm and res.best != ref:
         if rowset is not None:
             rs_all = [int(r) for r in rowset]
             ms_all = [int(m) for m in metrics] if metrics is not None else [metric] * n
@@ -221,7 +247,7 @@ def tune_fit(ev, plans, iters: int, metric: int = 0, rows: Optional[Sequence[int
         else:
             def run_all():
                 return ev.fit_batch(plans, iters, metric)[1]
-        full = tune(ev, run_all, [dict(BUILTIN_FIT), dict(res.best)], reps=reps, margin=margin)
+        full = tune(ev, run_all, [dict(ref), dict(res.best)], reps=reps, margin=margin)
         if full is not None:
             res = TuneResult(full.best, full.best_ms, full.builtin_ms, res.table, full.table)
     if res is not None and cache is not None:
@@ -242,7 +268,8 @@ def tune_eval(ev, prog, off, n: int, reps: int = 3, cache: Optional[TuningCache]
 
     def run():
         return ev.eval_words(prog, off, 0)[1]
-    res = tune(ev, run, space if space is not None else eval_space(n), reps=reps)
+    res = tune(ev, run, space if space is not None else [dict(BUILTIN_EVAL)] + eval_space(n),
+               reps=reps)
     if res is not None and cache is not None:
         cache.put(sig, res.best)
     return res
