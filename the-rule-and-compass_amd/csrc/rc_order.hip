@@ -31,6 +31,7 @@
  *    along one constant, over tiles and then over a segment's tiles.
  */
 #include "rc_fit_dev.h"
+#include "rc_block.h"
 #include "rc_fitvm.h"
 #include "rc_internal.h"
 #include "rc_order_kern.h"
@@ -680,13 +681,6 @@ void stage_sets(const RcCtx *c, const unsigned int *prog, const unsigned int *of
     }
 }
 
-size_t stage_take(size_t &cur, size_t bytes)
-{
-    const size_t o = (cur + 255) & ~(size_t)255;
-    cur = o + bytes;
-    return o;
-}
-
 /* coords / levels: nsegs each, or null; flags: nsegs ints at the device. */
 int stage_inputs(RcCtx *c, const unsigned int *prog, const unsigned int *off, const int *pcount,
                  int nsets, int nsegs, int kmax, const double *c0, const int *coords,
@@ -696,32 +690,22 @@ int stage_inputs(RcCtx *c, const unsigned int *prog, const unsigned int *off, co
     std::vector<int> lists(in->fast);
     lists.insert(lists.end(), in->general.begin(), in->general.end());
     const size_t ns = (size_t)nsegs;
-    size_t cur = 0;
-    const size_t o_prog = stage_take(cur, 4 * (size_t)off[nsets]);
-    const size_t o_off = stage_take(cur, 4 * ((size_t)nsets + 1));
-    const size_t o_pc = stage_take(cur, 4 * (size_t)nsets);
-    const size_t o_c0 = stage_take(cur, 8 * ns * (size_t)kmax);
-    const size_t o_code = stage_take(cur, 4 * in->code.size());
-    const size_t o_sets = stage_take(cur, sizeof(OrSet) * in->sets.size());
-    const size_t o_list = stage_take(cur, 4 * lists.size());
-    const size_t o_flag = stage_take(cur, 4 * flags.size());
-    const size_t o_co = stage_take(cur, coords ? 4 * ns : 0);
-    const size_t o_lv = stage_take(cur, levels ? 8 * ns : 0);
-    cur = stage_take(cur, 1);
-    std::vector<unsigned char> &h = b.h_in;
-    h.resize(cur);
-    memcpy(&h[o_prog], prog, 4 * (size_t)off[nsets]);
-    memcpy(&h[o_off], off, 4 * ((size_t)nsets + 1));
-    memcpy(&h[o_pc], pcount, 4 * (size_t)nsets);
-    memcpy(&h[o_c0], c0, 8 * ns * (size_t)kmax);
-    if (!in->code.empty()) memcpy(&h[o_code], in->code.data(), 4 * in->code.size());
-    memcpy(&h[o_sets], in->sets.data(), sizeof(OrSet) * in->sets.size());
-    memcpy(&h[o_list], lists.data(), 4 * lists.size());
-    memcpy(&h[o_flag], flags.data(), 4 * flags.size());
-    if (coords) memcpy(&h[o_co], coords, 4 * ns);
-    if (levels) memcpy(&h[o_lv], levels, 8 * ns);
-    if (rc_grow(c, (void **)&b.in, &b.in_cap, cur, 1) != 0 ||
-        hipMemcpyAsync(b.in, h.data(), cur, hipMemcpyHostToDevice, c->s_fit) != hipSuccess)
+    const size_t words = off[nsets];
+    RcBlock h(b.h_in, 4 * words + 8 * ns * (size_t)(kmax + 3) + 64 * (size_t)nsets +
+                          4 * in->code.size() + 4096);
+    const size_t o_prog = h.put(prog, 4 * words);
+    const size_t o_off = h.put(off, 4 * ((size_t)nsets + 1));
+    const size_t o_pc = h.put(pcount, 4 * (size_t)nsets);
+    const size_t o_c0 = h.put(c0, 8 * ns * (size_t)kmax);
+    const size_t o_code = h.put(in->code);
+    const size_t o_sets = h.put(in->sets);
+    const size_t o_list = h.put(lists);
+    const size_t o_flag = h.put(flags);
+    const size_t o_co = h.put(coords, coords ? 4 * ns : 0);
+    const size_t o_lv = h.put(levels, levels ? 8 * ns : 0);
+    const size_t bytes = b.h_in.size();
+    if (rc_grow(c, (void **)&b.in, &b.in_cap, bytes, 1) != 0 ||
+        hipMemcpyAsync(b.in, b.h_in.data(), bytes, hipMemcpyHostToDevice, c->s_fit) != hipSuccess)
         return -1;
     in->prog = (uint32_t *)(b.in + o_prog);
     in->off = (uint32_t *)(b.in + o_off);
