@@ -149,14 +149,17 @@ class _File:
 def run(fwd, rev, c, X, col_bytes, flags=0, bslots=None, aslots=None):
     """Forward value and constant gradients of every row of X (rows x vars).
     flags: the compiler options the streams were built with (inputs in U,
-    an 8-slot U file).  bslots / aslots: the sizes of the B and A files the
+    an 8-slot U file, tape values in B or in LDS slots).  bslots / aslots: the sizes of the B and A files the
     kernel runs the streams with (the 4-row assembly uses 8 and 2); slot
     numbers are masked to the file size, as the device masks them.
 
     The simulator writes every tape word's B slot and every general reverse
     word's A slot, NaN where the word keeps nothing (the compiler names the
     sink there), so a word that names a live slot where it should name the
-    sink corrupts the result."""
+    sink corrupts the result.  With VMC_SMALL_B all 8 slots of the B file may
+    hold values, and no slot is left for the sink: a word that keeps nothing must
+    name it all the same, and writes nothing, as on the device.  A VMF_TB word's
+    tape value goes to B or to the LDS file L, and U gets its sink."""
     X = np.asarray(X, np.float64)
     rows = X.shape[0]
     c = np.asarray(c, np.float64)
@@ -169,7 +172,21 @@ def run(fwd, rev, c, X, col_bytes, flags=0, bslots=None, aslots=None):
             U.set(q, X[:, q])
     nb = bslots or D["VM_B_SLOTS"]
     na = aslots or D["VM_A_SLOTS"]
-    B = _File("B", nb, rows, D["VM_B_SINK"] & (nb - 1))
+    small_b = bool(flags & D["VMC_SMALL_B"])
+    if small_b:
+        nb = 8
+    B = _File("B", nb, rows, None if small_b else D["VM_B_SINK"] & (nb - 1))
+    L = _File("L", D["VM_L_SLOTS"], rows, None)
+
+    def b_write(bs, keeps, x):
+        if not small_b:
+            B.set(bs & (nb - 1), x)
+        elif keeps:
+            assert bs < nb, f"B slot {bs} of an 8-slot file"
+            B.set(bs, x)
+        else:
+            assert bs == D["VM_B_SINK"], f"a word that keeps nothing names B slot {bs}"
+
     A = _File("A", na, rows, D["VM_A_SINK"] & (na - 1))
     garbage = np.full(rows, np.nan)
     tos = np.zeros(rows)
@@ -188,13 +205,13 @@ def run(fwd, rev, c, X, col_bytes, flags=0, bslots=None, aslots=None):
     for x, y in fw:
         x, y = int(x), int(y)
         us, ur, bs, xv, op = (y >> 8) & 15, (y >> 12) & 15, (y >> 16) & 15, (y >> 20) & 7, (y >> 23) & 31
-        bs &= nb - 1
         if small:
             ur &= 7
         uv = tos
         if x & D["VMF_UNMC"]:
             f = _unary(op, tos)
-            B.set(bs, _partial(op, tos, f) if x & D["VMF_NEED"] else garbage)
+            need = bool(x & D["VMF_NEED"])
+            b_write(bs, need, _partial(op, tos, f) if need else garbage)
             uv = f
             nt = f * cval(y)
         elif x & D["VMF_VMC"]:
@@ -230,9 +247,13 @@ def run(fwd, rev, c, X, col_bytes, flags=0, bslots=None, aslots=None):
                 uv = d0
                 if x & D["VMF_D1"]:
                     d1 = d1p
-            B.set(bs, d1)
+            b_write(bs, bool(x & D["VMF_D1"]), d1)
         else:
             raise AssertionError(f"forward word without a handler: {x:#x}")
+        if x & D["VMF_TB"]:
+            assert flags & (D["VMC_TAPE_B"] | D["VMC_TAPE_L"])
+            (B if flags & D["VMC_TAPE_B"] else L).set(us, uv)
+            us = usink
         if small:
             us &= 7
         if in_u and us < X.shape[1]:
@@ -266,15 +287,22 @@ def run(fwd, rev, c, X, col_bytes, flags=0, bslots=None, aslots=None):
         x, y = int(rw[i][0]), int(rw[i][1])
         ut, bt, as_, ar, xv, op = ((y >> 8) & 15, (y >> 12) & 15, (y >> 16) & 7, (y >> 19) & 7,
                                    (y >> 22) & 7, (y >> 25) & 31)
-        bt &= nb - 1
+        if not small_b:
+            bt &= nb - 1
         as_ &= na - 1
+
+        def tape():
+            if not y & D["VMR_Y_TB"]:
+                return U.get(ut)
+            assert flags & (D["VMC_TAPE_B"] | D["VMC_TAPE_L"])
+            return (B if flags & D["VMC_TAPE_B"] else L).get(ut)
         ar &= na - 1
 
         def pop():
             return A.get(ar) if ar != A.sink else np.full(rows, np.nan)
 
         if x & D["VMR_UNMC_N"]:
-            gw(x, z(a, U.get(ut)))
+            gw(x, z(a, tape()))
             a = z(z(a, cval(y)), B.get(bt))
         elif x & D["VMR_VMC"]:
             gw(x, z(a, xin(xv)))
@@ -282,15 +310,15 @@ def run(fwd, rev, c, X, col_bytes, flags=0, bslots=None, aslots=None):
         elif x & D["VMR_PUSH"]:
             A.set(as_, a)
         elif x & D["VMR_MULC_N"]:
-            gw(x, z(a, U.get(ut)))
+            gw(x, z(a, tape()))
             a = z(a, cval(y))
         elif x & D["VMR_UNMC_P"]:
-            gw(x, z(a, U.get(ut)))
+            gw(x, z(a, tape()))
             a = pop()
         elif x & D["VMR_UN"]:
-            a = z(a, U.get(ut))
+            a = z(a, tape())
         elif x & D["VMR_MULC_P"]:
-            gw(x, z(a, U.get(ut)))
+            gw(x, z(a, tape()))
             a = pop()
         elif x & D["VMR_MULV"]:
             a = z(a, xin(xv))
@@ -306,14 +334,14 @@ def run(fwd, rev, c, X, col_bytes, flags=0, bslots=None, aslots=None):
             rneed = bool(x & (D["VMR_RNODE"] | D["VMR_RCONST"]))
             gl = gr = None
             if x & D["VMR_UNARY"]:
-                gl = z(a, U.get(ut))
+                gl = z(a, tape())
             elif op == OP_ADD:
                 gl, gr = a.copy(), a.copy()
             elif op == OP_SUB:
                 gl, gr = a.copy(), -a
             else:
                 # only the partials of the children the sweep needs exist
-                gl = z(a, U.get(ut)) if lneed else None
+                gl = z(a, tape()) if lneed else None
                 gr = z(a, B.get(bt)) if rneed else None
             if x & D["VMR_LCONST"]:
                 gw(x, gl)

@@ -28,6 +28,7 @@ BINARY = [ADD, SUB, MUL, DIV, POW]
 
 
 INPUTS_IN_U, VALUE_ONLY, SMALL_U = 1, 2, 4
+TAPE_B, SMALL_B, TAPE_L = 8, 16, 32
 
 
 def compile_tree(tree, nvars=3, flags=0):
@@ -74,7 +75,7 @@ def check_tree(tree, X, rel=1e-9, flags=0):
             if not np.isfinite(g[j]):
                 continue
             assert abs(gv - g[j]) <= rel * (1.0 + abs(g[j])) * 10, (str(tree), r, j, gv, g[j])
-    if info[3] <= 7 and info[4] <= 1:
+    if info[3] <= 7 and info[4] <= 1 and not flags & SMALL_B:
         # On an 8-slot B file and a 2-slot A file (the 4-row assembly's) the
         # sinks are slots 7 and 1: the streams still compute the same.
         p4, g4 = fitvm_sim.run(fw, rv, plan.c0, X, COL_BYTES, flags, bslots=8, aslots=2)
@@ -250,3 +251,62 @@ def test_inputs_in_u_and_value_only_streams(flags, X):
                           flags=flags) == 0
     for name, build in EDGE:
         assert check_tree(build(), X, flags=flags) == 0, name
+
+
+def _sum_of_terms(rng, nv, terms, inner):
+    """`terms` terms c * u(x), the first `inner` of them c * u(c' v(x)): a tape
+    value a term, or two."""
+    ops = [SIN, SQUARE, COS, TANH, EXP, CUBE, GAUSS, SIG]
+    def term(i):
+        x = node(ops[int(rng.integers(len(ops)))], var(i % nv))
+        if i < inner:
+            x = node(ops[int(rng.integers(len(ops)))], node(MUL, const(0.3 + 0.1 * i), x))
+        return node(MUL, const(0.5 + 0.1 * i), x)
+    t = term(0)
+    for i in range(1, terms):
+        t = node([ADD, SUB][i % 2], t, term(i))
+    return t
+
+
+@pytest.mark.parametrize("tape", [TAPE_B, TAPE_L])
+def test_tapes_beyond_the_u_file(tape, X):
+    """The 4-row streams whose tape goes on in B or in LDS, from programs that U
+    still holds to those that neither form takes."""
+    rng = np.random.default_rng(5)
+    flags = INPUTS_IN_U | SMALL_B | tape
+    took = refused = beyond = 0
+    for terms in range(2, 21):
+        for inner in range(0, min(terms, 20 - terms) + 1, 2):
+            t = _sum_of_terms(rng, 3, terms, inner)
+            if host.gpu_fit_plan(t) is None:  # too many nodes
+                continue
+            rc = check_tree(t, X, rel=1e-8, flags=flags)
+            assert rc in (0, -3), (terms, inner, rc)
+            took += rc == 0
+            refused += rc == -3
+            in_u = compile_tree(t, 3, INPUTS_IN_U)[0]
+            assert not (in_u == 0 and rc != 0 and tape == TAPE_L), (terms, inner)
+            beyond += in_u == -3 and rc == 0
+    assert beyond >= 8 and took >= 40, (took, refused, beyond)
+    for _ in range(120):
+        t = full_tree(rng, int(rng.integers(2, 6)))
+        if t.constants() and host.gpu_fit_plan(t) is not None:
+            assert check_tree(t, X, rel=1e-8, flags=flags) in (0, -3)
+
+
+def test_simulator_catches_a_tape_slot_taken_twice(X):
+    # Plant the slot of another term's tape value into one LDS tape word: that
+    # term's gradient must move.
+    D = fitvm_sim.D
+    flags = INPUTS_IN_U | SMALL_B | TAPE_L
+    rc, plan, fw, rv, info = compile_tree(_sum_of_terms(np.random.default_rng(1), 3, 16, 0), 3, flags)
+    assert rc == 0 and info[5] >= 2
+    fw = fw.copy().reshape(-1, 2)
+    tb = [i for i in range(len(fw)) if fw[i, 0] & D["VMF_TB"]]
+    _, good = fitvm_sim.run(fw.ravel(), rv, plan.c0, X, COL_BYTES, flags)
+    wrong = fw.copy()
+    first = (int(fw[tb[0], 1]) >> 8) & 15
+    wrong[tb[1], 1] = (int(wrong[tb[1], 1]) & ~(15 << 8)) | (first << 8)
+    with pytest.raises(fitvm_sim.SlotError):  # the second value's slot is never written
+        fitvm_sim.run(wrong.ravel(), rv, plan.c0, X, COL_BYTES, flags)
+    assert sorted(good) == list(range(plan.nconst))
