@@ -128,3 +128,20 @@ def test_device_variation_at_the_slot_width_limits(ev, width, islands, pop, maxc
         ref = oracle.vary(parents, islands, pop, err, 13, 3, max_complexity=maxc, nvars=2,
                           init_depth=depth, dedup=dedup)
         _same(dev, ref)
+
+
+# Children whose attempts vy_try does not keep are made again from their
+# position, as in pools of 64 MB of attempts and more.  Most attempts of the
+# narrow pool fail its width filter.
+@pytest.mark.parametrize("width,islands,pop,maxc,depth", [(64, 4, 96, 30, 3), (16, 2, 48, 6, 2)])
+def test_children_made_again_are_the_kept_ones(ev, monkeypatch, width, islands, pop, maxc, depth):
+    parents, err = _parents(islands, pop, width, seed=29)
+    _say(f"pool vary: {islands} x {pop}, width {width}, attempts not kept")
+    ref = oracle.vary(parents, islands, pop, err, 29, 2, max_complexity=maxc, nvars=2,
+                      init_depth=depth)
+    for cap in ("0", None):
+        if cap is None:
+            monkeypatch.delenv("RCSR_VARY_KEPT_CAP")
+        else:
+            monkeypatch.setenv("RCSR_VARY_KEPT_CAP", cap)
+        _same(_device_vary(ev, parents, err, islands, pop, 29, 2, True, maxc=maxc, depth=depth), ref)

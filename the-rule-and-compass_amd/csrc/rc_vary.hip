@@ -42,6 +42,7 @@
 #include "rc_internal.h"
 
 #include <math.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -52,8 +53,9 @@ namespace {
 constexpr int VY_WMAX = 128;  /* widest supported pool slot */
 constexpr int VY_TRY = 8;     /* attempts precomputed per child */
 constexpr int VY_ATTEMPTS = 64;
-/* The most memory for the programs of vy_try's attempts; a pool whose attempts
-   need more makes the chosen ones again. */
+/* The most memory for the programs of vy_try's attempts (or the byte count in
+   the environment variable RCSR_VARY_KEPT_CAP); a pool whose attempts need more
+   makes the chosen ones again. */
 constexpr size_t VY_KEPT_BYTES = (size_t)64 << 20;
 constexpr int VY_MAXOPS = 64;
 constexpr uint32_t VY_HALT = 255;
@@ -730,7 +732,9 @@ extern "C" int rc_pool_vary(void *ctx, int from, int islands, int pop, unsigned 
     const size_t o_entry = vy_take(cur, (size_t)n * 4);
     const size_t o_elite = vy_take(cur, (size_t)islands * 4);
     const size_t kept_bytes = (size_t)n * VY_TRY * (size_t)width * 4;
-    const bool keep = g.dedup && kept_bytes <= VY_KEPT_BYTES;
+    size_t kept_cap = VY_KEPT_BYTES;
+    if (const char *e = getenv("RCSR_VARY_KEPT_CAP")) kept_cap = (size_t)strtoull(e, nullptr, 10);
+    const bool keep = g.dedup && kept_bytes <= kept_cap;
     const size_t o_kept = vy_take(cur, keep ? kept_bytes : 0);
     const size_t o_klen = vy_take(cur, (size_t)n * 2);
     const size_t o_kcost = vy_take(cur, (size_t)n * 2);
