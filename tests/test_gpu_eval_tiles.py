@@ -4,7 +4,6 @@ correlation score, and the rare operators' shared call, against f64
 reductions of the device's own predictions."""
 import numpy as np
 import pytest
-import torch
 
 from rcsr_hip import host, lib
 from rcsr_hip.expr import (ADD, ATAN2, CUBE, DIV, ERF, IF, LOG, MAX, MOD, MUL, POW, SIN, SQRT, SUB,
@@ -98,7 +97,7 @@ def test_correlation_of_predictions_with_an_outlier_in_the_first_row(n, tile, ou
     ev.close()
 
 
-def test_only_the_scores_with_further_sums_hold_memory_for_them():
+def test_only_the_scores_with_further_sums_hold_memory_for_them(free_memory):
     n, copies = 4096, 7500
     y, ev = _evaluator(n)
     prog, off = _words(TREES)
@@ -107,12 +106,12 @@ def test_only_the_scores_with_further_sums_hold_memory_for_them():
     boff = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
     assert ev.eval_words(big, boff, 0)[1] >= 0    # grows the sums that every score has too
     print(f"score memory: {len(boff) - 1} programs x {n} rows", flush=True)
-    free = torch.cuda.mem_get_info()[0]
+    free = free_memory()
     score, st, ms = ev.score_words(big, boff, 0)
     assert ms >= 0
     # 960 000 items: 8 bytes each for a second sum would be 7.7 MB; the values and
     # statuses of the call are 0.7 MB.
-    assert free - torch.cuda.mem_get_info()[0] <= 4 << 20
+    assert free - free_memory() <= 4 << 20
     ev.close()
 
 

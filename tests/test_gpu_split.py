@@ -6,7 +6,6 @@ import threading
 
 import numpy as np
 import pytest
-import torch
 
 from rcsr_hip import host, workloads
 from rcsr_hip.expr import ADD, COS, LOG, MUL, SIN, SQUARE, SUB, const, node, var
@@ -153,7 +152,7 @@ def test_implicit_relations_of_every_sweep(n, copies):
     ev.close()
 
 
-def test_implicit_scores_hold_two_sums_an_item():
+def test_implicit_scores_hold_two_sums_an_item(free_memory):
     """8000 candidates x 8192 rows are 128 000 items: 2 MB of sums, where the
     fit's triangles would be 236 MB.  A second thread watches the free memory."""
     n, copies = 8192, 8000
@@ -161,12 +160,12 @@ def test_implicit_scores_hold_two_sums_an_item():
     plans = [host.gpu_fit_plan(CURVE[0])] * copies
     assert ev.implicit_score_batch(plans)[2] >= 0
     print(f"split: implicit score memory, {copies} x {n}", flush=True)
-    before = torch.cuda.mem_get_info()[0]
+    before = free_memory()
     least, stop = [before], threading.Event()
 
     def watch():
         while not stop.is_set():
-            least[0] = min(least[0], torch.cuda.mem_get_info()[0])
+            least[0] = min(least[0], free_memory())
 
     t = threading.Thread(target=watch)
     t.start()
