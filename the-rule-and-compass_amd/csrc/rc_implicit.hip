@@ -13,21 +13,25 @@
  *            finite, or the norm is not positive (signed_distance 68-96).
  *
  * Layout.  Work items are (candidate, row tile; RcSplit) with one wave each; a
- * lane walks its rows of the tile and evaluates the candidate's post-order
- * records (the rch_fit_plan form) with per-lane value and adjoint arrays.
- * Three kinds of pass:
+ * lane walks its rows of the tile.  Three kinds of pass:
  *   SCORE  sum w * |d| (metric 0) or w * |f| (metric 1) and sum w;
  *   RSS    sum (sqrt(w) d)^2 at one constant vector;
  *   JAC    the central-difference Jacobian of r = sqrt(w) d in the constants
  *          (2k + 1 distances per row, h = 1e-6 (1 + |c_j|), implicit.rs:
- *          320-345) and the augmented Gram [J | r]^T [J | r]: the rows of a
- *          64-row step are staged in LDS and every Gram entry is owned by one
- *          lane that adds the 64 products in row order.
- * Partials are per item and reduced on the host in item order, so a
- * candidate's result does not depend on the batch.  The LM control
- * (Gaussian elimination with partial pivoting, lambda x6 / /8, clamp to
- * +-1e6, implicit.rs:215-253, 277-409) runs on the host between batched
- * passes: one JAC and one RSS launch per iteration for the whole batch.
+ *          320-345) and the augmented Gram [J | r]^T [J | r].
+ * Three kernels run a pass, each the candidates whose programs suit it:
+ * im_wide_kernel (rc_implicit_kern.hip: four sweeps side by side on a short
+ * register stack), im_fast_kernel (one sweep with forward tangents on a
+ * deeper register stack) and im_pass_kernel (the rch_fit_plan records in post
+ * order, with per-lane value and adjoint arrays).  The first two reduce the
+ * Gram of a 64-row step on FP64 MFMA; in im_pass_kernel every Gram entry is
+ * owned by one lane that adds the 64 products in row order.
+ * Partials are per item and added in item order, by im_ctrl_kernel in a fit and
+ * on the host for scores, so a candidate's result does not depend on the
+ * batch.  The LM control (Gaussian elimination with partial pivoting, lambda
+ * x6 / /8, clamp to +-1e6, implicit.rs:215-253, 277-409) is im_ctrl_kernel, one
+ * wave per candidate between the batch-wide passes: one JAC and one RSS launch
+ * per iteration for the whole batch, and no host round trip.
  */
 #include "rc_implicit_dev.h"
 #include "rc_internal.h"

@@ -176,10 +176,15 @@ struct RcCtx {
    beside 8192 rows; sub-tiles where they would leave slots empty.  A small
    table has small sub-tiles, or one island's 200 candidates of 1000 rows would
    be 200 waves; 512 rows are one step of the f32 loss kernel.  Measured against
-   groups throughout: 64 absolute-error fits x 100 003 rows 37.1 -> 11.2 ms, 128
-   correlation fits x 50 021 rows 20.3 -> 11.4, 128 implicit fits x 65 537 rows
-   242 -> 97, 200 fits x 1000 rows 1.38 -> 1.21; 1024 fits x 262 144 rows, which
-   keep groups, 198 -> 197. */
+   groups throughout, far below the line: 64 absolute-error fits x 100 003 rows
+   37.1 -> 11.2 ms, 128 correlation fits x 50 021 rows 20.3 -> 11.4, 128 implicit
+   fits x 65 537 rows 242 -> 97, 200 fits x 1000 rows 1.38 -> 1.21.  Nearer to it
+   (8 steps): 2000 fits x 8192 rows 16.4 -> 4.8 ms, 4000 17.5 -> 8.1, 8000
+   22.3 -> 14.7, 8000 x 1000 rows 4.29 -> 3.74, 2600 x 20 000 18.3 -> 10.9; 4200
+   implicit fits x 8192 rows 336 -> 176, 8000 506 -> 331, 8000 x 1000 rows
+   63.5 -> 62.1: nothing is lost up to the line.  Past it sub-tiles still cost
+   their ends: 9000 fits x 1000 to 5000 rows, which keep groups, are 1 to 2%
+   slower than with sums by group alone; 1024 x 262 144 rows the same. */
 constexpr int RC_GROUP_ROWS = 8192;
 constexpr long long RC_ITEMS_WANTED = 8192;
 struct RcSplit {
